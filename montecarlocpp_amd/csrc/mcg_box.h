@@ -1,0 +1,756 @@
+// mcg_box.h -- the step and the wavefront loop of scenes that are one
+// axis-aligned box: the slab, the bar, the film, the bulk cell and the porous
+// film (included by mcg_kernels.hip, in its anonymous namespace).
+//
+// The general step (flight_step / collide_step) reads everything about a
+// bundle's cell from LDS, because neighbouring lanes may be in different
+// cells, and tests each face against a plane record.  With one box all of
+// that is the same for every lane: the bounds, the face kinds and the tally's
+// geometry are wavefront-uniform (BoxCell, held in scalar registers), and a
+// step reads LDS only for what an event draws (the alias table, the mode's
+// mean free path and velocity) and for a diffuse face's rotation.  A specular
+// or periodic face needs no random numbers, so a wavefront whose events are
+// all of those kinds skips the Philox block and the direction draw.
+//
+// What bounds it: vector issue and, in a solve's drain, the latency of one
+// bundle's chain of dependent instructions (a dependent vector instruction
+// issues every 9 cycles from a lone wavefront, an independent one every 5);
+// the general step spends both on what one box does not need: LDS reads of the
+// cell (28 words) behind every step, address arithmetic per tally row, ~70
+// spilled scalars read back lane by lane, and per-step checks for traces.
+// Measured, general kernel against this one, same box: bar 1e7 bundles FP32
+// 5.68 -> 4.43 ms, 1e6 FP64 4.13 -> 3.17 ms, slab 1e5 FP64 562 -> 347 us, slab
+// 1e4 FP32 185 -> 122 us, porous film 1e7 64 x 64 85.3 -> 71.3 ms, film 1e6
+// (12 x 6 map, bundles of up to 10,000 steps) 26.8 -> 14.5 ms.
+//
+// Results: FP32 flight takes the same rounded operations on every quantity a
+// trajectory depends on as the general step, and FP64 the checker's, so
+// bundles take the same events bundle for bundle; the places where an
+// operation of the general step is left out (products with exact zeros and
+// ones) are noted where they are.
+#pragma once
+
+// Event kinds beyond mcg_bdry_kind, and the codes of the events a flight
+// finds: 4 x (2 axis + upper side) for a face, then the intrinsic event and
+// the pore wall.  A code is the bit offset of the event's kind in
+// BoxCell::kinds.
+enum : uint32_t { kKindIntrinsic = 8, kKindPore = 9 };
+enum : uint32_t { kCodeIntrinsic = 24, kCodePore = 28 };
+
+constexpr uint32_t kAlive = 0xFFFFFFFFu;
+
+// LDS row stride of a 1-D tally and of its difference array, in doubles: a
+// compile-time stride puts the rows of one column at immediate offsets of one
+// address (4 addresses a step instead of 16).
+constexpr int kBoxCols = 256;
+
+// Per-face data a step reads from LDS.
+template <typename F>
+struct BoxFace {
+    F rot[9];           // rotation taking z onto the inward normal
+    F pt[3];            // periodic translation
+    uint32_t spec_thr;
+    uint32_t pad[3];
+};
+
+// Wavefront-uniform description of the box and its tally.
+template <typename F>
+struct BoxCell {
+    F lo[3], hi[3];          // face positions
+    F klo[3], khi[3];        // FP32: positions beyond which a bundle is lost
+    F eps;                   // FP64: the kill tolerance
+    uint32_t kinds;          // 4 bits per event code
+    uint32_t planes;         // plane number of each face code, 4 bits each
+    uint32_t maxscat, maxloop;
+    uint32_t k0, k1;
+    int32_t nmodes;
+    int32_t counts;          // per-bundle counts are recorded
+    int32_t partial;         // some wall is partially specular
+    // tally: 0 none, 1 along one axis (a single cell is one axis of one
+    // cell), 2 a grid walked over its divided axes
+    int32_t tally, with_t, with_f, rows, cols;
+    uint32_t comp[3][3];                   // per tally axis: mask of each position component
+    int32_t last[3], stride[3];            // largest index, column stride
+    F o[3], inv[3], div[3];                // cell coordinate = div (inv (p - o))
+    // pore (kind of its wall, or -1)
+    int32_t pore;
+    F cx, cy, r2, rin2;      // axis, radius^2, (radius - tolerance)^2
+    F r;
+    uint32_t pore_thr;
+};
+
+// A quotient by a common divisor: the correctly rounded a / b of the IEEE
+// division sequence (reciprocal estimate, two Newton steps, quotient,
+// remainder correction) without its scaling steps, which leave operands of
+// this size unchanged; the reciprocal is shared by all quotients.
+struct Quotient {
+    double b, r;
+    __device__ __forceinline__ explicit Quotient(double d) : b(d) {
+        double x = __builtin_amdgcn_rcp(d);
+        x = __builtin_fma(x, __builtin_fma(-d, x, 1.0), x);
+        r = __builtin_fma(x, __builtin_fma(-d, x, 1.0), x);
+    }
+    __device__ __forceinline__ double operator()(double a) const {
+        const double q = a * r;
+        return __builtin_fma(__builtin_fma(-b, q, a), r, q);
+    }
+};
+
+template <typename F>
+struct BoxLane {
+    dev::V3<F> pos, dir;
+    F path;                  // free path left
+    F vel;                   // FP32: sign / velocity (a flight's signed time is one product); FP64: velocity
+    F sg;                    // the bundle's sign
+    uint32_t nscat, nbdry, nstep;
+    int64_t id;
+};
+
+// A grid walk in progress (see WalkN).  `left` counts the entries still to
+// add (crossings and the last segment): the lane walks while it is positive.
+template <typename F, int NA>
+struct BoxWalk {
+    F t[NA], dt[NA];         // next crossing parameter per axis (2: none left) and the step between crossings
+    int32_t n[NA], dcol[NA];
+    int32_t left;
+    int32_t idx;
+    F prev;
+    double amt[kMaxRows];
+};
+template <typename F>
+struct BoxWalk<F, 0> {
+    int32_t left;
+};
+
+template <typename F>
+struct BoxView {
+    const uint64_t* scat;
+    const F* mfp;
+    const F* vel;            // FP32 in LDS: 1 / velocity; else velocity
+    const BoxFace<F>* faces;
+    double* tally;
+};
+
+template <typename F>
+__device__ __forceinline__ dev::V3<F> unit_of(const dev::V3<F>& v) {
+    if constexpr (sizeof(F) == 4) {
+        return dev::normalized(v);
+    } else {
+        const F n2 = v.x * v.x + v.y * v.y + v.z * v.z;
+        const Quotient q(sqrt(n2));
+        return n2 > F(0) ? dev::V3<F>{q(v.x), q(v.y), q(v.z)} : v;
+    }
+}
+
+// The pore wall's normal at p, away from the axis (FP64 divides by the radius
+// as the checker does).
+template <typename F>
+__device__ __forceinline__ dev::V3<F> box_wall_normal(const BoxCell<F>& B, const dev::V3<F>& p) {
+    if constexpr (sizeof(F) == 8) {
+        const Quotient q(B.r);
+        return unit_of(dev::V3<F>{q(p.x - B.cx), q(p.y - B.cy), F(0)});
+    } else {
+        return unit_of(dev::V3<F>{p.x - B.cx, p.y - B.cy, F(0)});
+    }
+}
+
+// A value the compiler must keep as it is: uniform parameters would otherwise
+// be read again from memory inside the step (a wait each), and what is derived
+// from them (the Philox round keys) held across the loop and spilled.
+// Scalar registers are short in these kernels and vector registers are not,
+// so what the vector instructions of a step use as operands is kept in vector
+// registers.
+template <typename T>
+__device__ __forceinline__ void in_vector(T& x) {
+    asm volatile("" : "+v"(x));
+}
+template <typename T>
+__device__ __forceinline__ void in_scalar(T& x) {
+    asm volatile("" : "+s"(x));
+}
+
+template <typename F, int kAxes>
+__device__ __forceinline__ void box_pin(BoxCell<F>& B) {
+    in_scalar(B.kinds);
+    in_scalar(B.maxscat);
+    in_scalar(B.maxloop);
+    in_scalar(B.cols);
+    if constexpr (sizeof(F) == 8 && kAxes != 0) return;   // these kernels have no vector registers left
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        in_vector(B.lo[a]);
+        in_vector(B.hi[a]);
+        if constexpr (sizeof(F) == 4) {
+            in_vector(B.klo[a]);
+            in_vector(B.khi[a]);
+        }
+    }
+    if constexpr (sizeof(F) == 8) in_vector(B.eps);
+#pragma unroll
+    for (int q = 0; q < (kAxes == 0 ? 1 : kAxes); ++q) {
+        in_vector(B.o[q]);
+        in_vector(B.inv[q]);
+        in_vector(B.div[q]);
+        in_vector(B.last[q]);
+    }
+}
+
+// The component of v a tally axis runs along: the masks are all ones for it
+// and zero for the others.
+__device__ __forceinline__ float pick3(const uint32_t (&m)[3], const dev::V3<float>& v) {
+    return __uint_as_float((__float_as_uint(v.x) & m[0]) | (__float_as_uint(v.y) & m[1]) | (__float_as_uint(v.z) & m[2]));
+}
+__device__ __forceinline__ double pick3(const uint32_t (&m)[3], const dev::V3<double>& v) {
+    const uint32_t lo = (uint32_t(__double2loint(v.x)) & m[0]) | (uint32_t(__double2loint(v.y)) & m[1]) |
+                        (uint32_t(__double2loint(v.z)) & m[2]);
+    const uint32_t hi = (uint32_t(__double2hiint(v.x)) & m[0]) | (uint32_t(__double2hiint(v.y)) & m[1]) |
+                        (uint32_t(__double2hiint(v.z)) & m[2]);
+    return __hiloint2double(int(hi), int(lo));
+}
+
+// One entry of a walk: the share up to the next crossing to the current cell,
+// then the axis of that crossing advances.  Crossings of two axes at the same
+// parameter are two entries, the first axis first, the second of zero length.
+// Written without branches: after the last segment the advance changes
+// nothing that is read again.
+template <bool kMulti, typename F, int NA>
+__device__ __forceinline__ void box_walk_next(BoxWalk<F, NA>& W, const BoxCell<F>& B, double* tally) {
+    F tm = W.t[0], dt = W.dt[0];
+    int32_t n = W.n[0], dcol = W.dcol[0];
+    bool later[NA];   // the crossing is of axis q or a later one
+    later[0] = true;
+#pragma unroll
+    for (int q = 1; q < NA; ++q) {
+        later[q] = W.t[q] < tm;
+        tm = later[q] ? W.t[q] : tm;
+        dt = later[q] ? W.dt[q] : dt;
+        n = later[q] ? W.n[q] : n;
+        dcol = later[q] ? W.dcol[q] : dcol;
+    }
+    const double seg = double((W.left == 1 ? F(1) : tm) - W.prev);
+    double* p = tally + W.idx;
+    if (kMulti || B.with_t) {
+        unsafeAtomicAdd(p, W.amt[0] * seg);
+        p += B.cols;
+    }
+    if (kMulti || B.with_f) {
+        unsafeAtomicAdd(p, W.amt[1] * seg);
+        p += B.cols;
+        unsafeAtomicAdd(p, W.amt[2] * seg);
+        p += B.cols;
+        unsafeAtomicAdd(p, W.amt[3] * seg);
+    }
+    W.left--;
+    W.prev = tm;
+    W.idx += dcol;
+    n--;
+    const F t = n > 0 ? tm + dt : F(2);
+#pragma unroll
+    for (int q = 0; q < NA; ++q) {
+        bool mine = later[q];
+#pragma unroll
+        for (int r = q + 1; r < NA; ++r) mine = mine && !later[r];
+        W.t[q] = mine ? t : W.t[q];
+        W.n[q] = mine ? n : W.n[q];
+    }
+}
+
+template <int U, bool kMulti, typename F, int NA>
+__device__ __forceinline__ void box_walk_some(BoxWalk<F, NA>& W, const BoxCell<F>& B, double* tally) {
+    if (W.left > 0) {
+        box_walk_next<kMulti>(W, B, tally);
+        if constexpr (U > 1) box_walk_some<U - 1, kMulti>(W, B, tally);
+    }
+}
+
+// Adds one row of a 1-D flight: the first and last cells' shares and the
+// crossed interior as a range.
+template <typename F>
+struct Span {
+    double *first, *last, *beg, *end;   // row 0's addresses: cells, range start and end in the difference array
+    F fb, fe, scale;                    // shares of the end cells; FP32: 1 / cells crossed
+    bool one, range;
+};
+
+template <int kRow, typename F>
+__device__ __forceinline__ void add_row(const Span<F>& s, F amt, F ca) {
+    unsafeAtomicAdd(s.first + kRow * kBoxCols, double(s.one ? amt : ca * s.fb));
+    if (!s.one) unsafeAtomicAdd(s.last + kRow * kBoxCols, double(ca * s.fe));
+    if (s.range) {
+        unsafeAtomicAdd(s.beg + kRow * kBoxCols, double(ca));
+        unsafeAtomicAdd(s.end + kRow * kBoxCols, -double(ca));
+    }
+}
+
+// The tally of a flight pre -> L.pos of length dmin: added at once along one
+// axis, set up in W for a grid.
+template <typename F, int kAxes, bool kMulti>
+__device__ __forceinline__ void box_tally(const BoxCell<F>& B, const BoxView<F>& V, const BoxLane<F>& L,
+                                          const dev::V3<F>& pre, F dmin, BoxWalk<F, kAxes>& W) {
+    F dt;
+    if constexpr (sizeof(F) == 4) dt = dmin * L.vel;
+    else dt = L.sg * Quotient(L.vel)(dmin);
+    const F dx = L.sg * (L.pos.x - pre.x), dy = L.sg * (L.pos.y - pre.y), dz = L.sg * (L.pos.z - pre.z);
+    if constexpr (kAxes == 0) {
+        if (B.tally == 0) return;
+        const F b = B.div[0] * (B.inv[0] * (pick3(B.comp[0], pre) - B.o[0]));
+        const F e = B.div[0] * (B.inv[0] * (pick3(B.comp[0], L.pos) - B.o[0]));
+        const int bb = min(max(int(floor(b)), 0), B.last[0]);
+        const int ee = min(max(int(floor(e)), 0), B.last[0]);
+        const bool up = bb < ee;
+        const int lo = min(bb, ee) + 1, hi = max(bb, ee);
+        Span<F> s;
+        s.one = bb == ee;
+        s.range = lo < hi;
+        s.fb = up ? F(1 + bb) - b : b - F(bb);
+        s.fe = up ? e - F(ee) : F(1 + ee) - e;
+        s.first = V.tally + bb;
+        s.last = V.tally + ee;
+        s.beg = V.tally + kMaxRows * kBoxCols + lo;
+        s.end = V.tally + kMaxRows * kBoxCols + hi;
+        if constexpr (sizeof(F) == 4) {
+            const F rad = __builtin_amdgcn_rcpf(fabsf(e - b));
+            if (kMulti || B.with_t) add_row<0>(s, dt, dt * rad);
+            if (kMulti || B.with_f) {
+                add_row<1>(s, dx, dx * rad);
+                add_row<2>(s, dy, dy * rad);
+                add_row<3>(s, dz, dz * rad);
+            }
+        } else {
+            const Quotient q(fabs(e - b));
+            if (kMulti || B.with_t) add_row<0>(s, dt, q(dt));
+            if (kMulti || B.with_f) {
+                add_row<1>(s, dx, q(dx));
+                add_row<2>(s, dy, q(dy));
+                add_row<3>(s, dz, q(dz));
+            }
+        }
+    } else {
+        int idx = 0, left = 1;
+#pragma unroll
+        for (int q = 0; q < kAxes; ++q) {
+            const F b = B.div[q] * (B.inv[q] * (pick3(B.comp[q], pre) - B.o[q]));
+            const F e = B.div[q] * (B.inv[q] * (pick3(B.comp[q], L.pos) - B.o[q]));
+            const int bk = min(max(int(floor(b)), 0), B.last[q]);
+            const int ek = min(max(int(floor(e)), 0), B.last[q]);
+            const F dc = e - b;
+            const bool up = bk < ek;
+            idx += bk * B.stride[q];
+            const F first = F(up ? bk + 1 : bk) - b;
+            const int n = up ? ek - bk : bk - ek;
+            bool none;
+            F t;
+            if constexpr (sizeof(F) == 4) {
+                none = (fabsf(dc) < FLT_MIN) | (n == 0);
+                const F r = __builtin_amdgcn_rcpf(dc);
+                t = first * r;
+                W.dt[q] = fabsf(r);
+            } else {
+                none = (fabs(dc) < DBL_MIN) | (n == 0);
+                const Quotient d(none ? F(1) : dc);
+                t = d(first);
+                W.dt[q] = fabs(d(F(1)));
+            }
+            W.t[q] = none ? F(2) : t;
+            W.n[q] = none ? 0 : n;
+            left += none ? 0 : n;
+            W.dcol[q] = up ? B.stride[q] : -B.stride[q];
+        }
+        W.idx = idx;
+        W.prev = F(0);
+        W.left = left;
+        W.amt[0] = double(dt);
+        W.amt[1] = double(dx);
+        W.amt[2] = double(dy);
+        W.amt[3] = double(dz);
+    }
+}
+
+// One scatter-step: the flight (problem.cpp:401-416) and the event
+// (problem.cpp:418-433), as flight_step and collide_step take them.  Returns
+// the bundle's fate, kAlive while it lives.
+template <typename F, bool kLdsTables, int kAxes, bool kMulti>
+__device__ __forceinline__ uint32_t box_step(const BoxCell<F>& B, const BoxView<F>& V, BoxLane<F>& L,
+                                             BoxWalk<F, kAxes>& W) {
+    // ---- flight: the face ahead on each axis, the pore, the free path
+    const F p[3] = {L.pos.x, L.pos.y, L.pos.z}, u[3] = {L.dir.x, L.dir.y, L.dir.z};
+    F dmin = L.path;
+    uint32_t hit = kCodeIntrinsic;
+    int plane = -1;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const bool up = u[a] > F(0);
+        const uint32_t code = up ? 8u * a + 4u : 8u * a;
+        if constexpr (sizeof(F) == 4) {
+            // a face that rounding left just behind is met where the bundle stands
+            const F ta = ((up ? B.hi[a] : B.lo[a]) - p[a]) * __builtin_amdgcn_rcpf(u[a]);
+            const F t = ta < F(0) ? F(0) : ta;
+            const bool take = (u[a] != F(0)) & (t < dmin);
+            dmin = take ? t : dmin;
+            hit = take ? code : hit;
+        } else {
+            // -(c + n.p) / (n.u) of the checker's face loop: the normal's
+            // other components are zeros and its sign cancels.  Equal
+            // parameters keep the lower face number.
+            const F t = Quotient(u[a])((up ? B.hi[a] : B.lo[a]) - p[a]);
+            const int pl = int((B.planes >> code) & 15u);
+            const bool take = (u[a] != F(0)) & ((t < dmin) | ((t == dmin) & (plane >= 0) & (pl < plane)));
+            dmin = take ? t : dmin;
+            hit = take ? code : hit;
+            plane = take ? pl : plane;
+        }
+    }
+    if (B.pore >= 0) {
+        const F dx = p[0] - B.cx, dy = p[1] - B.cy;
+        const F bq = dx * u[0] + dy * u[1];
+        const F aq = u[0] * u[0] + u[1] * u[1];
+        const F cq = dx * dx + dy * dy - B.r2;
+        const F disc = bq * bq - aq * cq;
+        if ((bq < F(0)) & (disc >= F(0))) {
+            // a start on (or, by rounding, just inside) the wall heading in
+            // meets it at once
+            const F t = cq <= F(0) ? F(0) : dev::Real<F>::div(cq, dev::Real<F>::sqrt_(disc) - bq);
+            hit = t < dmin ? uint32_t(kCodePore) : hit;
+            dmin = t < dmin ? t : dmin;
+        }
+    }
+    L.path -= dmin;
+    if (L.path < dev::Real<F>::kMin) L.path = F(0);
+    const dev::V3<F> pre = L.pos;
+    L.pos = dev::V3<F>{pre.x + dmin * u[0], pre.y + dmin * u[1], pre.z + dmin * u[2]};
+    L.nstep++;
+    // kill test (subdomain.cpp:186-190)
+    bool outside;
+    if constexpr (sizeof(F) == 4) {
+        outside = (L.pos.x < B.klo[0]) | (L.pos.x > B.khi[0]) | (L.pos.y < B.klo[1]) | (L.pos.y > B.khi[1]) |
+                  (L.pos.z < B.klo[2]) | (L.pos.z > B.khi[2]);
+    } else {
+        outside = (dmin < -B.eps) | (L.pos.x - B.lo[0] < -B.eps) | (B.hi[0] - L.pos.x < -B.eps) |
+                  (L.pos.y - B.lo[1] < -B.eps) | (B.hi[1] - L.pos.y < -B.eps) | (L.pos.z - B.lo[2] < -B.eps) |
+                  (B.hi[2] - L.pos.z < -B.eps);
+    }
+    if (B.pore >= 0) {
+        const F dx = L.pos.x - B.cx, dy = L.pos.y - B.cy;
+        outside |= dx * dx + dy * dy < B.rin2;
+    }
+    uint32_t fate = MCG_ESCAPED;
+    if (!outside) {
+        box_tally<F, kAxes, kMulti>(B, V, L, pre, dmin, W);
+
+        // ---- event
+        uint32_t kind = (B.kinds >> hit) & 15u;
+        const bool intr = kind == kKindIntrinsic;
+        bool pore = false;
+        if (B.pore >= 0) {
+            pore = kind == kKindPore;
+            kind = pore ? uint32_t(B.pore) : kind;
+        }
+        uint32_t k0 = B.k0, k1 = B.k1;
+        in_scalar(k0);
+        in_scalar(k1);
+        const dev::Event ev{k0, k1, L.nstep, uint32_t(L.id), uint32_t(uint64_t(L.id) >> 32)};
+        const BoxFace<F>& P = V.faces[hit < kCodeIntrinsic ? hit >> 2 : 0u];
+        if (B.partial) {
+            if (kind == MCG_PARTIAL)
+                kind = ev.block(1).w < (pore ? B.pore_thr : P.spec_thr) ? uint32_t(MCG_SPEC) : uint32_t(MCG_DIFF);
+        }
+        L.nbdry += intr ? 0u : 1u;
+        const bool draws = intr | (kind == MCG_DIFF);
+        dev::V3<F> d = L.dir;
+        if (draws) {
+            // the event's random direction: isotropic cos(theta) = r or
+            // Lambertian sin^2(theta) = |r| about z, then turned onto the normal
+            const uint4 b0 = ev.block(0), b1 = low_block<F>(ev, 1);
+            const F r = dev::Real<F>::uniform(b0.x, b1.x) * F(2) + F(-1);
+            const F ar = r < F(0) ? -r : r;
+            const F sinT = dev::Real<F>::sqrt_(intr ? F(1) - r * r : ar);
+            const F cosT = intr ? r : dev::Real<F>::sqrt_(F(1) - ar);
+            const F q = dev::Real<F>::uniform(b0.y, b1.y) * F(2) + F(-1);
+            F sq, cq;
+            dev::Real<F>::sincos_pi(q, sq, cq);
+            d = dev::V3<F>{sinT * cq, sinT * sq, cosT};
+            L.nscat++;
+            if (intr) {
+                const uint32_t mode = dev::alias_draw(V.scat, uint32_t(B.nmodes), b0.w);
+                const F mfp = V.mfp[mode], vel = V.vel[mode];
+                L.path = draw_path<F>(ev, b0, b1, mfp);
+                if constexpr (sizeof(F) == 8) L.vel = vel;
+                else if constexpr (kLdsTables) L.vel = L.sg * vel;
+                else L.vel = L.sg * __builtin_amdgcn_rcpf(vel);
+            } else {
+                F m[9];
+#pragma unroll
+                for (int i = 0; i < 9; ++i) m[i] = P.rot[i];
+                if (pore) rotation_to_wall(box_wall_normal(B, L.pos), m);
+                d = dev::matvec(m, d);
+            }
+        }
+        if (kind == MCG_SPEC) {
+            // I - 2 n n^T of an axis: the component's sign
+            const uint32_t axis = hit >> 3;
+            d.x = axis == 0u ? -d.x : d.x;
+            d.y = axis == 1u ? -d.y : d.y;
+            d.z = axis == 2u ? -d.z : d.z;
+            if (pore) {
+                F m[9];
+                reflection_off(box_wall_normal(B, L.pos), m);
+                d = dev::matvec(m, L.dir);
+            }
+        }
+        if (kind == MCG_PERI) {
+            // the map's rotation is the identity (box_cell takes no other)
+            L.pos = dev::V3<F>{L.pos.x + P.pt[0], L.pos.y + P.pt[1], L.pos.z + P.pt[2]};
+        }
+        L.dir = unit_of(d);
+        fate = L.nstep >= B.maxloop ? uint32_t(MCG_MAXLOOP) : kAlive;
+        fate = L.nscat >= B.maxscat ? uint32_t(MCG_MAXSCAT) : fate;
+        fate = kind == MCG_ISOT ? uint32_t(MCG_ABSORBED) : fate;
+    }
+    return fate;
+}
+
+// Kernel parameters read where they are used: the pointer goes through an
+// opaque move, so that the loads stay in the (rare) emission rounds instead of
+// being held in scalar registers across the loop and spilled.
+template <typename F>
+using ParamPtr = const __attribute__((address_space(4))) KParams<F>*;
+
+template <typename F>
+__device__ __forceinline__ ParamPtr<F> params_here(ParamPtr<F> kp) {
+    asm volatile("" : "+s"(kp));
+    return kp;
+}
+
+// A pointer that the parameters hold, known to point to global memory (read
+// from memory it would be addressed as generic).
+template <typename T>
+__device__ __forceinline__ T* in_global(T* p) {
+    return (T*)(__attribute__((address_space(1))) T*)p;
+}
+
+// LDS layout: [scat alias | mfp | vel] (when kLdsTables), faces, tally.
+template <typename F>
+__host__ __device__ inline size_t box_lds_tables(int nmodes) {
+    return (size_t(nmodes) * (8 + 2 * sizeof(F)) + 15) & ~size_t(15);
+}
+
+// doubles of the LDS tally: fixed strides for a 1-D tally, rows x cols for a grid
+template <typename F>
+__host__ __device__ inline int box_tally_doubles(const BoxCell<F>& B) {
+    return B.tally == 1 ? 2 * kMaxRows * kBoxCols : (B.tally == 2 ? B.rows * B.cols : 0);
+}
+
+template <typename F, bool kLdsTables>
+__device__ __forceinline__ BoxView<F> box_stage(ParamPtr<F> kp, const BoxCell<F>& B, unsigned char* lds,
+                                                int tid, int nthreads) {
+    const uint64_t* const g_scat = in_global(kp->scat_alias);
+    const F* const g_mfp = in_global(kp->mode_mfp);
+    const F* const g_vel = in_global(kp->mode_vel);
+    BoxView<F> v;
+    size_t off = 0;
+    if constexpr (kLdsTables) {
+        const int n = B.nmodes;
+        uint64_t* s = reinterpret_cast<uint64_t*>(lds);
+        F* m = reinterpret_cast<F*>(lds + 8 * size_t(n));
+        F* q = m + n;
+        for (int i = tid; i < n; i += nthreads) {
+            s[i] = g_scat[i];
+            m[i] = g_mfp[i];
+            const F vel = g_vel[i];
+            if constexpr (sizeof(F) == 4) q[i] = __builtin_amdgcn_rcpf(vel);
+            else q[i] = vel;
+        }
+        v.scat = s;
+        v.mfp = m;
+        v.vel = q;
+        off = box_lds_tables<F>(n);
+    } else {
+        v.scat = g_scat;
+        v.mfp = g_mfp;
+        v.vel = g_vel;
+    }
+    BoxFace<F>* f = reinterpret_cast<BoxFace<F>*>(lds + off);
+    if (tid < 6) {
+        const DevPlane<F>& P = in_global(kp->planes)[(B.planes >> (4 * tid)) & 15u];
+        for (int i = 0; i < 9; ++i) f[tid].rot[i] = P.rot[i];
+        for (int i = 0; i < 3; ++i) f[tid].pt[i] = P.pt[i];
+        f[tid].spec_thr = P.spec_thr;
+    }
+    v.faces = f;
+    v.tally = reinterpret_cast<double*>(lds + off + 6 * sizeof(BoxFace<F>));
+    const int nt = box_tally_doubles(B);
+    for (int i = tid; i < nt; i += nthreads) v.tally[i] = 0.0;
+    return v;
+}
+
+// Adds a workgroup's LDS tally into the solve's global tally (after a barrier).
+template <typename F>
+__device__ __forceinline__ void box_flush(ParamPtr<F> kp, const BoxCell<F>& B, const double* tally, int tid,
+                                          int nthreads) {
+    double* const direct = in_global(kp->direct);
+    double* const diff = in_global(kp->diff);
+    if (B.tally == 1) {
+        // LDS rows 0..3 are T, qx, qy, qz; the solve's first row is its first kind
+        const int r0 = B.with_t ? 0 : 1;
+        for (int i = tid; i < B.rows * kBoxCols; i += nthreads) {
+            const int r = i / kBoxCols, c = i % kBoxCols;
+            const double a = tally[(r0 + r) * kBoxCols + c], d = tally[(kMaxRows + r0 + r) * kBoxCols + c];
+            if (a != 0.0 && c < B.cols) unsafeAtomicAdd(direct + r * B.cols + c, a);
+            if (d != 0.0 && c <= B.cols) unsafeAtomicAdd(diff + r * (B.cols + 1) + c, d);
+        }
+    } else if (B.tally == 2) {
+        for (int i = tid; i < B.rows * B.cols; i += nthreads) {
+            const double a = tally[i];
+            if (a != 0.0) unsafeAtomicAdd(direct + i, a);
+        }
+    }
+}
+
+// Emission into a box lane (emit of the general path).
+template <typename F, bool kLdsTables>
+__device__ __forceinline__ void box_emit(ParamPtr<F> kp, const BoxCell<F>& B, const BoxView<F>& V, int64_t n,
+                                         BoxLane<F>& L) {
+    KParams<F> K;
+    K.emitters = in_global(kp->emitters);
+    K.emit_cdf = in_global(kp->emit_cdf);
+    K.sdoms = in_global(kp->sdoms);
+    K.pores = in_global(kp->pores);
+    K.nemitter = kp->nemitter;
+    K.npore = kp->npore;
+    K.nmodes = B.nmodes;
+    K.k0 = kp->k0;
+    K.k1 = kp->k1;
+    Lane<F> T;
+    emit<F>(K, in_global(kp->flux_alias), V.mfp, n, T);
+    L.pos = T.pos;
+    L.dir = T.dir;
+    L.path = T.scat_next;
+    L.sg = F(T.sign);
+    if constexpr (sizeof(F) == 8) L.vel = V.vel[T.mode];
+    else if constexpr (kLdsTables) L.vel = L.sg * V.vel[T.mode];
+    else L.vel = L.sg * __builtin_amdgcn_rcpf(V.vel[T.mode]);
+    L.nscat = L.nbdry = L.nstep = 0;
+    L.id = n;
+}
+
+// A wavefront's loop over the bundles it claims (trajectory_kernel's loop).
+// The refill is looked at only when some lane has run out of work since the
+// last look: a wavefront left with a few long-lived bundles goes from step to
+// step without it.
+template <typename F, bool kLdsTables, int kAxes, bool kMulti>
+__device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, const BoxView<F>& V, int lane) {
+    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
+    int64_t pool_base = 0, pool_lim = 0, seen = 0;
+    bool active = false, full = false, drained = false;
+    BoxLane<F> L, N;
+    BoxWalk<F, kAxes> W;
+    W.left = 0;
+    unsigned long long steps = 0, n_end = 0, n_abs = 0, n_esc = 0;   // wavefront-uniform
+    uint64_t busy = ~0ull, last_busy = 0ull;
+    for (;;) {
+        if (busy != last_busy || busy == 0ull) {
+            const bool walking = W.left > 0;
+            const ParamPtr<F> k = params_here<F>(kp);
+            const int64_t count = k->count;
+            if constexpr (sizeof(F) == 4) {
+                if (!active && !walking && full) {
+                    L = N;
+                    full = false;
+                    active = true;
+                }
+                const bool near_end = count - seen < k->tail;
+                const bool empty = !full && !drained && (!near_end || (!active && !walking));
+                const uint64_t me = __ballot(empty);
+                if (me != 0ull && (popc(me) >= kSlotQuorum || popc(__ballot(empty && !active && !walking)) >= kEmitQuorum ||
+                                   __ballot(active || walking) == 0ull)) {
+                    const int64_t mine = claim(empty, lane, lt_mask, pool_base, pool_lim, in_global(k->next), k->chunk, count,
+                                               k->tail, &seen);
+                    if (empty) {
+                        if (mine < count) {
+                            box_emit<F, kLdsTables>(k, B, V, k->first + mine, N);
+                            full = true;
+                        } else {
+                            drained = true;
+                        }
+                    }
+                    if (!active && !walking && full) {
+                        L = N;
+                        full = false;
+                        active = true;
+                    }
+                }
+                if (__ballot(active || walking || full || !drained) == 0ull) break;
+            } else {
+                const bool need = !active && !drained && !walking;
+                if (emit_now<kEmitQuorumFp64>(need, active || walking)) {
+                    const int64_t mine = claim(need, lane, lt_mask, pool_base, pool_lim, in_global(k->next), k->chunk);
+                    if (need) {
+                        if (mine < count) {
+                            box_emit<F, kLdsTables>(k, B, V, k->first + mine, L);
+                            active = true;
+                        } else {
+                            drained = true;
+                        }
+                    }
+                }
+                if (__ballot(active || walking) == 0ull) break;
+            }
+            last_busy = __ballot(active || walking);
+        }
+        const bool go = active && !(W.left > 0);
+        steps += popc(__ballot(go));
+        uint32_t fate = kAlive;
+        if (go) fate = box_step<F, kLdsTables, kAxes, kMulti>(B, V, L, W);
+        const uint64_t ended = __ballot(fate != kAlive);
+        if (ended != 0ull) {
+            n_end += popc(ended);
+            n_abs += popc(__ballot(fate == MCG_ABSORBED));
+            n_esc += popc(__ballot(fate == MCG_ESCAPED));
+            if (fate != kAlive) {
+                active = false;
+                if (B.counts) {
+                    const ParamPtr<F> k = params_here<F>(kp);
+                    const int64_t i = L.id - k->first;
+                    in_global(k->c_nscat)[i] = L.nscat;
+                    in_global(k->c_nbdry)[i] = L.nbdry;
+                    in_global(k->c_nstep)[i] = L.nstep;
+                    in_global(k->c_fate)[i] = fate;
+                }
+            }
+        }
+        if constexpr (kAxes != 0) {
+            // the walk phase (walk_phase): while kWalkQuorum lanes walk or no
+            // other lane has a step to take
+            for (;;) {
+                const uint64_t m = __ballot(W.left > 0);
+                if (m == 0ull || (popc(m) < kWalkQuorum && __ballot(active && !(W.left > 0)) != 0ull)) break;
+                box_walk_some<kWalkUnroll, kMulti>(W, B, V.tally);
+            }
+        }
+        busy = __ballot(active || W.left > 0);
+    }
+    if (lane == 0 && n_end != 0) {
+        unsigned long long* const c = in_global(params_here<F>(kp)->counters);
+        atomicAdd(c + C_STEPS, steps);
+        atomicAdd(c + C_ESC, n_esc);
+        atomicAdd(c + C_ABS, n_abs);
+        atomicAdd(c + C_TRUNC, n_end - n_abs - n_esc);
+        atomicAdd(c + C_BUNDLES, n_end);
+    }
+}
+
+// A solve of a one-box scene (the kernel parameters come first: params_here
+// reads them through the kernel-argument segment).
+template <typename F, bool kLdsTables, int kAxes, bool kMulti>
+__global__ void __launch_bounds__(1024) box_kernel(KParams<F> Karg, BoxCell<F> Barg) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int tid = threadIdx.x;
+    const ParamPtr<F> kp = (ParamPtr<F>)__builtin_amdgcn_kernarg_segment_ptr();
+    BoxCell<F> B = Barg;
+    box_pin<F, kAxes>(B);
+    const BoxView<F> V = box_stage<F, kLdsTables>(params_here<F>(kp), B, lds, tid, blockDim.x);
+    __syncthreads();
+    box_run<F, kLdsTables, kAxes, kMulti>(B, kp, V, tid & (kWave - 1));
+    __syncthreads();
+    box_flush(params_here<F>(kp), B, V.tally, tid, blockDim.x);
+}

@@ -633,6 +633,38 @@ __device__ __forceinline__ bool accumulate(const DevSdom<F>& S, const Sink& sink
     }
 }
 
+// I - 2 n n^T of a pore wall's normal (column-major).
+template <typename F>
+__device__ __forceinline__ void reflection_off(const dev::V3<F>& n, F (&r)[9]) {
+    const F nv[3] = {n.x, n.y, n.z};
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) r[3 * c + q] = (q == c ? F(1) : F(0)) - F(2) * (nv[q] * nv[c]);
+}
+
+// The rotation taking z onto a pore wall's normal (n.z = 0, so never the
+// antiparallel case; column-major).
+template <typename F>
+__device__ __forceinline__ void rotation_to_wall(const dev::V3<F>& n, F (&r)[9]) {
+    const F s = dev::Real<F>::sqrt_((F(1) + n.z) * F(2));
+    const F invs = F(1) / s;
+    const F qx = -n.y * invs, qy = n.x * invs, qz = F(0) * invs, qw = s * F(0.5);
+    const F tx = F(2) * qx, ty = F(2) * qy, tz = F(2) * qz;
+    const F twx = tx * qw, twy = ty * qw, twz = tz * qw;
+    const F txx = tx * qx, txy = ty * qx, txz = tz * qx;
+    const F tyy = ty * qy, tyz = tz * qy, tzz = tz * qz;
+    r[0] = F(1) - (tyy + tzz);
+    r[1] = txy + twz;
+    r[2] = txz - twy;
+    r[3] = txy - twz;
+    r[4] = F(1) - (txx + tzz);
+    r[5] = tyz + twx;
+    r[6] = txz + twy;
+    r[7] = tyz - twx;
+    r[8] = F(1) - (txx + tyy);
+}
+
 // Scatter off a cylindrical pore wall.  The wall normal at the hit point
 // points away from the axis (into the material); the reflection and the
 // Lambertian rotation are built from it as for a planar face.
@@ -648,27 +680,13 @@ __device__ __forceinline__ void pore_scatter(const DevPore<F>& Q, const dev::Eve
         n = dev::normalized(dev::V3<F>{L.pos.x - Q.cx, L.pos.y - Q.cy, F(0)});
     int kind = Q.kind;
     if (kind == MCG_PARTIAL) kind = spec_word<F>(ev, b1) < Q.spec_thr ? MCG_SPEC : MCG_DIFF;
+    F r[9];
     if (kind == MCG_SPEC) {
-        const F nv[3] = {n.x, n.y, n.z};
-        F r[9];
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-#pragma unroll
-            for (int q = 0; q < 3; ++q) r[3 * c + q] = (q == c ? F(1) : F(0)) - F(2) * (nv[q] * nv[c]);
+        reflection_off(n, r);
         L.dir = dev::normalized(dev::matvec(r, L.dir));
         return;
     }
-    // rotation taking z onto n (n.z = 0, so never the antiparallel case)
-    const F s = dev::Real<F>::sqrt_((F(1) + n.z) * F(2));
-    const F invs = F(1) / s;
-    const F qx = -n.y * invs, qy = n.x * invs, qz = F(0) * invs, qw = s * F(0.5);
-    const F tx = F(2) * qx, ty = F(2) * qy, tz = F(2) * qz;
-    const F twx = tx * qw, twy = ty * qw, twz = tz * qw;
-    const F txx = tx * qx, txy = ty * qx, txz = tz * qx;
-    const F tyy = ty * qy, tyz = tz * qy, tzz = tz * qz;
-    const F r[9] = {F(1) - (tyy + tzz), txy + twz, txz - twy,
-                    txy - twz, F(1) - (txx + tzz), tyz + twx,
-                    txz + twy, tyz - twx, F(1) - (txx + tyy)};
+    rotation_to_wall(n, r);
     L.dir = dev::normalized(dev::matvec(r, dev::draw_aniso<F>(b0, b1, false)));
     L.nscat++;
 }
@@ -1347,6 +1365,8 @@ __device__ __forceinline__ int64_t claim(bool need, int lane, uint64_t lt_mask, 
     }
     return mine;
 }
+
+#include "mcg_box.h"
 
 // Single solve: persistent grid, every lane refilled from the solve's global
 // bundle counter until the range [first, first + count) is exhausted.
@@ -2159,6 +2179,131 @@ void fill_params(mcg_scene* sc, const HostProblem& p, KParams<F>& K) {
     K.trace_id = -1;
 }
 
+// The wavefront-uniform description of a scene that is one axis-aligned box
+// (mcg_box.h); false when the scene or the problem needs the general kernel:
+//  - faces other than specular, diffuse, partial, isothermal or periodic onto
+//    the box itself by a pure translation along the face's axis;
+//  - a tally by scatter order (more than kMaxRows rows), a 1-D tally of more
+//    than kBoxCols - 1 cells (the fixed LDS stride), grid axes that are not
+//    x, y, z in order;
+//  - maxscat past 32 bits (the step compares 32-bit counts).
+// Its values are those of the uploaded records, so a step's operands are the
+// general kernel's.
+template <typename F>
+bool box_cell(const HostScene& h, const HostProblem& p, BoxCell<F>& B) {
+    if (h.sdoms.size() != 1 || !h.sdoms[0].box || h.planes.size() != 6 || p.rows > kMaxRows ||
+        p.tally > MCG_MULTI || p.maxscat > 0xFFFFFFFEll)
+        return false;
+    DevSdom<F> S;
+    convert_sdom(h.sdoms[0], S, sizeof(F) == 4 ? double(FLT_EPSILON) / DBL_EPSILON : 1.0);
+    B = BoxCell<F>{};
+    B.kinds = (uint32_t(kKindIntrinsic) << kCodeIntrinsic) | (uint32_t(kKindPore) << kCodePore);
+    for (int a = 0; a < 3; ++a) {
+        B.lo[a] = S.bmin[a];
+        B.hi[a] = S.bmax[a];
+        B.klo[a] = S.kmin[a];
+        B.khi[a] = S.kmax[a];
+        for (int up = 0; up < 2; ++up) {
+            const int pl = S.pbeg + (up ? S.fmax[a] : S.fmin[a]);
+            DevPlane<F> P;
+            convert_plane(h.planes[pl], P);
+            if (P.kind == MCG_INTER) return false;
+            if (P.kind == MCG_PARTIAL) B.partial = 1;
+            if (P.kind == MCG_PERI) {
+                if (P.target != 0) return false;
+                for (int i = 0; i < 9; ++i)
+                    if (P.prot[i] != (i % 4 == 0 ? F(1) : F(0))) return false;
+            }
+            const uint32_t code = 8u * a + 4u * up;
+            B.kinds |= uint32_t(P.kind) << code;
+            B.planes |= uint32_t(pl) << code;
+        }
+    }
+    B.eps = S.eps;
+    B.maxscat = uint32_t(p.maxscat);
+    B.maxloop = uint32_t(std::min<int64_t>(p.maxloop, 0xFFFFFFFEll));
+    B.k0 = uint32_t(p.seed);
+    B.k1 = uint32_t(p.seed >> 32);
+    B.nmodes = int32_t(h.mode_cell.size());
+    B.rows = int32_t(p.rows);
+    B.cols = int32_t(h.cols);
+    B.with_t = p.tally == MCG_TEMP || p.tally == MCG_MULTI;
+    B.with_f = p.tally == MCG_FLUX || p.tally == MCG_MULTI;
+    // tally axes: coordinate k = div_k inv_k . (p - o); one nonzero entry per
+    // row of inv, so the other products are exact zeros
+    int axes[3], na = 0;
+    if (S.accum == -1) axes[na++] = 0;
+    else if (S.accum >= 0 && S.accum < 3) axes[na++] = S.accum;
+    else if (S.accum == 3) {
+        axes[na++] = S.gax[0];
+        axes[na++] = S.gax[1];
+    } else if (S.accum == 4) {
+        for (int k = 0; k < 3; ++k) axes[na++] = k;
+    }
+    B.tally = S.accum < -1 ? 0 : (S.accum < 3 ? 1 : 2);
+    for (int q = 0; q < na; ++q) {
+        const int k = axes[q];
+        int c = -1;
+        for (int j = 0; j < 3; ++j)
+            if (S.inv[k + 3 * j] != F(0)) {
+                if (c >= 0) return false;
+                c = j;
+            }
+        if (c < 0) return false;
+        B.comp[q][c] = 0xFFFFFFFFu;
+        B.o[q] = S.o[c];
+        B.inv[q] = S.inv[k + 3 * c];
+        B.div[q] = S.accum == -1 ? F(0) : S.divf[k];
+        B.last[q] = S.accum == -1 ? 0 : S.max[k];
+        B.stride[q] = S.stride[k];
+    }
+    if (B.tally != 0 && S.col_off != 0) return false;
+    if (B.tally == 1 && B.cols >= kBoxCols) return false;
+    B.pore = -1;
+    if (S.pore >= 0) {
+        DevPore<F> Q;
+        convert_pore(h.pores[S.pore], Q, sizeof(F) == 4 ? double(FLT_EPSILON) / DBL_EPSILON : 1.0);
+        const F rr = Q.r - Q.eps;
+        B.pore = Q.kind;
+        if (Q.kind == MCG_PARTIAL) B.partial = 1;
+        B.cx = Q.cx;
+        B.cy = Q.cy;
+        B.r = Q.r;
+        B.r2 = Q.r2;
+        B.rin2 = rr * rr;
+        B.pore_thr = Q.spec_thr;
+    }
+    return true;
+}
+
+// The box kernel of a tally (axes of its grid, 0 without one; all four Multi
+// rows or any) and of tables staged in LDS or read from global memory.
+template <typename F, int kAxes>
+const void* pick_box_kernel(bool tables, bool multi) {
+    if (multi)
+        return tables ? reinterpret_cast<const void*>(box_kernel<F, true, kAxes, true>)
+                      : reinterpret_cast<const void*>(box_kernel<F, false, kAxes, true>);
+    return tables ? reinterpret_cast<const void*>(box_kernel<F, true, kAxes, false>)
+                  : reinterpret_cast<const void*>(box_kernel<F, false, kAxes, false>);
+}
+template <typename F>
+const void* pick_box_kernel(bool tables, bool multi, int axes) {
+    return axes == 0 ? pick_box_kernel<F, 0>(tables, multi)
+                     : (axes == 2 ? pick_box_kernel<F, 2>(tables, multi) : pick_box_kernel<F, 3>(tables, multi));
+}
+
+// LDS of a box launch: the faces and the tally, and the tables when they fit
+// beside them.  False when the tally does not fit.
+template <typename F>
+bool box_lds_plan(const BoxCell<F>& B, bool tables_allowed, size_t limit, bool& tables, size_t& bytes) {
+    bytes = 6 * sizeof(BoxFace<F>) + size_t(box_tally_doubles(B)) * sizeof(double);
+    if (bytes > limit) return false;
+    const size_t tab = box_lds_tables<F>(B.nmodes);
+    tables = tables_allowed && bytes + tab <= limit;
+    if (tables) bytes += tab;
+    return true;
+}
+
 // Clears tallies and counters: one launch instead of several memsets, and
 // usable inside a captured graph (memset nodes in captured graphs are
 // avoided).
@@ -2185,6 +2330,24 @@ __global__ void fold_copies_kernel(double* a, size_t n, const double* priv, size
 // Private copies of a tally that stays in global memory (one per XCD)
 constexpr int kTallyCopies = 8;
 
+// Launch of a one-box solve.
+template <typename F>
+int launch_box(mcg_scene* sc, const HostProblem& p, KParams<F>& K, BoxCell<F>& cell, const void* fn, size_t lds,
+               hipStream_t stream) {
+    HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+    int per_cu = std::max<int>(1, int(sc->lds_limit / lds));
+    const int block = sc->tune.block > 0 ? sc->tune.block : (per_cu == 1 ? 1024 : 512);
+    per_cu = std::min(per_cu, std::max(1, 2048 / block));
+    if (sc->tune.blocks_per_cu > 0) per_cu = std::min(per_cu, int(sc->tune.blocks_per_cu));
+    const int64_t needed = (p.count + block - 1) / block;
+    const int grid = int(std::max<int64_t>(1, std::min<int64_t>(int64_t(sc->num_cu) * per_cu, needed)));
+    K.tail = int64_t(MCG_TAIL_LANES) * grid * block;
+    void* args[] = {&K, &cell};
+    HIP_TRY(hipLaunchKernel(fn, dim3(grid), dim3(block), args, lds, stream));
+    HIP_TRY(hipGetLastError());
+    return MCG_OK;
+}
+
 // Launch shape and LDS plan of a single solve, then the launch on `stream`
 // (K holds the solve's buffers; its LDS and tail fields are set here).
 template <typename F>
@@ -2192,6 +2355,16 @@ int launch_solve(mcg_scene* sc, const HostProblem& p, KParams<F>& K, hipStream_t
                  bool may_allocate = false) {
     const HostScene& h = sc->host;
     const int rows = int(p.rows);
+    BoxCell<F> cell;
+    bool box_tables = false;
+    size_t box_lds = 0;
+    if (K.trace_id < 0 && !(h.has_grid && sc->tune.defer_walks < 0) && box_cell<F>(h, p, cell) &&
+        box_lds_plan<F>(cell, sc->tune.lds_tables >= 0, sc->lds_limit, box_tables, box_lds)) {
+        cell.counts = K.c_nscat != nullptr;
+        const int axes = cell.tally == 2 ? (h.grid_2d ? 2 : 3) : 0;
+        return launch_box<F>(sc, p, K, cell, pick_box_kernel<F>(box_tables, p.tally == MCG_MULTI && cell.tally != 0, axes),
+                             box_lds, stream);
+    }
     const size_t geo = lds_bytes<F>(h, rows, false, false);
     const LdsPlan lp = plan_lds(geo, lds_bytes<F>(h, rows, true, false) - geo,
                                 lds_bytes<F>(h, rows, false, true) - geo, h.has_grid,
