@@ -68,7 +68,11 @@ struct BoxCell {
     int32_t partial;         // some wall is partially specular
     // tally: 0 none, 1 along one axis (a single cell is one axis of one
     // cell), 2 a grid walked over its divided axes
-    int32_t tally, with_t, with_f, rows, cols;
+    // rowmask: the quantities tallied (bit 0 T, 1-3 the flux components);
+    // rows, cols: shape of the LDS tally, from row0, col0 of the solve's map
+    // of gcols columns (the whole map, or the part of it this workgroup tallies)
+    int32_t tally, rowmask, rows, cols, row0, col0, gcols;
+    int32_t part, parts, colparts;   // see box_part
     uint32_t comp[3][3];                   // per tally axis: mask of each position component
     int32_t last[3], stride[3];            // largest index, column stride
     F o[3], inv[3], div[3];                // cell coordinate = div (inv (p - o))
@@ -213,7 +217,7 @@ __device__ __forceinline__ double pick3(const uint32_t (&m)[3], const dev::V3<do
 // parameter are two entries, the first axis first, the second of zero length.
 // Written without branches: after the last segment the advance changes
 // nothing that is read again.
-template <bool kMulti, typename F, int NA>
+template <int kRows, typename F, int NA>
 __device__ __forceinline__ void box_walk_next(BoxWalk<F, NA>& W, const BoxCell<F>& B, double* tally) {
     F tm = W.t[0], dt = W.dt[0];
     int32_t n = W.n[0], dcol = W.dcol[0];
@@ -229,16 +233,17 @@ __device__ __forceinline__ void box_walk_next(BoxWalk<F, NA>& W, const BoxCell<F
     }
     const double seg = double((W.left == 1 ? F(1) : tm) - W.prev);
     double* p = tally + W.idx;
-    if (kMulti || B.with_t) {
-        unsafeAtomicAdd(p, W.amt[0] * seg);
-        p += B.cols;
-    }
-    if (kMulti || B.with_f) {
-        unsafeAtomicAdd(p, W.amt[1] * seg);
-        p += B.cols;
-        unsafeAtomicAdd(p, W.amt[2] * seg);
-        p += B.cols;
-        unsafeAtomicAdd(p, W.amt[3] * seg);
+    if constexpr (kRows == 1) {
+        // one row, perhaps a range of its columns
+        if (uint32_t(W.idx) < uint32_t(B.cols)) unsafeAtomicAdd(p, W.amt[0] * seg);
+    } else {
+#pragma unroll
+        for (int j = 0; j < kMaxRows; ++j) {
+            if (kRows == kMaxRows || (B.rowmask >> j & 1)) {
+                unsafeAtomicAdd(p, W.amt[j] * seg);
+                p += B.cols;
+            }
+        }
     }
     W.left--;
     W.prev = tm;
@@ -255,11 +260,11 @@ __device__ __forceinline__ void box_walk_next(BoxWalk<F, NA>& W, const BoxCell<F
     }
 }
 
-template <int U, bool kMulti, typename F, int NA>
+template <int U, int kRows, typename F, int NA>
 __device__ __forceinline__ void box_walk_some(BoxWalk<F, NA>& W, const BoxCell<F>& B, double* tally) {
     if (W.left > 0) {
-        box_walk_next<kMulti>(W, B, tally);
-        if constexpr (U > 1) box_walk_some<U - 1, kMulti>(W, B, tally);
+        box_walk_next<kRows>(W, B, tally);
+        if constexpr (U > 1) box_walk_some<U - 1, kRows>(W, B, tally);
     }
 }
 
@@ -284,13 +289,15 @@ __device__ __forceinline__ void add_row(const Span<F>& s, F amt, F ca) {
 
 // The tally of a flight pre -> L.pos of length dmin: added at once along one
 // axis, set up in W for a grid.
-template <typename F, int kAxes, bool kMulti>
+template <typename F, int kAxes, int kRows>
 __device__ __forceinline__ void box_tally(const BoxCell<F>& B, const BoxView<F>& V, const BoxLane<F>& L,
                                           const dev::V3<F>& pre, F dmin, BoxWalk<F, kAxes>& W) {
     F dt;
     if constexpr (sizeof(F) == 4) dt = dmin * L.vel;
     else dt = L.sg * Quotient(L.vel)(dmin);
     const F dx = L.sg * (L.pos.x - pre.x), dy = L.sg * (L.pos.y - pre.y), dz = L.sg * (L.pos.z - pre.z);
+    // the one row's amount
+    const F only = B.rowmask & 1 ? dt : (B.rowmask & 2 ? dx : (B.rowmask & 4 ? dy : dz));
     if constexpr (kAxes == 0) {
         if (B.tally == 0) return;
         const F b = B.div[0] * (B.inv[0] * (pick3(B.comp[0], pre) - B.o[0]));
@@ -310,16 +317,20 @@ __device__ __forceinline__ void box_tally(const BoxCell<F>& B, const BoxView<F>&
         s.end = V.tally + kMaxRows * kBoxCols + hi;
         if constexpr (sizeof(F) == 4) {
             const F rad = __builtin_amdgcn_rcpf(fabsf(e - b));
-            if (kMulti || B.with_t) add_row<0>(s, dt, dt * rad);
-            if (kMulti || B.with_f) {
+            if constexpr (kRows == 1) {
+                add_row<0>(s, only, only * rad);
+            } else {
+                if (kRows == kMaxRows || B.rowmask & 1) add_row<0>(s, dt, dt * rad);
                 add_row<1>(s, dx, dx * rad);
                 add_row<2>(s, dy, dy * rad);
                 add_row<3>(s, dz, dz * rad);
             }
         } else {
             const Quotient q(fabs(e - b));
-            if (kMulti || B.with_t) add_row<0>(s, dt, q(dt));
-            if (kMulti || B.with_f) {
+            if constexpr (kRows == 1) {
+                add_row<0>(s, only, q(only));
+            } else {
+                if (kRows == kMaxRows || B.rowmask & 1) add_row<0>(s, dt, q(dt));
                 add_row<1>(s, dx, q(dx));
                 add_row<2>(s, dy, q(dy));
                 add_row<3>(s, dz, q(dz));
@@ -356,10 +367,10 @@ __device__ __forceinline__ void box_tally(const BoxCell<F>& B, const BoxView<F>&
             left += none ? 0 : n;
             W.dcol[q] = up ? B.stride[q] : -B.stride[q];
         }
-        W.idx = idx;
+        W.idx = kRows == 1 ? idx - B.col0 : idx;
         W.prev = F(0);
         W.left = left;
-        W.amt[0] = double(dt);
+        W.amt[0] = double(kRows == 1 ? only : dt);
         W.amt[1] = double(dx);
         W.amt[2] = double(dy);
         W.amt[3] = double(dz);
@@ -369,7 +380,7 @@ __device__ __forceinline__ void box_tally(const BoxCell<F>& B, const BoxView<F>&
 // One scatter-step: the flight (problem.cpp:401-416) and the event
 // (problem.cpp:418-433), as flight_step and collide_step take them.  Returns
 // the bundle's fate, kAlive while it lives.
-template <typename F, bool kLdsTables, int kAxes, bool kMulti>
+template <typename F, bool kLdsTables, int kAxes, int kRows>
 __device__ __forceinline__ uint32_t box_step(const BoxCell<F>& B, const BoxView<F>& V, BoxLane<F>& L,
                                              BoxWalk<F, kAxes>& W) {
     // ---- flight: the face ahead on each axis, the pore, the free path
@@ -435,7 +446,7 @@ __device__ __forceinline__ uint32_t box_step(const BoxCell<F>& B, const BoxView<
     }
     uint32_t fate = MCG_ESCAPED;
     if (!outside) {
-        box_tally<F, kAxes, kMulti>(B, V, L, pre, dmin, W);
+        box_tally<F, kAxes, kRows>(B, V, L, pre, dmin, W);
 
         // ---- event
         uint32_t kind = (B.kinds >> hit) & 15u;
@@ -590,8 +601,8 @@ __device__ __forceinline__ void box_flush(ParamPtr<F> kp, const BoxCell<F>& B, c
     double* const direct = in_global(kp->direct);
     double* const diff = in_global(kp->diff);
     if (B.tally == 1) {
-        // LDS rows 0..3 are T, qx, qy, qz; the solve's first row is its first kind
-        const int r0 = B.with_t ? 0 : 1;
+        // LDS row j is the quantity j (row 0 the only one of a one-row tally)
+        const int r0 = B.rows == 1 || (B.rowmask & 1) ? 0 : 1;
         for (int i = tid; i < B.rows * kBoxCols; i += nthreads) {
             const int r = i / kBoxCols, c = i % kBoxCols;
             const double a = tally[(r0 + r) * kBoxCols + c], d = tally[(kMaxRows + r0 + r) * kBoxCols + c];
@@ -599,10 +610,11 @@ __device__ __forceinline__ void box_flush(ParamPtr<F> kp, const BoxCell<F>& B, c
             if (d != 0.0 && c <= B.cols) unsafeAtomicAdd(diff + r * (B.cols + 1) + c, d);
         }
     } else if (B.tally == 2) {
-        for (int i = tid; i < B.rows * B.cols; i += nthreads) {
-            const double a = tally[i];
-            if (a != 0.0) unsafeAtomicAdd(direct + i, a);
-        }
+        for (int r = 0; r < B.rows; ++r)
+            for (int c = tid; c < B.cols; c += nthreads) {
+                const double a = tally[r * B.cols + c];
+                if (a != 0.0) unsafeAtomicAdd(direct + size_t(B.row0 + r) * B.gcols + B.col0 + c, a);
+            }
     }
 }
 
@@ -637,7 +649,7 @@ __device__ __forceinline__ void box_emit(ParamPtr<F> kp, const BoxCell<F>& B, co
 // The refill is looked at only when some lane has run out of work since the
 // last look: a wavefront left with a few long-lived bundles goes from step to
 // step without it.
-template <typename F, bool kLdsTables, int kAxes, bool kMulti>
+template <typename F, bool kLdsTables, int kAxes, int kRows>
 __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, const BoxView<F>& V, int lane) {
     const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
     int64_t pool_base = 0, pool_lim = 0, seen = 0;
@@ -652,6 +664,8 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
             const bool walking = W.left > 0;
             const ParamPtr<F> k = params_here<F>(kp);
             const int64_t count = k->count;
+            unsigned long long* const next =
+                B.part == 0 ? in_global(k->next) : in_global(k->part_next) + (B.part - 1);
             if constexpr (sizeof(F) == 4) {
                 if (!active && !walking && full) {
                     L = N;
@@ -663,7 +677,7 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
                 const uint64_t me = __ballot(empty);
                 if (me != 0ull && (popc(me) >= kSlotQuorum || popc(__ballot(empty && !active && !walking)) >= kEmitQuorum ||
                                    __ballot(active || walking) == 0ull)) {
-                    const int64_t mine = claim(empty, lane, lt_mask, pool_base, pool_lim, in_global(k->next), k->chunk, count,
+                    const int64_t mine = claim(empty, lane, lt_mask, pool_base, pool_lim, next, k->chunk, count,
                                                k->tail, &seen);
                     if (empty) {
                         if (mine < count) {
@@ -683,7 +697,7 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
             } else {
                 const bool need = !active && !drained && !walking;
                 if (emit_now<kEmitQuorumFp64>(need, active || walking)) {
-                    const int64_t mine = claim(need, lane, lt_mask, pool_base, pool_lim, in_global(k->next), k->chunk);
+                    const int64_t mine = claim(need, lane, lt_mask, pool_base, pool_lim, next, k->chunk);
                     if (need) {
                         if (mine < count) {
                             box_emit<F, kLdsTables>(k, B, V, k->first + mine, L);
@@ -700,7 +714,7 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
         const bool go = active && !(W.left > 0);
         steps += popc(__ballot(go));
         uint32_t fate = kAlive;
-        if (go) fate = box_step<F, kLdsTables, kAxes, kMulti>(B, V, L, W);
+        if (go) fate = box_step<F, kLdsTables, kAxes, kRows>(B, V, L, W);
         const uint64_t ended = __ballot(fate != kAlive);
         if (ended != 0ull) {
             n_end += popc(ended);
@@ -708,7 +722,7 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
             n_esc += popc(__ballot(fate == MCG_ESCAPED));
             if (fate != kAlive) {
                 active = false;
-                if (B.counts) {
+                if (B.counts && B.part == 0) {
                     const ParamPtr<F> k = params_here<F>(kp);
                     const int64_t i = L.id - k->first;
                     in_global(k->c_nscat)[i] = L.nscat;
@@ -724,12 +738,12 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
             for (;;) {
                 const uint64_t m = __ballot(W.left > 0);
                 if (m == 0ull || (popc(m) < kWalkQuorum && __ballot(active && !(W.left > 0)) != 0ull)) break;
-                box_walk_some<kWalkUnroll, kMulti>(W, B, V.tally);
+                box_walk_some<kWalkUnroll, kRows>(W, B, V.tally);
             }
         }
         busy = __ballot(active || W.left > 0);
     }
-    if (lane == 0 && n_end != 0) {
+    if (lane == 0 && n_end != 0 && B.part == 0) {
         unsigned long long* const c = in_global(params_here<F>(kp)->counters);
         atomicAdd(c + C_STEPS, steps);
         atomicAdd(c + C_ESC, n_esc);
@@ -739,18 +753,52 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
     }
 }
 
+// A map larger than the LDS is tallied in parts (rows of it, or column ranges
+// of a row), each by its own workgroups, which run all of the solve's bundles
+// and add only to their part: workgroup w takes part w % parts.  The bundles'
+// counts and statistics are those of part 0.
+//
+// Why: adding in global memory is bound by the rate of FP64 atomics past the
+// LDS, 1.1e10 a second for the whole GPU, four per cell a flight crosses, so a
+// 128 x 128 map ran at 2e8 scatter-steps a second; running the bundles once per
+// part and adding in LDS costs parts / (parts running at once) more steps.
+// Porous film, 2e5 bundles, 128 x 128 Multi map (4 parts): 153 -> 9.7 ms.
+template <typename F>
+__device__ __forceinline__ void box_part(BoxCell<F>& B) {
+    if (B.parts == 1) return;
+    B.part = int32_t(blockIdx.x % uint32_t(B.parts));
+    const int32_t r = B.part / B.colparts, c = B.part % B.colparts;
+    if (B.colparts > 1) {   // one row, a range of its columns
+        B.row0 = r;
+        B.col0 = c * B.cols;
+        B.cols = min(B.cols, B.gcols - B.col0);
+    } else {
+        B.row0 = r * B.rows;
+    }
+    // the quantities of rows [row0, row0 + rows) among those tallied
+    int32_t mask = 0, row = 0;
+    for (int j = 0; j < kMaxRows; ++j) {
+        if (!(B.rowmask >> j & 1)) continue;
+        if (row >= B.row0 && row < B.row0 + B.rows) mask |= 1 << j;
+        ++row;
+    }
+    B.rows = min(B.rows, row - B.row0);
+    B.rowmask = mask;
+}
+
 // A solve of a one-box scene (the kernel parameters come first: params_here
 // reads them through the kernel-argument segment).
-template <typename F, bool kLdsTables, int kAxes, bool kMulti>
+template <typename F, bool kLdsTables, int kAxes, int kRows>
 __global__ void __launch_bounds__(1024) box_kernel(KParams<F> Karg, BoxCell<F> Barg) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int tid = threadIdx.x;
     const ParamPtr<F> kp = (ParamPtr<F>)__builtin_amdgcn_kernarg_segment_ptr();
     BoxCell<F> B = Barg;
+    if constexpr (kAxes != 0) box_part(B);
     box_pin<F, kAxes>(B);
     const BoxView<F> V = box_stage<F, kLdsTables>(params_here<F>(kp), B, lds, tid, blockDim.x);
     __syncthreads();
-    box_run<F, kLdsTables, kAxes, kMulti>(B, kp, V, tid & (kWave - 1));
+    box_run<F, kLdsTables, kAxes, kRows>(B, kp, V, tid & (kWave - 1));
     __syncthreads();
     box_flush(params_here<F>(kp), B, V.tally, tid, blockDim.x);
 }

@@ -127,6 +127,7 @@ struct KParams {
     double* diff;     // rows x (cols + 1), row-major
     unsigned long long* counters;
     unsigned long long* next;   // bundle claim counter (offset into [first, first + count))
+    unsigned long long* part_next;   // claim counters of a tally's parts after the first (box kernel)
     uint32_t* c_nscat;
     uint32_t* c_nbdry;
     uint32_t* c_nstep;
@@ -2227,8 +2228,9 @@ bool box_cell(const HostScene& h, const HostProblem& p, BoxCell<F>& B) {
     B.nmodes = int32_t(h.mode_cell.size());
     B.rows = int32_t(p.rows);
     B.cols = int32_t(h.cols);
-    B.with_t = p.tally == MCG_TEMP || p.tally == MCG_MULTI;
-    B.with_f = p.tally == MCG_FLUX || p.tally == MCG_MULTI;
+    B.gcols = B.cols;
+    B.rowmask = p.tally == MCG_TEMP ? 1 : (p.tally == MCG_FLUX ? 14 : 15);
+    B.parts = B.colparts = 1;
     // tally axes: coordinate k = div_k inv_k . (p - o); one nonzero entry per
     // row of inv, so the other products are exact zeros
     int axes[3], na = 0;
@@ -2276,27 +2278,54 @@ bool box_cell(const HostScene& h, const HostProblem& p, BoxCell<F>& B) {
     return true;
 }
 
-// The box kernel of a tally (axes of its grid, 0 without one; all four Multi
-// rows or any) and of tables staged in LDS or read from global memory.
+// The box kernel of a tally (axes of its grid, 0 without one; rows: all four
+// Multi rows, one, or any) and of tables staged in LDS or read from global
+// memory.
+template <typename F, int kAxes, int kRows>
+const void* pick_box_kernel(bool tables) {
+    return tables ? reinterpret_cast<const void*>(box_kernel<F, true, kAxes, kRows>)
+                  : reinterpret_cast<const void*>(box_kernel<F, false, kAxes, kRows>);
+}
 template <typename F, int kAxes>
-const void* pick_box_kernel(bool tables, bool multi) {
-    if (multi)
-        return tables ? reinterpret_cast<const void*>(box_kernel<F, true, kAxes, true>)
-                      : reinterpret_cast<const void*>(box_kernel<F, false, kAxes, true>);
-    return tables ? reinterpret_cast<const void*>(box_kernel<F, true, kAxes, false>)
-                  : reinterpret_cast<const void*>(box_kernel<F, false, kAxes, false>);
+const void* pick_box_kernel(bool tables, int rows) {
+    return rows == kMaxRows ? pick_box_kernel<F, kAxes, kMaxRows>(tables)
+                            : (rows == 1 ? pick_box_kernel<F, kAxes, 1>(tables) : pick_box_kernel<F, kAxes, 0>(tables));
 }
 template <typename F>
-const void* pick_box_kernel(bool tables, bool multi, int axes) {
-    return axes == 0 ? pick_box_kernel<F, 0>(tables, multi)
-                     : (axes == 2 ? pick_box_kernel<F, 2>(tables, multi) : pick_box_kernel<F, 3>(tables, multi));
+const void* pick_box_kernel(bool tables, int rows, int axes) {
+    return axes == 0 ? pick_box_kernel<F, 0>(tables, rows)
+                     : (axes == 2 ? pick_box_kernel<F, 2>(tables, rows) : pick_box_kernel<F, 3>(tables, rows));
 }
 
-// LDS of a box launch: the faces and the tally, and the tables when they fit
-// beside them.  False when the tally does not fit.
+// Parts a map may be split into.  Past this the repeated steps cost more than
+// they save: a part costs a full run of the bundles (2e-10 s a scatter-step
+// with a fine map's walk), the global map 1e-10 s per added cell and row, so
+// 64 parts pay from about 130 adds a step, which a map of that size
+// (64 x 160 KiB) takes.
+constexpr int kMaxParts = 64;
+
+// LDS of a box launch: the faces and the tally (in parts, when `split`, if the
+// whole does not fit), and the tables when they fit beside them.  False when
+// the tally does not fit.
 template <typename F>
-bool box_lds_plan(const BoxCell<F>& B, bool tables_allowed, size_t limit, bool& tables, size_t& bytes) {
-    bytes = 6 * sizeof(BoxFace<F>) + size_t(box_tally_doubles(B)) * sizeof(double);
+bool box_lds_plan(BoxCell<F>& B, bool split, bool tables_allowed, size_t limit, bool& tables, size_t& bytes) {
+    const size_t faces = 6 * sizeof(BoxFace<F>);
+    const int64_t room = limit > faces ? int64_t((limit - faces) / sizeof(double)) : 0;
+    if (B.tally == 2 && int64_t(B.rows) * B.cols > room) {
+        if (!split || room == 0) return false;
+        if (B.cols <= room) {
+            const int fit = int(room / B.cols);
+            B.parts = (B.rows + fit - 1) / fit;
+            B.rows = (B.rows + B.parts - 1) / B.parts;
+        } else {
+            B.colparts = int((B.cols + room - 1) / room);
+            B.parts = B.rows * B.colparts;
+            B.rows = 1;
+            B.cols = (B.cols + B.colparts - 1) / B.colparts;
+        }
+        if (B.parts > kMaxParts) return false;
+    }
+    bytes = faces + size_t(box_tally_doubles(B)) * sizeof(double);
     if (bytes > limit) return false;
     const size_t tab = box_lds_tables<F>(B.nmodes);
     tables = tables_allowed && bytes + tab <= limit;
@@ -2339,11 +2368,13 @@ int launch_box(mcg_scene* sc, const HostProblem& p, KParams<F>& K, BoxCell<F>& c
     const int block = sc->tune.block > 0 ? sc->tune.block : (per_cu == 1 ? 1024 : 512);
     per_cu = std::min(per_cu, std::max(1, 2048 / block));
     if (sc->tune.blocks_per_cu > 0) per_cu = std::min(per_cu, int(sc->tune.blocks_per_cu));
+    // each part of the tally takes the same share of the workgroups
     const int64_t needed = (p.count + block - 1) / block;
-    const int grid = int(std::max<int64_t>(1, std::min<int64_t>(int64_t(sc->num_cu) * per_cu, needed)));
+    const int64_t share = std::max<int64_t>(1, int64_t(sc->num_cu) * per_cu / cell.parts);
+    const int grid = int(std::max<int64_t>(1, std::min(share, needed)));
     K.tail = int64_t(MCG_TAIL_LANES) * grid * block;
     void* args[] = {&K, &cell};
-    HIP_TRY(hipLaunchKernel(fn, dim3(grid), dim3(block), args, lds, stream));
+    HIP_TRY(hipLaunchKernel(fn, dim3(grid * cell.parts), dim3(block), args, lds, stream));
     HIP_TRY(hipGetLastError());
     return MCG_OK;
 }
@@ -2359,11 +2390,10 @@ int launch_solve(mcg_scene* sc, const HostProblem& p, KParams<F>& K, hipStream_t
     bool box_tables = false;
     size_t box_lds = 0;
     if (K.trace_id < 0 && !(h.has_grid && sc->tune.defer_walks < 0) && box_cell<F>(h, p, cell) &&
-        box_lds_plan<F>(cell, sc->tune.lds_tables >= 0, sc->lds_limit, box_tables, box_lds)) {
+        box_lds_plan<F>(cell, K.part_next != nullptr, sc->tune.lds_tables >= 0, sc->lds_limit, box_tables, box_lds)) {
         cell.counts = K.c_nscat != nullptr;
         const int axes = cell.tally == 2 ? (h.grid_2d ? 2 : 3) : 0;
-        return launch_box<F>(sc, p, K, cell, pick_box_kernel<F>(box_tables, p.tally == MCG_MULTI && cell.tally != 0, axes),
-                             box_lds, stream);
+        return launch_box<F>(sc, p, K, cell, pick_box_kernel<F>(box_tables, cell.rows, axes), box_lds, stream);
     }
     const size_t geo = lds_bytes<F>(h, rows, false, false);
     const LdsPlan lp = plan_lds(geo, lds_bytes<F>(h, rows, true, false) - geo,
@@ -2430,7 +2460,7 @@ int run_solve(mcg_scene* sc, const HostProblem& p, double* out, mcg_counts* coun
     DevBuf<uint32_t> cnt;
     int rc;
     const size_t nall = nd + nf + C_COUNT;   // counters: C_COUNT 8-byte words after the tallies
-    if ((rc = sc->ws_tally.reserve(nall))) return rc;
+    if ((rc = sc->ws_tally.reserve(nall + kMaxParts))) return rc;   // then the claim counters of a tally's parts
     if (sc->ws_cdf.p == nullptr || sc->ws_cdf.n < p.emit_cdf.size() || sc->ws_cdf_host != p.emit_cdf) {
         if ((rc = sc->ws_cdf.reserve(p.emit_cdf.size()))) return rc;
         HIP_TRY(hipMemcpy(sc->ws_cdf.p, p.emit_cdf.data(), p.emit_cdf.size() * sizeof(int64_t),
@@ -2450,11 +2480,12 @@ int run_solve(mcg_scene* sc, const HostProblem& p, double* out, mcg_counts* coun
     const bool want_counts = counts && counts->nscat && counts->nbdry && counts->nstep && counts->fate;
     if (want_counts && (rc = cnt.alloc(size_t(4) * p.count))) return rc;
     hipLaunchKernelGGL(zero_kernel, dim3(int(std::min<size_t>(1024, (nd + nf + 255) / 256 + 1))), dim3(256), 0, 0,
-                       direct, nd + nf, static_cast<double*>(nullptr), size_t(0), ctr, size_t(C_COUNT));
+                       direct, nd + nf, static_cast<double*>(nullptr), size_t(0), ctr, size_t(C_COUNT + kMaxParts));
     HIP_TRY(hipGetLastError());
 
     KParams<F> K{};
     fill_params<F>(sc, p, K);
+    K.part_next = ctr + C_COUNT;
     K.emit_cdf = sc->ws_cdf.p;
     K.direct = direct;
     K.diff = diff;

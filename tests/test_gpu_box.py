@@ -1,6 +1,7 @@
 """The one-box kernel at the edges of its rule and of its tally layout: 1-D
 tallies up to the fixed LDS row stride and past it (the general kernel), a
-single cell, no tally, 2-D and 3-D maps, each tally kind, every face kind it
+single cell, no tally, 2-D and 3-D maps, maps larger than the LDS (in parts
+of several rows, one row, or a range of columns, and past the most parts), each tally kind, every face kind it
 takes, a box away from the origin, a pore of each kind of wall.
 
 FP64 is compared with the checker: per-bundle counts exactly, tallies to 1e-9
@@ -59,6 +60,11 @@ CASES = {
     "grid_xz_temp": (lambda: box(L, (8, 0, 3), WALLS), abi.TEMP),
     "grid_2x2": (lambda: box(L, (2, 2, 0), WALLS), abi.MULTI),
     "grid_3d": (lambda: box(L, (7, 5, 3), WALLS), abi.MULTI),
+    "parts_rows": (lambda: box(L, (100, 60, 0), WALLS), abi.MULTI),
+    "parts_3d": (lambda: box(L, (40, 16, 16), WALLS), abi.MULTI),
+    "parts_cols_odd": (lambda: box(L, (211, 149, 0), WALLS), abi.TEMP),
+    "parts_cols_flux": (lambda: scenes.porous_film(div=(160, 131, 0)), abi.FLUX),
+    "parts_past_most": (lambda: box(L, (1200, 1201, 0), WALLS), abi.TEMP),
     "film": (lambda: scenes.film((2e-7, 1e-7, 2e-7), (6, 3, 0), 0.2), abi.MULTI),
     "bulk_all_periodic": (lambda: box(L, (9, 0, 0), [scenes.face(abi.PERI)] * 6, grad=(-1e6, 0.0, 0.0), peri=(0, 1, 2)),
                           abi.MULTI),
