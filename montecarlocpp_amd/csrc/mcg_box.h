@@ -73,6 +73,7 @@ struct BoxCell {
     // of gcols columns (the whole map, or the part of it this workgroup tallies)
     int32_t tally, rowmask, rows, cols, row0, col0, gcols;
     int32_t part, parts, colparts;   // see box_part
+    unsigned long long* next;        // claim counter of the part
     uint32_t comp[3][3];                   // per tally axis: mask of each position component
     int32_t last[3], stride[3];            // largest index, column stride
     F o[3], inv[3], div[3];                // cell coordinate = div (inv (p - o))
@@ -233,15 +234,22 @@ __device__ __forceinline__ void box_walk_next(BoxWalk<F, NA>& W, const BoxCell<F
     }
     const double seg = double((W.left == 1 ? F(1) : tm) - W.prev);
     double* p = tally + W.idx;
-    if constexpr (kRows == 1) {
-        // one row, perhaps a range of its columns
-        if (uint32_t(W.idx) < uint32_t(B.cols)) unsafeAtomicAdd(p, W.amt[0] * seg);
-    } else {
+    if constexpr (kRows == kMaxRows) {
 #pragma unroll
         for (int j = 0; j < kMaxRows; ++j) {
-            if (kRows == kMaxRows || (B.rowmask >> j & 1)) {
-                unsafeAtomicAdd(p, W.amt[j] * seg);
-                p += B.cols;
+            unsafeAtomicAdd(p, W.amt[j] * seg);
+            p += B.cols;
+        }
+    } else if (uint32_t(W.idx) < uint32_t(B.cols)) {   // perhaps a range of the columns
+        if constexpr (kRows == 1) {
+            unsafeAtomicAdd(p, W.amt[0] * seg);
+        } else {
+#pragma unroll
+            for (int j = 0; j < kMaxRows; ++j) {
+                if (B.rowmask >> j & 1) {
+                    unsafeAtomicAdd(p, W.amt[j] * seg);
+                    p += B.cols;
+                }
             }
         }
     }
@@ -317,20 +325,16 @@ __device__ __forceinline__ void box_tally(const BoxCell<F>& B, const BoxView<F>&
         s.end = V.tally + kMaxRows * kBoxCols + hi;
         if constexpr (sizeof(F) == 4) {
             const F rad = __builtin_amdgcn_rcpf(fabsf(e - b));
-            if constexpr (kRows == 1) {
-                add_row<0>(s, only, only * rad);
-            } else {
-                if (kRows == kMaxRows || B.rowmask & 1) add_row<0>(s, dt, dt * rad);
+            if (kRows == kMaxRows || B.rowmask & 1) add_row<0>(s, dt, dt * rad);
+            if (kRows == kMaxRows || B.rowmask & 2) {
                 add_row<1>(s, dx, dx * rad);
                 add_row<2>(s, dy, dy * rad);
                 add_row<3>(s, dz, dz * rad);
             }
         } else {
             const Quotient q(fabs(e - b));
-            if constexpr (kRows == 1) {
-                add_row<0>(s, only, q(only));
-            } else {
-                if (kRows == kMaxRows || B.rowmask & 1) add_row<0>(s, dt, q(dt));
+            if (kRows == kMaxRows || B.rowmask & 1) add_row<0>(s, dt, q(dt));
+            if (kRows == kMaxRows || B.rowmask & 2) {
                 add_row<1>(s, dx, q(dx));
                 add_row<2>(s, dy, q(dy));
                 add_row<3>(s, dz, q(dz));
@@ -367,7 +371,7 @@ __device__ __forceinline__ void box_tally(const BoxCell<F>& B, const BoxView<F>&
             left += none ? 0 : n;
             W.dcol[q] = up ? B.stride[q] : -B.stride[q];
         }
-        W.idx = kRows == 1 ? idx - B.col0 : idx;
+        W.idx = kRows == kMaxRows ? idx : idx - B.col0;
         W.prev = F(0);
         W.left = left;
         W.amt[0] = double(kRows == 1 ? only : dt);
@@ -601,8 +605,7 @@ __device__ __forceinline__ void box_flush(ParamPtr<F> kp, const BoxCell<F>& B, c
     double* const direct = in_global(kp->direct);
     double* const diff = in_global(kp->diff);
     if (B.tally == 1) {
-        // LDS row j is the quantity j (row 0 the only one of a one-row tally)
-        const int r0 = B.rows == 1 || (B.rowmask & 1) ? 0 : 1;
+        const int r0 = B.rowmask & 1 ? 0 : 1;   // LDS row j is the quantity j
         for (int i = tid; i < B.rows * kBoxCols; i += nthreads) {
             const int r = i / kBoxCols, c = i % kBoxCols;
             const double a = tally[(r0 + r) * kBoxCols + c], d = tally[(kMaxRows + r0 + r) * kBoxCols + c];
@@ -664,8 +667,7 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
             const bool walking = W.left > 0;
             const ParamPtr<F> k = params_here<F>(kp);
             const int64_t count = k->count;
-            unsigned long long* const next =
-                B.part == 0 ? in_global(k->next) : in_global(k->part_next) + (B.part - 1);
+            unsigned long long* const next = in_global(B.next);
             if constexpr (sizeof(F) == 4) {
                 if (!active && !walking && full) {
                     L = N;
@@ -764,14 +766,14 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
 // part and adding in LDS costs parts / (parts running at once) more steps.
 // Porous film, 2e5 bundles, 128 x 128 Multi map (4 parts): 153 -> 9.7 ms.
 template <typename F>
-__device__ __forceinline__ void box_part(BoxCell<F>& B) {
+__host__ __device__ inline void box_part(BoxCell<F>& B, uint32_t w) {
     if (B.parts == 1) return;
-    B.part = int32_t(blockIdx.x % uint32_t(B.parts));
+    B.part = int32_t(w % uint32_t(B.parts));
     const int32_t r = B.part / B.colparts, c = B.part % B.colparts;
     if (B.colparts > 1) {   // one row, a range of its columns
         B.row0 = r;
         B.col0 = c * B.cols;
-        B.cols = min(B.cols, B.gcols - B.col0);
+        B.cols = B.cols < B.gcols - B.col0 ? B.cols : B.gcols - B.col0;
     } else {
         B.row0 = r * B.rows;
     }
@@ -782,7 +784,7 @@ __device__ __forceinline__ void box_part(BoxCell<F>& B) {
         if (row >= B.row0 && row < B.row0 + B.rows) mask |= 1 << j;
         ++row;
     }
-    B.rows = min(B.rows, row - B.row0);
+    B.rows = B.rows < row - B.row0 ? B.rows : row - B.row0;
     B.rowmask = mask;
 }
 
@@ -794,11 +796,119 @@ __global__ void __launch_bounds__(1024) box_kernel(KParams<F> Karg, BoxCell<F> B
     const int tid = threadIdx.x;
     const ParamPtr<F> kp = (ParamPtr<F>)__builtin_amdgcn_kernarg_segment_ptr();
     BoxCell<F> B = Barg;
-    if constexpr (kAxes != 0) box_part(B);
+    if constexpr (kAxes != 0) box_part(B, blockIdx.x);
+    B.next = B.part == 0 ? kp->next : kp->part_next + (B.part - 1);
+    B.k0 = kp->k0;
+    B.k1 = kp->k1;
     box_pin<F, kAxes>(B);
     const BoxView<F> V = box_stage<F, kLdsTables>(params_here<F>(kp), B, lds, tid, blockDim.x);
     __syncthreads();
     box_run<F, kLdsTables, kAxes, kRows>(B, kp, V, tid & (kWave - 1));
     __syncthreads();
     box_flush(params_here<F>(kp), B, V.tally, tid, blockDim.x);
+}
+
+// ------------------------------------------------------------------ batches
+// Many one-box solves in one persistent launch.  A workgroup stages a solve,
+// runs the bundles it claims until none are left, adds its LDS tally to the
+// solve's and takes the next solve.  Each visit costs the staging and a drain
+// (the last bundles' remaining steps, during which lanes idle), so a workgroup
+// should make few visits and those where most work is left:
+//  - it starts at the solve its share of the estimated work lies in
+//    (BoxSolve::work_before), so solves begin with workgroups in proportion;
+//  - then it takes the solve with the most estimated work left per workgroup
+//    already on it, and leaves a solve to the workgroups on it when what is
+//    left is no more than one bundle per lane of theirs.
+// Every solve is finished: one with unclaimed bundles and no visitor is always
+// taken, and a visitor leaves only when nothing is unclaimed (a stale read of
+// a counter can only add a visit that finds nothing).
+// Every solve visited in turn by the general step, before, and this: 256 slabs
+// 17.3 -> 13.5 ms a call, 24 mixed solves replayed 19.7 -> 11.7 ms, same box.
+template <typename F>
+struct BoxSolve {
+    KParams<F> K;                  // first: box_run reads it through ParamPtr
+    BoxCell<F> B;
+    uint32_t* visitors;            // workgroups on the solve
+    double work_before, work;      // estimated work of the solves before this one, and of one bundle
+    int32_t tables, pad;           // sampling tables staged in LDS
+};
+
+template <typename F, bool kLdsTables, int kAxes, int kRows>
+__device__ __forceinline__ void box_visit(const BoxCell<F>& cell, ParamPtr<F> kp, unsigned char* lds, int tid,
+                                          int nthreads) {
+    BoxCell<F> B = cell;
+    box_pin<F, kAxes>(B);
+    const BoxView<F> V = box_stage<F, kLdsTables>(params_here<F>(kp), B, lds, tid, nthreads);
+    __syncthreads();
+    box_run<F, kLdsTables, kAxes, kRows>(B, kp, V, tid & (kWave - 1));
+    __syncthreads();
+    box_flush(params_here<F>(kp), B, V.tally, tid, nthreads);
+    __syncthreads();
+}
+
+// The solve with the most estimated work left per workgroup on it, -1 when no
+// solve needs another workgroup (uniform over the workgroup; LDS is free).
+template <typename F>
+__device__ int box_pick(const BoxSolve<F>* solves, int n, unsigned char* lds, int tid, int nthreads) {
+    unsigned long long* const key = reinterpret_cast<unsigned long long*>(lds);
+    if (tid == 0) *key = 0ull;
+    __syncthreads();
+    unsigned long long best = 0ull;
+    for (int i = tid; i < n; i += nthreads) {
+        const BoxSolve<F>& s = solves[i];
+        const int64_t left =
+            s.K.count - int64_t(__hip_atomic_load(s.B.next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        if (left <= 0) continue;
+        const uint32_t v = __hip_atomic_load(s.visitors, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (v != 0 && left <= int64_t(v) * nthreads) continue;
+        // spread workgroups that look at the same moment
+        const uint32_t mix = (blockIdx.x * 2654435761u + uint32_t(i) * 40503u) >> 24;
+        const float score = float(double(left) * s.work) / float(v + 1) * (1.0f + float(mix) * (1.0f / 512.0f));
+        const unsigned long long k = (uint64_t(__float_as_uint(fmaxf(score, FLT_MIN))) << 32) | uint32_t(i);
+        best = k > best ? k : best;
+    }
+    if (best != 0ull) atomicMax(key, best);
+    __syncthreads();
+    best = *key;
+    __syncthreads();
+    return best == 0ull ? -1 : int(uint32_t(best));
+}
+
+// kAxes: axes of the grids among the solves (0 when all tallies are 1-D).
+template <typename F, int kAxes>
+__global__ void __launch_bounds__(1024) box_batch_kernel(const BoxSolve<F>* solves, int n) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int tid = threadIdx.x, nthreads = blockDim.x;
+    // the solve this workgroup's share of the work starts in: the last one
+    // whose work begins at or before it
+    const double total = solves[n - 1].work_before + solves[n - 1].work * double(solves[n - 1].K.count);
+    const double at = total * ((double(blockIdx.x) + 0.5) / double(gridDim.x));
+    int lo = 0, hi = n - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (solves[mid].work_before <= at) lo = mid;
+        else hi = mid - 1;
+    }
+    for (int si = lo; si >= 0; si = box_pick(solves, n, lds, tid, nthreads)) {
+        const auto* sv = (const __attribute__((address_space(4))) BoxSolve<F>*)(solves + __builtin_amdgcn_readfirstlane(si));
+        const ParamPtr<F> kp = (ParamPtr<F>)sv;
+        BoxCell<F> B = *(const BoxCell<F>*)&sv->B;
+        B.k0 = kp->k0;
+        B.k1 = kp->k1;
+        uint32_t* const visitors = in_global(sv->visitors);
+        if (tid == 0) atomicAdd(visitors, 1u);
+        if (kAxes == 0 || B.tally != 2) {
+            if (B.rowmask == 15) box_visit<F, true, 0, kMaxRows>(B, kp, lds, tid, nthreads);
+            else box_visit<F, true, 0, 0>(B, kp, lds, tid, nthreads);
+        } else if constexpr (kAxes != 0) {
+            if (sv->tables) {
+                if (B.rowmask == 15) box_visit<F, true, kAxes, kMaxRows>(B, kp, lds, tid, nthreads);
+                else box_visit<F, true, kAxes, 0>(B, kp, lds, tid, nthreads);
+            } else {
+                if (B.rowmask == 15) box_visit<F, false, kAxes, kMaxRows>(B, kp, lds, tid, nthreads);
+                else box_visit<F, false, kAxes, 0>(B, kp, lds, tid, nthreads);
+            }
+        }
+        if (tid == 0) atomicSub(visitors, 1u);
+    }
 }

@@ -2223,8 +2223,6 @@ bool box_cell(const HostScene& h, const HostProblem& p, BoxCell<F>& B) {
     B.eps = S.eps;
     B.maxscat = uint32_t(p.maxscat);
     B.maxloop = uint32_t(std::min<int64_t>(p.maxloop, 0xFFFFFFFEll));
-    B.k0 = uint32_t(p.seed);
-    B.k1 = uint32_t(p.seed >> 32);
     B.nmodes = int32_t(h.mode_cell.size());
     B.rows = int32_t(p.rows);
     B.cols = int32_t(h.cols);
@@ -2288,12 +2286,14 @@ const void* pick_box_kernel(bool tables) {
 }
 template <typename F, int kAxes>
 const void* pick_box_kernel(bool tables, int rows) {
-    return rows == kMaxRows ? pick_box_kernel<F, kAxes, kMaxRows>(tables)
-                            : (rows == 1 ? pick_box_kernel<F, kAxes, 1>(tables) : pick_box_kernel<F, kAxes, 0>(tables));
+    if (rows == kMaxRows) return pick_box_kernel<F, kAxes, kMaxRows>(tables);
+    if constexpr (kAxes != 0)
+        if (rows == 1) return pick_box_kernel<F, kAxes, 1>(tables);
+    return pick_box_kernel<F, kAxes, 0>(tables);
 }
 template <typename F>
 const void* pick_box_kernel(bool tables, int rows, int axes) {
-    return axes == 0 ? pick_box_kernel<F, 0>(tables, rows)
+    return axes == 0 ? pick_box_kernel<F, 0>(tables, rows == 1 ? 0 : rows)
                      : (axes == 2 ? pick_box_kernel<F, 2>(tables, rows) : pick_box_kernel<F, 3>(tables, rows));
 }
 
@@ -2303,6 +2303,13 @@ const void* pick_box_kernel(bool tables, int rows, int axes) {
 // 64 parts pay from about 130 adds a step, which a map of that size
 // (64 x 160 KiB) takes.
 constexpr int kMaxParts = 64;
+
+// LDS of a box solve's faces and tally, with its tables or without.
+template <typename F>
+size_t box_lds_bytes(const BoxCell<F>& B, bool tables) {
+    return 6 * sizeof(BoxFace<F>) + size_t(box_tally_doubles(B)) * sizeof(double) +
+           (tables ? box_lds_tables<F>(B.nmodes) : 0);
+}
 
 // LDS of a box launch: the faces and the tally (in parts, when `split`, if the
 // whole does not fit), and the tables when they fit beside them.  False when
@@ -2325,11 +2332,10 @@ bool box_lds_plan(BoxCell<F>& B, bool split, bool tables_allowed, size_t limit, 
         }
         if (B.parts > kMaxParts) return false;
     }
-    bytes = faces + size_t(box_tally_doubles(B)) * sizeof(double);
+    bytes = box_lds_bytes(B, false);
     if (bytes > limit) return false;
-    const size_t tab = box_lds_tables<F>(B.nmodes);
-    tables = tables_allowed && bytes + tab <= limit;
-    if (tables) bytes += tab;
+    tables = tables_allowed && box_lds_bytes(B, true) <= limit;
+    if (tables) bytes = box_lds_bytes(B, true);
     return true;
 }
 
@@ -2929,8 +2935,6 @@ int run_trace_from(mcg_scene* sc, const HostProblem& p, const TraceStart<F>& sta
 
 // Launch plan of a batch: per-solve tally offsets, LDS layout, launch shape.
 struct BatchPlan {
-    std::vector<size_t> off_direct, off_diff;
-    size_t n_direct = 0, n_diff = 0;
     size_t lds = 0;
     bool tables = true, tally = true;
     int walk = 0;              // axes of deferred tally walks (walk_axes)
@@ -2977,27 +2981,23 @@ int plan_shape(int n, mcg_scene* const* scenes, const HostProblem* P, const mcg_
     return MCG_OK;
 }
 
-template <typename F>
-int plan_batch(int n, mcg_scene* const* scenes, const HostProblem* P, const mcg_tune* tune,
-               BatchPlan& B) {
-    int rc = plan_shape<F>(n, scenes, P, tune, B);
-    if (rc) return rc;
-    B.off_direct.resize(n);
-    B.off_diff.resize(n);
-    B.n_direct = B.n_diff = 0;
-    int64_t total = 0;
-    for (int i = 0; i < n; ++i) {
-        const HostScene& h = scenes[i]->host;
-        B.off_direct[i] = B.n_direct;
-        B.off_diff[i] = B.n_diff;
-        B.n_direct += size_t(P[i].rows) * h.cols;
-        B.n_diff += size_t(P[i].rows) * (h.cols + 1);
-        total += P[i].count;
+// Offsets of each solve's tallies in a batch's buffers.
+struct BatchOffsets {
+    std::vector<size_t> direct, diff;
+    size_t n_direct = 0, n_diff = 0;
+    void make(int n, mcg_scene* const* scenes, const HostProblem* P) {
+        direct.resize(n);
+        diff.resize(n);
+        n_direct = n_diff = 0;
+        for (int i = 0; i < n; ++i) {
+            const HostScene& h = scenes[i]->host;
+            direct[i] = n_direct;
+            diff[i] = n_diff;
+            n_direct += size_t(P[i].rows) * h.cols;
+            n_diff += size_t(P[i].rows) * (h.cols + 1);
+        }
     }
-    // no more workgroups than there are bundles to give each lane one
-    B.grid = int(std::max<int64_t>(1, std::min<int64_t>(B.grid, (total + B.block - 1) / B.block)));
-    return MCG_OK;
-}
+};
 
 // Enqueue one batch launch on `stream`.
 template <typename F>
@@ -3010,41 +3010,206 @@ int launch_batch(const BatchPlan& B, const KParams<F>* kp, int nsolves, hipStrea
     return MCG_OK;
 }
 
+// A batch's launches: its one-box solves in one box_batch_kernel launch, the
+// others in one batch_kernel launch.
+template <typename F>
+struct BatchWork {
+    std::vector<int> general;            // solves of the general kernel
+    BatchPlan plan;                      // their launch
+    std::vector<KParams<F>> kparams;
+    std::vector<BoxSolve<F>> box;        // one entry per one-box solve and part of its map
+    std::vector<int> box_of;             // the entry's solve
+    size_t box_lds = 0;
+    int box_block = 0, box_grid = 0, box_axes = 0, box_chunk = kChunk;
+    size_t words = 0;                    // claim counters of parts and visitor counts (8-byte words, cleared per launch)
+
+    // Splits the solves and plans both launches.
+    int make(int n, mcg_scene* const* sc, const HostProblem* P, const mcg_tune* tune) {
+        general.clear();
+        box.clear();
+        box_of.clear();
+        words = 0;
+        if (tune && (tune->defer_walks < -1 || tune->defer_walks > 1))
+            return set_error(MCG_EINVAL, "defer_walks must be -1, 0 or 1");
+        const size_t limit = sc[0]->lds_limit;
+        const bool tables = !(tune && tune->lds_tables < 0);
+        size_t with = 0;                 // LDS with every solve's tables staged
+        std::vector<BoxCell<F>> cells;
+        std::vector<int> cell_of;
+        for (int i = 0; i < n; ++i) {
+            if (sc[i]->device != sc[0]->device) return set_error(MCG_EINVAL, "batch scenes on different devices");
+            const HostScene& h = sc[i]->host;
+            BoxCell<F> c;
+            bool tab = false;
+            size_t bytes = 0;
+            const bool ok = !(h.has_grid && tune && tune->defer_walks < 0) && box_cell<F>(h, P[i], c) &&
+                            box_lds_plan<F>(c, true, tables, limit, tab, bytes) && (c.tally == 2 || tab);
+            if (!ok) {
+                general.push_back(i);
+                continue;
+            }
+            const size_t full = box_lds_bytes(c, true);
+            with = std::max(with, full);
+            if (c.tally == 2) box_axes = std::max(box_axes, h.grid_2d ? 2 : 3);
+            cells.push_back(c);
+            cell_of.push_back(i);
+        }
+        // 2-D and 3-D grids in one launch walk three axes: a 2-D grid's third
+        // axis has one cell
+        box_lds = std::min(with, limit);
+        double before = 0.0;
+        for (size_t j = 0; j < cells.size(); ++j) {
+            BoxCell<F>& c = cells[j];
+            const HostProblem& p = P[cell_of[j]];
+            const HostScene& h = sc[cell_of[j]]->host;
+            if (c.tally == 2 && box_axes == 3 && h.grid_2d) {
+                c.o[2] = c.inv[2] = c.div[2] = F(0);
+                c.last[2] = c.stride[2] = 0;
+            }
+            // rough cost of a bundle: its steps (an absorber ends it after
+            // some; otherwise the scatter cap does) and the cells they cross
+            bool absorbs = false;
+            for (const auto& pl : h.planes) absorbs = absorbs || pl.kind == MCG_ISOT;
+            double cost = absorbs ? 8.0 : 1.5 * double(std::min<int64_t>(p.maxscat, 1000));
+            if (c.tally == 2) cost *= 1.0 + double(c.last[0] + c.last[1] + c.last[2]) / 64.0;
+            for (int q = 0; q < c.parts; ++q) {
+                BoxSolve<F> e{};
+                e.B = c;
+                box_part(e.B, uint32_t(q));
+                e.work = cost;
+                e.work_before = before;
+                e.tables = tables && box_lds_bytes(e.B, true) <= box_lds ? 1 : 0;
+                before += cost * double(p.count);
+                box.push_back(e);
+                box_of.push_back(cell_of[j]);
+                words += c.parts > 1 && q > 0 ? 2 : 1;
+            }
+        }
+        if (!box.empty()) {
+            int per_cu = std::max<int>(1, int(limit / box_lds));
+            box_block = tune && tune->block ? tune->block : (per_cu == 1 ? 1024 : 512);
+            if (box_block < 64 || box_block > 1024 || box_block % 64 != 0)
+                return set_error(MCG_EINVAL, "block must be a multiple of 64 from 64 to 1024");
+            per_cu = std::min(per_cu, std::max(1, 2048 / box_block));
+            if (tune && tune->blocks_per_cu > 0) per_cu = std::min(per_cu, int(tune->blocks_per_cu));
+            box_grid = sc[0]->num_cu * per_cu;
+            box_chunk = tune && tune->chunk > 0 ? tune->chunk : kChunk;
+        }
+        if (!general.empty()) {
+            std::vector<mcg_scene*> gs;
+            std::vector<HostProblem> gp;
+            for (int i : general) {
+                gs.push_back(sc[i]);
+                gp.push_back(P[i]);
+            }
+            int rc = plan_shape<F>(int(gs.size()), gs.data(), gp.data(), tune, plan);
+            if (rc) return rc;
+        }
+        return MCG_OK;
+    }
+
+    // The launches' parameters from the solves' (K[i], with its buffers,
+    // bundle range and seed); `ctl` points to `words` cleared words.
+    void fill(const KParams<F>* K, unsigned long long* ctl) {
+        int64_t total = 0;
+        kparams.clear();
+        for (int i : general) {
+            kparams.push_back(K[i]);
+            kparams.back().chunk = plan.chunk;
+            kparams.back().lds_tally = plan.tally ? 1 : 0;
+            total += K[i].count;
+        }
+        if (!general.empty())
+            plan.grid = int(std::max<int64_t>(1, std::min<int64_t>(plan.grid, (total + plan.block - 1) / plan.block)));
+        total = 0;
+        double work = 0.0;
+        for (size_t j = 0; j < box.size(); ++j) {
+            box[j].work_before = work;
+            work += box[j].work * double(K[box_of[j]].count);
+            total += K[box_of[j]].count;
+        }
+        if (box.empty()) return;
+        box_grid = int(std::max<int64_t>(1, std::min<int64_t>(box_grid, (total + box_block - 1) / box_block)));
+        for (size_t j = 0; j < box.size(); ++j) {
+            BoxSolve<F>& e = box[j];
+            e.K = K[box_of[j]];
+            e.K.chunk = box_chunk;
+            // claims shrink within kTailLanes bundles per lane of the
+            // workgroups its share of the work brings
+            const double wgs = work > 0.0 ? double(box_grid) * e.work * double(e.K.count) / work : 1.0;
+            e.K.tail = int64_t(MCG_TAIL_LANES) * box_block * std::max<int64_t>(1, int64_t(wgs + 0.5));
+            e.B.next = e.B.part == 0 ? e.K.next : ctl++;
+            e.visitors = reinterpret_cast<uint32_t*>(ctl++);
+        }
+    }
+
+    // Enqueues both launches (box_dev, k_dev: device copies of box, kparams).
+    int launch(const BoxSolve<F>* box_dev, const KParams<F>* k_dev, hipStream_t stream) const {
+        if (!box.empty()) {
+            const void* fn = box_kernel_fn();
+            int nbox = int(box.size());
+            HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(box_lds)));
+            void* args[] = {&box_dev, &nbox};
+            HIP_TRY(hipLaunchKernel(fn, dim3(box_grid), dim3(box_block), args, box_lds, stream));
+            HIP_TRY(hipGetLastError());
+        }
+        if (!general.empty()) return launch_batch<F>(plan, k_dev, int(general.size()), stream);
+        return MCG_OK;
+    }
+    // Sets the kernels' LDS attributes (before a capture).
+    int prepare() const {
+        if (!box.empty())
+            HIP_TRY(hipFuncSetAttribute(box_kernel_fn(), hipFuncAttributeMaxDynamicSharedMemorySize, int(box_lds)));
+        if (!general.empty())
+            HIP_TRY(hipFuncSetAttribute(pick_kernel<F>(KernelKind::Batch, plan.tables, plan.tally, plan.walk),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(plan.lds)));
+        return MCG_OK;
+    }
+    const void* box_kernel_fn() const {
+        return box_axes == 0 ? reinterpret_cast<const void*>(box_batch_kernel<F, 0>)
+                             : (box_axes == 2 ? reinterpret_cast<const void*>(box_batch_kernel<F, 2>)
+                                              : reinterpret_cast<const void*>(box_batch_kernel<F, 3>));
+    }
+};
+
 template <typename F>
 int run_batch(int n, mcg_scene* const* scenes, const HostProblem* P, double* const* outs,
               mcg_stats* stats, const mcg_tune* tune) {
     auto t0 = std::chrono::steady_clock::now();
     HIP_TRY(hipSetDevice(scenes[0]->device));
-    BatchPlan B;
-    int rc = plan_batch<F>(n, scenes, P, tune, B);
+    BatchWork<F> B;
+    int rc = B.make(n, scenes, P, tune);
     if (rc) return rc;
+    BatchOffsets off;
+    off.make(n, scenes, P);
     DevBuf<double> direct, diff;
     DevBuf<unsigned long long> ctr;
     DevBuf<int64_t> cdf;
     DevBuf<KParams<F>> kp;
+    DevBuf<BoxSolve<F>> bp;
     std::vector<int64_t> cdf_all;
     std::vector<size_t> cdf_off(n);
     for (int i = 0; i < n; ++i) {
         cdf_off[i] = cdf_all.size();
         cdf_all.insert(cdf_all.end(), P[i].emit_cdf.begin(), P[i].emit_cdf.end());
     }
-    if ((rc = direct.alloc(B.n_direct))) return rc;
-    if ((rc = diff.alloc(B.n_diff))) return rc;
-    if ((rc = ctr.alloc(size_t(C_COUNT) * n))) return rc;
+    if ((rc = direct.alloc(off.n_direct))) return rc;
+    if ((rc = diff.alloc(off.n_diff))) return rc;
+    if ((rc = ctr.alloc(size_t(C_COUNT) * n + B.words))) return rc;
     if ((rc = cdf.upload(cdf_all.data(), cdf_all.size()))) return rc;
     std::vector<KParams<F>> K(n);
     for (int i = 0; i < n; ++i) {
         K[i] = KParams<F>{};
         fill_params<F>(scenes[i], P[i], K[i]);
         K[i].emit_cdf = cdf.p + cdf_off[i];
-        K[i].direct = direct.p + B.off_direct[i];
-        K[i].diff = diff.p + B.off_diff[i];
+        K[i].direct = direct.p + off.direct[i];
+        K[i].diff = diff.p + off.diff[i];
         K[i].counters = ctr.p + size_t(C_COUNT) * i;
         K[i].next = K[i].counters + C_NEXT;
-        K[i].chunk = B.chunk;
-        K[i].lds_tally = B.tally ? 1 : 0;
     }
-    if ((rc = kp.upload(K.data(), K.size()))) return rc;
+    B.fill(K.data(), ctr.p + size_t(C_COUNT) * n);
+    if ((rc = kp.upload(B.kparams.data(), B.kparams.size()))) return rc;
+    if ((rc = bp.upload(B.box.data(), B.box.size()))) return rc;
     HIP_TRY(hipMemset(direct.p, 0, direct.n * sizeof(double)));
     HIP_TRY(hipMemset(diff.p, 0, diff.n * sizeof(double)));
     HIP_TRY(hipMemset(ctr.p, 0, ctr.n * sizeof(unsigned long long)));
@@ -3052,7 +3217,7 @@ int run_batch(int n, mcg_scene* const* scenes, const HostProblem* P, double* con
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
     HIP_TRY(hipEventRecord(e0, 0));
-    if ((rc = launch_batch<F>(B, kp.p, n, 0))) return rc;
+    if ((rc = B.launch(bp.p, kp.p, 0))) return rc;
     HIP_TRY(hipEventRecord(e1, 0));
     HIP_TRY(hipEventSynchronize(e1));
     float ms = 0.f;
@@ -3066,7 +3231,7 @@ int run_batch(int n, mcg_scene* const* scenes, const HostProblem* P, double* con
     HIP_TRY(hipMemcpy(hc.data(), ctr.p, hc.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost));
     const double wall = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     for (int i = 0; i < n; ++i) {
-        finalise_field(scenes[i]->host, P[i], hd.data() + B.off_direct[i], hf.data() + B.off_diff[i], outs[i]);
+        finalise_field(scenes[i]->host, P[i], hd.data() + off.direct[i], hf.data() + off.diff[i], outs[i]);
         const unsigned long long* c = hc.data() + size_t(C_COUNT) * i;
         if (stats) {
             stats[i].bundles = int64_t(c[C_BUNDLES]);
@@ -3239,11 +3404,13 @@ template <typename F>
 struct GraphBatch : GraphBatchBase {
     std::vector<mcg_scene*> sc;
     std::vector<HostProblem> P;
-    BatchPlan B;
+    BatchWork<F> B;
+    BatchOffsets off;
     DevBuf<double> direct, diff;
     DevBuf<unsigned long long> ctr;
     DevBuf<int64_t> cdf;
     DevBuf<KParams<F>> kp;
+    DevBuf<BoxSolve<F>> bp;
     std::vector<KParams<F>> K;
     hipStream_t stream = nullptr;
     hipGraph_t graph = nullptr;
@@ -3261,43 +3428,43 @@ struct GraphBatch : GraphBatchBase {
 
     int create(const mcg_tune* tune) {
         HIP_TRY(hipSetDevice(sc[0]->device));
-        int rc = plan_batch<F>(n, sc.data(), P.data(), tune, B);
+        int rc = B.make(n, sc.data(), P.data(), tune);
         if (rc) return rc;
+        off.make(n, sc.data(), P.data());
         std::vector<int64_t> cdf_all;
         std::vector<size_t> cdf_off(n);
         for (int i = 0; i < n; ++i) {
             cdf_off[i] = cdf_all.size();
             cdf_all.insert(cdf_all.end(), P[i].emit_cdf.begin(), P[i].emit_cdf.end());
         }
-        if ((rc = direct.alloc(B.n_direct))) return rc;
-        if ((rc = diff.alloc(B.n_diff))) return rc;
-        if ((rc = ctr.alloc(size_t(C_COUNT) * n))) return rc;
+        if ((rc = direct.alloc(off.n_direct))) return rc;
+        if ((rc = diff.alloc(off.n_diff))) return rc;
+        if ((rc = ctr.alloc(size_t(C_COUNT) * n + B.words))) return rc;
         if ((rc = cdf.upload(cdf_all.data(), cdf_all.size()))) return rc;
         K.resize(n);
         for (int i = 0; i < n; ++i) {
             K[i] = KParams<F>{};
             fill_params<F>(sc[i], P[i], K[i]);
             K[i].emit_cdf = cdf.p + cdf_off[i];
-            K[i].direct = direct.p + B.off_direct[i];
-            K[i].diff = diff.p + B.off_diff[i];
+            K[i].direct = direct.p + off.direct[i];
+            K[i].diff = diff.p + off.diff[i];
             K[i].counters = ctr.p + size_t(C_COUNT) * i;
             K[i].next = K[i].counters + C_NEXT;
-            K[i].chunk = B.chunk;
-            K[i].lds_tally = B.tally ? 1 : 0;
         }
-        if ((rc = kp.upload(K.data(), K.size()))) return rc;
+        B.fill(K.data(), ctr.p + size_t(C_COUNT) * n);
+        if ((rc = kp.upload(B.kparams.data(), B.kparams.size()))) return rc;
+        if ((rc = bp.upload(B.box.data(), B.box.size()))) return rc;
         HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
         HIP_TRY(hipEventCreate(&e0));
         HIP_TRY(hipEventCreate(&e1));
         // the kernel's LDS limit is an attribute of the function, set before capture
-        HIP_TRY(hipFuncSetAttribute(pick_kernel<F>(KernelKind::Batch, B.tables, B.tally, B.walk),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(B.lds)));
+        if ((rc = B.prepare())) return rc;
         HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
         const size_t total = direct.n + diff.n + ctr.n;
         const int zblocks = int(std::min<size_t>(1024, (total + 255) / 256));
         hipLaunchKernelGGL(zero_kernel, dim3(std::max(1, zblocks)), dim3(256), 0, stream, direct.p, direct.n,
                            diff.p, diff.n, ctr.p, ctr.n);
-        rc = launch_batch<F>(B, kp.p, n, stream);
+        rc = B.launch(bp.p, kp.p, stream);
         hipGraph_t g = nullptr;
         const hipError_t ec = hipStreamEndCapture(stream, &g);
         if (rc) {
@@ -3318,7 +3485,11 @@ struct GraphBatch : GraphBatchBase {
                 K[i].k0 = uint32_t(seeds[i]);
                 K[i].k1 = uint32_t(seeds[i] >> 32);
             }
-            HIP_TRY(hipMemcpy(kp.p, K.data(), K.size() * sizeof(KParams<F>), hipMemcpyHostToDevice));
+            B.fill(K.data(), ctr.p + size_t(C_COUNT) * n);
+            if (!B.kparams.empty())
+                HIP_TRY(hipMemcpy(kp.p, B.kparams.data(), B.kparams.size() * sizeof(KParams<F>), hipMemcpyHostToDevice));
+            if (!B.box.empty())
+                HIP_TRY(hipMemcpy(bp.p, B.box.data(), B.box.size() * sizeof(BoxSolve<F>), hipMemcpyHostToDevice));
         }
         HIP_TRY(hipEventRecord(e0, stream));
         HIP_TRY(hipGraphLaunch(exec, stream));
@@ -3333,7 +3504,7 @@ struct GraphBatch : GraphBatchBase {
         HIP_TRY(hipMemcpy(hc.data(), ctr.p, hc.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost));
         const double wall = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
         for (int i = 0; i < n; ++i) {
-            finalise_field(sc[i]->host, P[i], hd.data() + B.off_direct[i], hf.data() + B.off_diff[i], outs[i]);
+            finalise_field(sc[i]->host, P[i], hd.data() + off.direct[i], hf.data() + off.diff[i], outs[i]);
             const unsigned long long* c = hc.data() + size_t(C_COUNT) * i;
             if (stats) {
                 stats[i].bundles = int64_t(c[C_BUNDLES]);
@@ -3404,6 +3575,8 @@ struct Request {
 struct StepSlot {
     DevBuf<KParams<float>> kp32;
     DevBuf<KParams<double>> kp64;
+    DevBuf<BoxSolve<float>> bp32;
+    DevBuf<BoxSolve<double>> bp64;
     DevBuf<unsigned long long> nx32, nx64;   // per-request bundle claim counters of the step
     hipStream_t stream = nullptr;            // this slot's stream (default priority)
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -3582,7 +3755,7 @@ int retire(mcg_server* sv, Request* r) {
 // Enqueue one precision group of a step on the server's stream.
 template <typename F>
 int enqueue_group(mcg_server* sv, StepSlot& slot, const std::vector<Request*>& reqs,
-                  const std::vector<int64_t>& take, DevBuf<KParams<F>>& kpbuf,
+                  const std::vector<int64_t>& take, DevBuf<KParams<F>>& kpbuf, DevBuf<BoxSolve<F>>& bpbuf,
                   DevBuf<unsigned long long>& nxbuf) {
     const int n = int(reqs.size());
     std::vector<mcg_scene*> sc(n);
@@ -3591,13 +3764,11 @@ int enqueue_group(mcg_server* sv, StepSlot& slot, const std::vector<Request*>& r
         sc[i] = reqs[i]->scene.get();
         P[i] = reqs[i]->P;
     }
-    BatchPlan B;
-    int rc = plan_shape<F>(n, sc.data(), P.data(), &sv->tune, B);
+    BatchWork<F> B;
+    int rc = B.make(n, sc.data(), P.data(), &sv->tune);
     if (rc) return rc;
-    int64_t handed = 0;
-    for (int64_t t : take) handed += t;
-    B.grid = int(std::max<int64_t>(1, std::min<int64_t>(B.grid, (handed + B.block - 1) / B.block)));
-    if (nxbuf.n < size_t(n) && (rc = nxbuf.alloc(size_t(n) * 2))) return rc;
+    const size_t words = size_t(n) + B.words;
+    if (nxbuf.n < words && (rc = nxbuf.alloc(words * 2))) return rc;
     std::vector<KParams<F>> K(n);
     for (int i = 0; i < n; ++i) {
         Request* r = reqs[i];
@@ -3608,18 +3779,21 @@ int enqueue_group(mcg_server* sv, StepSlot& slot, const std::vector<Request*>& r
         K[i].diff = r->diff.p;
         K[i].counters = r->ctr.p;
         K[i].next = nxbuf.p + i;
-        K[i].chunk = B.chunk;
         K[i].first = r->P.first + r->cursor;   // this step's share of the request's bundles
         K[i].count = take[i];
-        K[i].lds_tally = B.tally ? 1 : 0;
         r->cursor += take[i];
         slot.handed.push_back({r, take[i]});
     }
-    if (kpbuf.n < size_t(n) && (rc = kpbuf.alloc(size_t(n) * 2))) return rc;
-    // synchronous copy: kpbuf of this slot is not in use on the device
-    HIP_TRY(hipMemcpy(kpbuf.p, K.data(), K.size() * sizeof(KParams<F>), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemsetAsync(nxbuf.p, 0, size_t(n) * sizeof(unsigned long long), slot.stream));
-    return launch_batch<F>(B, kpbuf.p, n, slot.stream);
+    B.fill(K.data(), nxbuf.p + n);
+    if (kpbuf.n < B.kparams.size() && (rc = kpbuf.alloc(B.kparams.size() * 2))) return rc;
+    if (bpbuf.n < B.box.size() && (rc = bpbuf.alloc(B.box.size() * 2))) return rc;
+    // synchronous copies: this slot's buffers are not in use on the device
+    if (!B.kparams.empty())
+        HIP_TRY(hipMemcpy(kpbuf.p, B.kparams.data(), B.kparams.size() * sizeof(KParams<F>), hipMemcpyHostToDevice));
+    if (!B.box.empty())
+        HIP_TRY(hipMemcpy(bpbuf.p, B.box.data(), B.box.size() * sizeof(BoxSolve<F>), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemsetAsync(nxbuf.p, 0, words * sizeof(unsigned long long), slot.stream));
+    return B.launch(bpbuf.p, kpbuf.p, slot.stream);
 }
 
 // Hand out fair shares of the step budget and enqueue the step in `slot`;
@@ -3661,8 +3835,8 @@ int enqueue_step(mcg_server* sv, StepSlot& slot, StepSlot& other) {
     }
     sv->fresh.clear();
     if (slot.ez_set) HIP_TRY(hipEventRecord(slot.ez, slot.stream));
-    if (!g32.empty() && (rc = enqueue_group<float>(sv, slot, g32, t32, slot.kp32, slot.nx32))) return rc;
-    if (!g64.empty() && (rc = enqueue_group<double>(sv, slot, g64, t64, slot.kp64, slot.nx64))) return rc;
+    if (!g32.empty() && (rc = enqueue_group<float>(sv, slot, g32, t32, slot.kp32, slot.bp32, slot.nx32))) return rc;
+    if (!g64.empty() && (rc = enqueue_group<double>(sv, slot, g64, t64, slot.kp64, slot.bp64, slot.nx64))) return rc;
     HIP_TRY(hipEventRecord(slot.e1, slot.stream));
     slot.live = true;
     return MCG_OK;

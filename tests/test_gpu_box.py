@@ -113,3 +113,39 @@ def test_fp32_matches_general_steps(name):
         assert sb[k] == se[k]
     if fe.size:
         close(fb, fe, 1e-5)
+
+
+@pytest.mark.parametrize("precision", [abi.FP64, abi.FP32_FLIGHT])
+def test_batch_of_all_matches_single(precision):
+    """Every case above in one batch, several sizes of each: the one-box solves
+    share a launch (1-D, 2-D and 3-D tallies, parts, all tally kinds), the
+    others the general batch kernel.  Statistics exactly, tallies to 1e-9
+    (other summation orders)."""
+    mat = materials.si_like(300.0)
+    scs, probs = [], []
+    for i, name in enumerate(sorted(CASES)):
+        dom, tally = CASES[name]
+        scs.append(engine.Scene(mat, dom()))
+        probs.append(scenes.problem((7, 1500, 9001)[i % 3], tally=tally, maxscat=60, seed=20 + i, precision=precision))
+    alone = [sc.solve(p) for sc, p in zip(scs, probs)]
+    fields, stats = engine.batch_solve(scs, probs)
+    with engine.Batch(scs, probs) as b:
+        replays = [b.run() for _ in range(2)]
+    for got_f, got_s in [(fields, stats)] + replays:
+        for (fa, sa, _), fb, sb in zip(alone, got_f, got_s):
+            for k in ("bundles", "steps", "escapes", "absorbed", "truncated"):
+                assert sa[k] == sb[k]
+            if fa.size:
+                close(fb, fa, 1e-9)
+    for sc in scs:
+        sc.close()
+
+
+def test_batch_of_one_tiny_solve():
+    mat, dom = materials.si_like(300.0), CASES["cols_255"][0]()
+    with engine.Scene(mat, dom) as sc:
+        prob = scenes.problem(2, seed=3, precision=abi.FP32_FLIGHT)
+        fa, sa, _ = sc.solve(prob)
+        fb, sb = engine.batch_solve([sc], [prob])
+    assert sa["steps"] == sb[0]["steps"]
+    close(fb[0], fa, 1e-9)
