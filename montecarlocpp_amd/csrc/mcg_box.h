@@ -39,6 +39,7 @@ enum : uint32_t { kCodeIntrinsic = 24, kCodePore = 28 };
 
 constexpr uint32_t kAlive = 0xFFFFFFFFu;
 
+
 // LDS row stride of a 1-D tally and of its difference array, in doubles: a
 // compile-time stride puts the rows of one column at immediate offsets of one
 // address (4 addresses a step instead of 16).
@@ -381,13 +382,12 @@ __device__ __forceinline__ void box_tally(const BoxCell<F>& B, const BoxView<F>&
     }
 }
 
-// One scatter-step: the flight (problem.cpp:401-416) and the event
-// (problem.cpp:418-433), as flight_step and collide_step take them.  Returns
-// the bundle's fate, kAlive while it lives.
-template <typename F, bool kLdsTables, int kAxes, int kRows>
-__device__ __forceinline__ uint32_t box_step(const BoxCell<F>& B, const BoxView<F>& V, BoxLane<F>& L,
-                                             BoxWalk<F, kAxes>& W) {
-    // ---- flight: the face ahead on each axis, the pore, the free path
+// The flight of a scatter-step (problem.cpp:401-416, flight_step): the face
+// ahead on each axis, the pore, the free path; moves L and returns the event's
+// code.  pre and dmin describe the flight; outside is the kill test.
+template <typename F>
+__device__ __forceinline__ uint32_t box_flight(const BoxCell<F>& B, BoxLane<F>& L, dev::V3<F>& pre, F& dmin_out,
+                                               bool& outside_out) {
     const F p[3] = {L.pos.x, L.pos.y, L.pos.z}, u[3] = {L.dir.x, L.dir.y, L.dir.z};
     F dmin = L.path;
     uint32_t hit = kCodeIntrinsic;
@@ -431,7 +431,8 @@ __device__ __forceinline__ uint32_t box_step(const BoxCell<F>& B, const BoxView<
     }
     L.path -= dmin;
     if (L.path < dev::Real<F>::kMin) L.path = F(0);
-    const dev::V3<F> pre = L.pos;
+    pre = L.pos;
+    dmin_out = dmin;
     L.pos = dev::V3<F>{pre.x + dmin * u[0], pre.y + dmin * u[1], pre.z + dmin * u[2]};
     L.nstep++;
     // kill test (subdomain.cpp:186-190)
@@ -448,33 +449,93 @@ __device__ __forceinline__ uint32_t box_step(const BoxCell<F>& B, const BoxView<
         const F dx = L.pos.x - B.cx, dy = L.pos.y - B.cy;
         outside |= dx * dx + dy * dy < B.rin2;
     }
-    uint32_t fate = MCG_ESCAPED;
-    if (!outside) {
-        box_tally<F, kAxes, kRows>(B, V, L, pre, dmin, W);
+    outside_out = outside;
+    return hit;
+}
 
-        // ---- event
-        uint32_t kind = (B.kinds >> hit) & 15u;
-        const bool intr = kind == kKindIntrinsic;
-        bool pore = false;
-        if (B.pore >= 0) {
-            pore = kind == kKindPore;
-            kind = pore ? uint32_t(B.pore) : kind;
+// What an event may draw: the isotropic and the Lambertian direction (about
+// z), the free path and speed of a scattered mode, the word of the
+// partial-specularity test.
+template <typename F>
+struct Draws {
+    dev::V3<F> iso, lam;
+    F path, vel;
+    uint32_t spec;
+};
+
+template <typename F, bool kLdsTables>
+__device__ __forceinline__ F box_mode_speed(const BoxView<F>& V, uint32_t mode) {
+    const F vel = V.vel[mode];
+    if constexpr (sizeof(F) == 8 || kLdsTables) return vel;
+    else return __builtin_amdgcn_rcpf(vel);
+}
+
+template <typename F>
+__device__ __forceinline__ dev::Event box_event_stream(const BoxCell<F>& B, uint32_t event, int64_t id) {
+    uint32_t k0 = B.k0, k1 = B.k1;
+    in_scalar(k0);
+    in_scalar(k1);
+    return dev::Event{k0, k1, event, uint32_t(id), uint32_t(uint64_t(id) >> 32)};
+}
+
+// All draws of one event, whatever its kind (the drain's draws ahead).
+template <typename F, bool kLdsTables>
+__device__ __forceinline__ Draws<F> box_draws(const BoxCell<F>& B, const BoxView<F>& V, uint32_t event, int64_t id) {
+    const dev::Event ev = box_event_stream(B, event, id);
+    const uint4 b0 = ev.block(0), b1 = low_block<F>(ev, 1);
+    Draws<F> D;
+    D.spec = b1.w;
+    if constexpr (sizeof(F) == 4)
+        if (B.partial) D.spec = ev.block(1).w;
+    const F r = dev::Real<F>::uniform(b0.x, b1.x) * F(2) + F(-1);
+    const F ar = r < F(0) ? -r : r;
+    const F si = dev::Real<F>::sqrt_(F(1) - r * r), sl = dev::Real<F>::sqrt_(ar);
+    const F q = dev::Real<F>::uniform(b0.y, b1.y) * F(2) + F(-1);
+    F sq, cq;
+    dev::Real<F>::sincos_pi(q, sq, cq);
+    D.iso = dev::V3<F>{si * cq, si * sq, r};
+    D.lam = dev::V3<F>{sl * cq, sl * sq, dev::Real<F>::sqrt_(F(1) - ar)};
+    const uint32_t mode = dev::alias_draw(V.scat, uint32_t(B.nmodes), b0.w);
+    D.path = draw_path<F>(ev, b0, b1, V.mfp[mode]);
+    D.vel = box_mode_speed<F, kLdsTables>(V, mode);
+    return D;
+}
+
+// The event of a scatter-step (problem.cpp:418-433, collide_step), with its
+// draws given (kAhead) or made here as far as the event needs them.  Returns
+// the bundle's fate, kAlive while it lives.
+template <typename F, bool kLdsTables, bool kAhead>
+__device__ __forceinline__ uint32_t box_event(const BoxCell<F>& B, const BoxView<F>& V, uint32_t hit, BoxLane<F>& L,
+                                              const Draws<F>& ahead) {
+    uint32_t kind = (B.kinds >> hit) & 15u;
+    const bool intr = kind == kKindIntrinsic;
+    bool pore = false;
+    if (B.pore >= 0) {
+        pore = kind == kKindPore;
+        kind = pore ? uint32_t(B.pore) : kind;
+    }
+    const BoxFace<F>& P = V.faces[hit < kCodeIntrinsic ? hit >> 2 : 0u];
+    const dev::Event ev = box_event_stream(B, L.nstep, L.id);
+    if (B.partial) {
+        if (kind == MCG_PARTIAL) {
+            uint32_t w;
+            if constexpr (kAhead) w = ahead.spec;
+            else w = ev.block(1).w;
+            kind = w < (pore ? B.pore_thr : P.spec_thr) ? uint32_t(MCG_SPEC) : uint32_t(MCG_DIFF);
         }
-        uint32_t k0 = B.k0, k1 = B.k1;
-        in_scalar(k0);
-        in_scalar(k1);
-        const dev::Event ev{k0, k1, L.nstep, uint32_t(L.id), uint32_t(uint64_t(L.id) >> 32)};
-        const BoxFace<F>& P = V.faces[hit < kCodeIntrinsic ? hit >> 2 : 0u];
-        if (B.partial) {
-            if (kind == MCG_PARTIAL)
-                kind = ev.block(1).w < (pore ? B.pore_thr : P.spec_thr) ? uint32_t(MCG_SPEC) : uint32_t(MCG_DIFF);
-        }
-        L.nbdry += intr ? 0u : 1u;
-        const bool draws = intr | (kind == MCG_DIFF);
-        dev::V3<F> d = L.dir;
-        if (draws) {
-            // the event's random direction: isotropic cos(theta) = r or
-            // Lambertian sin^2(theta) = |r| about z, then turned onto the normal
+    }
+    L.nbdry += intr ? 0u : 1u;
+    dev::V3<F> d = L.dir;
+    if (intr | (kind == MCG_DIFF)) {
+        // isotropic cos(theta) = r or Lambertian sin^2(theta) = |r| about z,
+        // then turned onto the normal
+        F path = F(0), vel = F(0);
+        if constexpr (kAhead) {
+            d = dev::V3<F>{intr ? ahead.iso.x : ahead.lam.x, intr ? ahead.iso.y : ahead.lam.y,
+                           intr ? ahead.iso.z : ahead.lam.z};
+            path = ahead.path;
+            vel = ahead.vel;
+        } else {
             const uint4 b0 = ev.block(0), b1 = low_block<F>(ev, 1);
             const F r = dev::Real<F>::uniform(b0.x, b1.x) * F(2) + F(-1);
             const F ar = r < F(0) ? -r : r;
@@ -484,42 +545,60 @@ __device__ __forceinline__ uint32_t box_step(const BoxCell<F>& B, const BoxView<
             F sq, cq;
             dev::Real<F>::sincos_pi(q, sq, cq);
             d = dev::V3<F>{sinT * cq, sinT * sq, cosT};
-            L.nscat++;
             if (intr) {
                 const uint32_t mode = dev::alias_draw(V.scat, uint32_t(B.nmodes), b0.w);
-                const F mfp = V.mfp[mode], vel = V.vel[mode];
-                L.path = draw_path<F>(ev, b0, b1, mfp);
-                if constexpr (sizeof(F) == 8) L.vel = vel;
-                else if constexpr (kLdsTables) L.vel = L.sg * vel;
-                else L.vel = L.sg * __builtin_amdgcn_rcpf(vel);
-            } else {
-                F m[9];
+                const F mfp = V.mfp[mode];
+                vel = box_mode_speed<F, kLdsTables>(V, mode);
+                path = draw_path<F>(ev, b0, b1, mfp);
+            }
+        }
+        L.nscat++;
+        if (intr) {
+            L.path = path;
+            L.vel = sizeof(F) == 4 ? L.sg * vel : vel;
+        } else {
+            F m[9];
 #pragma unroll
-                for (int i = 0; i < 9; ++i) m[i] = P.rot[i];
-                if (pore) rotation_to_wall(box_wall_normal(B, L.pos), m);
-                d = dev::matvec(m, d);
-            }
+            for (int i = 0; i < 9; ++i) m[i] = P.rot[i];
+            if (pore) rotation_to_wall(box_wall_normal(B, L.pos), m);
+            d = dev::matvec(m, d);
         }
-        if (kind == MCG_SPEC) {
-            // I - 2 n n^T of an axis: the component's sign
-            const uint32_t axis = hit >> 3;
-            d.x = axis == 0u ? -d.x : d.x;
-            d.y = axis == 1u ? -d.y : d.y;
-            d.z = axis == 2u ? -d.z : d.z;
-            if (pore) {
-                F m[9];
-                reflection_off(box_wall_normal(B, L.pos), m);
-                d = dev::matvec(m, L.dir);
-            }
+    }
+    if (kind == MCG_SPEC) {
+        // I - 2 n n^T of an axis: the component's sign
+        const uint32_t axis = hit >> 3;
+        d.x = axis == 0u ? -d.x : d.x;
+        d.y = axis == 1u ? -d.y : d.y;
+        d.z = axis == 2u ? -d.z : d.z;
+        if (pore) {
+            F m[9];
+            reflection_off(box_wall_normal(B, L.pos), m);
+            d = dev::matvec(m, L.dir);
         }
-        if (kind == MCG_PERI) {
-            // the map's rotation is the identity (box_cell takes no other)
-            L.pos = dev::V3<F>{L.pos.x + P.pt[0], L.pos.y + P.pt[1], L.pos.z + P.pt[2]};
-        }
-        L.dir = unit_of(d);
-        fate = L.nstep >= B.maxloop ? uint32_t(MCG_MAXLOOP) : kAlive;
-        fate = L.nscat >= B.maxscat ? uint32_t(MCG_MAXSCAT) : fate;
-        fate = kind == MCG_ISOT ? uint32_t(MCG_ABSORBED) : fate;
+    }
+    if (kind == MCG_PERI) {
+        // the map's rotation is the identity (box_cell takes no other)
+        L.pos = dev::V3<F>{L.pos.x + P.pt[0], L.pos.y + P.pt[1], L.pos.z + P.pt[2]};
+    }
+    L.dir = unit_of(d);
+    uint32_t fate = L.nstep >= B.maxloop ? uint32_t(MCG_MAXLOOP) : kAlive;
+    fate = L.nscat >= B.maxscat ? uint32_t(MCG_MAXSCAT) : fate;
+    fate = kind == MCG_ISOT ? uint32_t(MCG_ABSORBED) : fate;
+    return fate;
+}
+
+// One scatter-step.
+template <typename F, bool kLdsTables, int kAxes, int kRows>
+__device__ __forceinline__ uint32_t box_step(const BoxCell<F>& B, const BoxView<F>& V, BoxLane<F>& L,
+                                             BoxWalk<F, kAxes>& W) {
+    dev::V3<F> pre;
+    F dmin;
+    bool outside;
+    const uint32_t hit = box_flight(B, L, pre, dmin, outside);
+    uint32_t fate = MCG_ESCAPED;
+    if (!outside) {
+        box_tally<F, kAxes, kRows>(B, V, L, pre, dmin, W);
+        fate = box_event<F, kLdsTables, false>(B, V, hit, L, Draws<F>{});
     }
     return fate;
 }
@@ -648,6 +727,170 @@ __device__ __forceinline__ void box_emit(ParamPtr<F> kp, const BoxCell<F>& B, co
     L.id = n;
 }
 
+// Lane l's value of x as lane addr / 4 of the wavefront holds it (all lanes
+// take part).
+__device__ __forceinline__ int lane_pull(int addr, int x) { return __builtin_amdgcn_ds_bpermute(addr, x); }
+__device__ __forceinline__ uint32_t lane_pull(int addr, uint32_t x) { return uint32_t(lane_pull(addr, int(x))); }
+__device__ __forceinline__ float lane_pull(int addr, float x) {
+    return __int_as_float(lane_pull(addr, __float_as_int(x)));
+}
+__device__ __forceinline__ int64_t lane_pull(int addr, int64_t x) {
+    const uint32_t lo = lane_pull(addr, uint32_t(uint64_t(x))), hi = lane_pull(addr, uint32_t(uint64_t(x) >> 32));
+    return int64_t(uint64_t(lo) | (uint64_t(hi) << 32));
+}
+__device__ __forceinline__ double lane_pull(int addr, double x) {
+    return __hiloint2double(lane_pull(addr, __double2hiint(x)), lane_pull(addr, __double2loint(x)));
+}
+template <typename F>
+__device__ __forceinline__ dev::V3<F> lane_pull(int addr, const dev::V3<F>& v) {
+    return dev::V3<F>{lane_pull(addr, v.x), lane_pull(addr, v.y), lane_pull(addr, v.z)};
+}
+
+struct BoxStats {   // wavefront-uniform
+    unsigned long long steps = 0, ended = 0, absorbed = 0, escaped = 0;
+};
+
+// Books the lanes whose bundle ended (fate not kAlive); all lanes call.
+template <typename F>
+__device__ __forceinline__ void box_end(const BoxCell<F>& B, ParamPtr<F> kp, const BoxLane<F>& L, uint32_t fate,
+                                        bool& active, BoxStats& st) {
+    const uint64_t ended = __ballot(fate != kAlive);
+    if (ended == 0ull) return;
+    st.ended += popc(ended);
+    st.absorbed += popc(__ballot(fate == MCG_ABSORBED));
+    st.escaped += popc(__ballot(fate == MCG_ESCAPED));
+    if (fate != kAlive) {
+        active = false;
+        if (B.counts && B.part == 0) {
+            const ParamPtr<F> k = params_here<F>(kp);
+            const int64_t i = L.id - k->first;
+            in_global(k->c_nscat)[i] = L.nscat;
+            in_global(k->c_nbdry)[i] = L.nbdry;
+            in_global(k->c_nstep)[i] = L.nstep;
+            in_global(k->c_fate)[i] = fate;
+        }
+    }
+}
+
+// The drain of a wavefront: its last bundles, at most kDrainLanes, with no id
+// left to claim.  What bounds it is the chain of a step's instructions, one
+// bundle each, while most lanes are idle; so the idle lanes take over what does
+// not depend on the bundle's path.  The bundles sit in the first `span` lanes
+// (a power of two) and step together;
+//  - the draws of a bundle's next 64 / span events (they depend on the id and
+//    the event's number alone) are made by 64 / span lanes at once, and a step
+//    fetches its event's;
+//  - a flight's tally is left to a lane of its own, and the 64 lanes' flights
+//    are tallied (and their grid walks walked) together once all hold one.
+// A step is then its flight and its event's turn.
+// A lone bundle's step, before and now (us, FP32 / FP64): slab 1.19 / 2.08 and
+// 0.78 / 1.02, film (12 x 6 map) 1.87 / 2.87 and 0.81 / 1.52, porous film
+// (64 x 64) 2.92 / 3.77 and 0.92 / 1.72; bar 1e6 FP64 3.24 -> 2.01 ms, film 1e6
+// 12.5 -> 7.75 ms.  8, 16 or 32 lanes: bar FP64 2.11 / 2.01 / 1.96 ms, film
+// 7.84 / 7.75 / 7.70 ms, 256 slabs 13.05 / 12.99 / 13.08 ms.
+#ifndef MCG_DRAIN_LANES
+#define MCG_DRAIN_LANES 16
+#endif
+constexpr int kDrainLanes = MCG_DRAIN_LANES;
+
+template <typename F, bool kLdsTables, int kAxes, int kRows>
+__device__ __forceinline__ void box_drain(const BoxCell<F>& B, ParamPtr<F> kp, const BoxView<F>& V, int lane,
+                                          uint64_t lt_mask, BoxLane<F>& L, bool active, BoxStats& st) {
+    int span = 2 * kDrainLanes, shift = 0;   // lanes the bundles sit in; log2 of the draws ahead per bundle
+    int at = 0, ahead = 0;                   // next event among the draws ahead, how many there are
+    int slot = 0;                            // lanes holding a flight to tally
+    Draws<F> D;
+    dev::V3<F> fpre, fpos;                   // this lane's flight to tally
+    F fdmin = F(0), fvel = F(0);
+    bool pending = false;
+    for (;;) {
+        const uint64_t live = __ballot(active);
+        if (live == 0ull || slot + span > kWave) {
+            // the flights held are tallied together
+            BoxWalk<F, kAxes> W;
+            W.left = 0;
+            if (pending) {
+                BoxLane<F> T;
+                T.pos = fpos;
+                T.sg = fvel < F(0) ? F(-1) : F(1);
+                T.vel = sizeof(F) == 4 ? fvel : fabs(fvel);
+                box_tally<F, kAxes, kRows>(B, V, T, fpre, fdmin, W);
+            }
+            if constexpr (kAxes != 0)
+                while (__ballot(W.left > 0) != 0ull) box_walk_some<kWalkUnroll, kRows>(W, B, V.tally);
+            pending = false;
+            slot = 0;
+        }
+        if (live == 0ull) return;
+        const int n = popc(live);
+        if (2 * n <= span) {
+            // the live bundles into the first lanes, in order
+            const int to = active ? popc(live & lt_mask) : n + popc(~live & lt_mask);
+            const int from = 4 * __builtin_amdgcn_ds_permute(4 * to, lane);
+            L.pos = lane_pull(from, L.pos);
+            L.dir = lane_pull(from, L.dir);
+            L.path = lane_pull(from, L.path);
+            L.vel = lane_pull(from, L.vel);
+            L.sg = lane_pull(from, L.sg);
+            L.nscat = lane_pull(from, L.nscat);
+            L.nbdry = lane_pull(from, L.nbdry);
+            L.nstep = lane_pull(from, L.nstep);
+            L.id = lane_pull(from, L.id);
+            active = lane < n;
+            span = 1;
+            shift = 6;
+            while (span < n) {
+                span *= 2;
+                --shift;
+            }
+            ahead = at = 0;
+        }
+        if (at == ahead) {
+            // lane l draws event number l % (64 / span) ahead of bundle l / (64 / span)
+            const int of = 4 * (lane >> shift);
+            const int64_t id = lane_pull(of, L.id);
+            const uint32_t event = lane_pull(of, L.nstep) + 1u + uint32_t(lane & ((1 << shift) - 1));
+            D = box_draws<F, kLdsTables>(B, V, event, id);
+            at = 0;
+            ahead = 1 << shift;
+        }
+        // (pulled by every lane: a lane that is switched off passes nothing on)
+        Draws<F> E;
+        const int src = 4 * (((lane << shift) + at) & (kWave - 1));
+        E.iso = lane_pull(src, D.iso);
+        E.lam = lane_pull(src, D.lam);
+        E.path = lane_pull(src, D.path);
+        E.vel = lane_pull(src, D.vel);
+        E.spec = B.partial ? lane_pull(src, D.spec) : 0u;
+        ++at;
+        dev::V3<F> pre = L.pos;
+        F dmin = F(0);
+        bool outside = true;
+        uint32_t hit = kCodeIntrinsic;
+        if (active) hit = box_flight(B, L, pre, dmin, outside);
+        st.steps += n;
+        // flights to lanes slot .. slot + span - 1
+        const bool flown = active && !outside;
+        const uint64_t flights = __ballot(flown);
+        const int give = lane - slot;
+        const int giver = 4 * (give & (kWave - 1));
+        const dev::V3<F> gpre = lane_pull(giver, pre), gpos = lane_pull(giver, L.pos);
+        const F gdmin = lane_pull(giver, dmin), gvel = lane_pull(giver, sizeof(F) == 4 ? L.vel : L.sg * L.vel);
+        if (uint32_t(give) < uint32_t(span) && (flights >> (give & (kWave - 1)) & 1ull)) {
+            fpre = gpre;
+            fpos = gpos;
+            fdmin = gdmin;
+            fvel = gvel;
+            pending = true;
+        }
+        slot += span;
+        uint32_t fate = kAlive;
+        if (flown) fate = box_event<F, kLdsTables, true>(B, V, hit, L, E);
+        else if (active) fate = MCG_ESCAPED;
+        box_end(B, kp, L, fate, active, st);
+    }
+}
+
 // A wavefront's loop over the bundles it claims (trajectory_kernel's loop).
 // The refill is looked at only when some lane has run out of work since the
 // last look: a wavefront left with a few long-lived bundles goes from step to
@@ -660,7 +903,7 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
     BoxLane<F> L, N;
     BoxWalk<F, kAxes> W;
     W.left = 0;
-    unsigned long long steps = 0, n_end = 0, n_abs = 0, n_esc = 0;   // wavefront-uniform
+    BoxStats st;
     uint64_t busy = ~0ull, last_busy = 0ull;
     for (;;) {
         if (busy != last_busy || busy == 0ull) {
@@ -712,28 +955,19 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
                 if (__ballot(active || walking) == 0ull) break;
             }
             last_busy = __ballot(active || walking);
-        }
-        const bool go = active && !(W.left > 0);
-        steps += popc(__ballot(go));
-        uint32_t fate = kAlive;
-        if (go) fate = box_step<F, kLdsTables, kAxes, kRows>(B, V, L, W);
-        const uint64_t ended = __ballot(fate != kAlive);
-        if (ended != 0ull) {
-            n_end += popc(ended);
-            n_abs += popc(__ballot(fate == MCG_ABSORBED));
-            n_esc += popc(__ballot(fate == MCG_ESCAPED));
-            if (fate != kAlive) {
-                active = false;
-                if (B.counts && B.part == 0) {
-                    const ParamPtr<F> k = params_here<F>(kp);
-                    const int64_t i = L.id - k->first;
-                    in_global(k->c_nscat)[i] = L.nscat;
-                    in_global(k->c_nbdry)[i] = L.nbdry;
-                    in_global(k->c_nstep)[i] = L.nstep;
-                    in_global(k->c_fate)[i] = fate;
-                }
+            // no id left (one lane found none) and few bundles: the drain
+            if (__ballot(drained) != 0ull && __ballot(full) == 0ull && popc(__ballot(active)) <= kDrainLanes) {
+                if constexpr (kAxes != 0)
+                    while (__ballot(W.left > 0) != 0ull) box_walk_some<kWalkUnroll, kRows>(W, B, V.tally);
+                box_drain<F, kLdsTables, kAxes, kRows>(B, kp, V, lane, lt_mask, L, active, st);
+                break;
             }
         }
+        const bool go = active && !(W.left > 0);
+        st.steps += popc(__ballot(go));
+        uint32_t fate = kAlive;
+        if (go) fate = box_step<F, kLdsTables, kAxes, kRows>(B, V, L, W);
+        box_end(B, kp, L, fate, active, st);
         if constexpr (kAxes != 0) {
             // the walk phase (walk_phase): while kWalkQuorum lanes walk or no
             // other lane has a step to take
@@ -745,13 +979,13 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
         }
         busy = __ballot(active || W.left > 0);
     }
-    if (lane == 0 && n_end != 0 && B.part == 0) {
+    if (lane == 0 && st.ended != 0 && B.part == 0) {
         unsigned long long* const c = in_global(params_here<F>(kp)->counters);
-        atomicAdd(c + C_STEPS, steps);
-        atomicAdd(c + C_ESC, n_esc);
-        atomicAdd(c + C_ABS, n_abs);
-        atomicAdd(c + C_TRUNC, n_end - n_abs - n_esc);
-        atomicAdd(c + C_BUNDLES, n_end);
+        atomicAdd(c + C_STEPS, st.steps);
+        atomicAdd(c + C_ESC, st.escaped);
+        atomicAdd(c + C_ABS, st.absorbed);
+        atomicAdd(c + C_TRUNC, st.ended - st.absorbed - st.escaped);
+        atomicAdd(c + C_BUNDLES, st.ended);
     }
 }
 
