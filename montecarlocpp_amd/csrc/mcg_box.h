@@ -39,6 +39,16 @@ enum : uint32_t { kCodeIntrinsic = 24, kCodePore = 28 };
 
 constexpr uint32_t kAlive = 0xFFFFFFFFu;
 
+// Walking lanes below which a walk phase of a four-row map ends (kWalkQuorum
+// for fewer rows).  Four FP64 LDS adds a crossing bound such a map: the LDS
+// takes 10 cycles for an add of 20 lanes and 20 for one of 64 (bank conflicts
+// even out), so fuller phases pay although they leave fewer lanes to step.
+// Porous film 1e7, 64 x 64, quorum 20 / 32 / 40 / 44 / 48: 70.8 / 66.6 / 65.1 /
+// 64.7 / 66.1 ms; 24 mixed solves replayed 11.07 / 11.1 / 11.2 / 11.3 / 11.5 ms.
+// One row at a time (a 128 x 128 map in parts) is bound by the steps: quorum
+// 20 / 28 / 36 / 44: 9.6 / 9.8 / 10.2 / 11.3 ms.
+constexpr int kBoxWalkQuorum4 = 36;
+
 
 // LDS row stride of a 1-D tally and of its difference array, in doubles: a
 // compile-time stride puts the rows of one column at immediate offsets of one
@@ -973,7 +983,7 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
             // other lane has a step to take
             for (;;) {
                 const uint64_t m = __ballot(W.left > 0);
-                if (m == 0ull || (popc(m) < kWalkQuorum && __ballot(active && !(W.left > 0)) != 0ull)) break;
+                if (m == 0ull || (popc(m) < (kRows == kMaxRows ? kBoxWalkQuorum4 : kWalkQuorum) && __ballot(active && !(W.left > 0)) != 0ull)) break;
                 box_walk_some<kWalkUnroll, kRows>(W, B, V.tally);
             }
         }
