@@ -37,8 +37,6 @@
 enum : uint32_t { kKindIntrinsic = 8, kKindPore = 9 };
 enum : uint32_t { kCodeIntrinsic = 24, kCodePore = 28 };
 
-constexpr uint32_t kAlive = 0xFFFFFFFFu;
-
 // Walking lanes below which a walk phase of a four-row map ends (kWalkQuorum
 // for fewer rows).  Four FP64 LDS adds a crossing bound such a map: the LDS
 // takes 10 cycles for an add of 20 lanes and 20 for one of 64 (bank conflicts

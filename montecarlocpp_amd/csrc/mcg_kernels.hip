@@ -666,19 +666,24 @@ __device__ __forceinline__ void rotation_to_wall(const dev::V3<F>& n, F (&r)[9])
     r[8] = F(1) - (txx + tyy);
 }
 
+// The pore wall's normal at p, away from the axis.  FP64 divides by the radius
+// as the checker does; FP32 flight normalises the offset from the axis directly
+// (the same direction).
+template <typename F>
+__device__ __forceinline__ dev::V3<F> wall_normal(const DevPore<F>& Q, const dev::V3<F>& p) {
+    if constexpr (sizeof(F) == 8)
+        return dev::normalized(dev::V3<F>{(p.x - Q.cx) / Q.r, (p.y - Q.cy) / Q.r, F(0)});
+    else
+        return dev::normalized(dev::V3<F>{p.x - Q.cx, p.y - Q.cy, F(0)});
+}
+
 // Scatter off a cylindrical pore wall.  The wall normal at the hit point
 // points away from the axis (into the material); the reflection and the
 // Lambertian rotation are built from it as for a planar face.
 template <typename F>
 __device__ __forceinline__ void pore_scatter(const DevPore<F>& Q, const dev::Event& ev, const uint4& b0,
                                              const uint4& b1, Lane<F>& L) {
-    // FP64 divides by the radius as the checker does; FP32 flight
-    // normalises the offset from the axis directly (the same direction)
-    dev::V3<F> n;
-    if constexpr (sizeof(F) == 8)
-        n = dev::normalized(dev::V3<F>{(L.pos.x - Q.cx) / Q.r, (L.pos.y - Q.cy) / Q.r, F(0)});
-    else
-        n = dev::normalized(dev::V3<F>{L.pos.x - Q.cx, L.pos.y - Q.cy, F(0)});
+    const dev::V3<F> n = wall_normal(Q, L.pos);
     int kind = Q.kind;
     if (kind == MCG_PARTIAL) kind = spec_word<F>(ev, b1) < Q.spec_thr ? MCG_SPEC : MCG_DIFF;
     F r[9];
@@ -822,6 +827,8 @@ struct LaneStats {
     }
 };
 
+constexpr uint32_t kAlive = 0xFFFFFFFFu;   // no fate yet
+
 // FP32 flight at an Inter face with several partners, when rounding has
 // left the point inside none of them: the partner it is least outside of
 // (the deepest face violation, in units of that cell's tolerance), with the
@@ -855,6 +862,25 @@ __device__ __forceinline__ int inter_nearest(const View<F>& V, const DevPlane<F>
         }
     }
     return best;
+}
+
+// The cell an Inter face's crossing continues in (boundary.cpp:349-359), -1
+// when no partner holds the point.
+template <typename F>
+__device__ __forceinline__ int inter_target(const KParams<F>& K, const View<F>& V, const DevPlane<F>& P,
+                                            dev::V3<F>& pos) {
+    if (P.icnt == 1) return P.target;
+    int target = -1;
+    for (int c = 0; c < P.icnt; ++c) {
+        const int cand = K.inter_list[P.ibeg + c];
+        if (inside(V.planes, V.sdoms[cand], V.pores, pos)) {
+            target = cand;
+            break;
+        }
+    }
+    if constexpr (sizeof(F) == 4)
+        if (target < 0) target = inter_nearest(V, P, K.inter_list, pos);
+    return target;
 }
 
 // The intrinsic and planar-face scatters of FP32 flight in one code path:
@@ -909,42 +935,24 @@ __device__ __forceinline__ void scatter_fp32(const KParams<F>& K, const View<F>&
     } else if (kind == MCG_ISOT) {
         fate = MCG_ABSORBED;
     } else if (kind == MCG_INTER) {
-        int target = -1;
-        if (P.icnt == 1) {
-            target = P.target;
-        } else {
-            for (int c = 0; c < P.icnt; ++c) {
-                const int cand = K.inter_list[P.ibeg + c];
-                if (inside(V.planes, V.sdoms[cand], V.pores, L.pos)) {
-                    target = cand;
-                    break;
-                }
-            }
-            if (target < 0) target = inter_nearest(V, P, K.inter_list, L.pos);
-        }
+        const int target = inter_target<F>(K, V, P, L.pos);
         if (target < 0) fate = MCG_ESCAPED;
         else L.sdom = target;
     }
 }
 
-// The flight half of a scatter-step (problem.cpp:401-416): advect to the
-// nearest face, pore wall or intrinsic event, the kill test, and the tally of
-// the flight.  Returns the event (a plane index, -1 intrinsic, -3 the pore)
-// and sets fate to MCG_ESCAPED when the bundle is lost; dmin and apos receive
-// the distance and the position after the flight.  `walking` is set when the
-// flight's 2-D / 3-D tally walk was deferred to W (FP32 flight only).
-template <typename F, int kDefer>
-__device__ __forceinline__ int flight_step(const KParams<F>& K, const View<F>& V, const Sink& sink,
-                                           Lane<F>& L, WalkOf<F, kDefer>& W, bool& walking, uint32_t& fate,
-                                           F& dmin_out, dev::V3<F>& apos, int32_t& pbeg_out,
-                                           int32_t& pore_out) {
-    walking = false;
+// The flight of a scatter-step (problem.cpp:401-413): advect to the nearest
+// face, pore wall or intrinsic event and the kill test.  Returns the event (a
+// plane index, -1 intrinsic, -3 the pore) and sets fate to MCG_ESCAPED when the
+// bundle is lost; pre and dmin_out receive the start and the distance, pbeg_out
+// and pore_out the cell's face base and pore (the collision gets them from
+// here rather than read them again behind the tally's LDS atomics).
+template <typename F>
+__device__ __forceinline__ int advect_step(const View<F>& V, Lane<F>& L, uint32_t& fate, F& dmin_out,
+                                           dev::V3<F>& pre, int32_t& pbeg_out, int32_t& pore_out) {
     const DevSdom<F>& S = V.sdoms[L.sdom];
-    const F vel = V.vel[L.mode];
     // the cell's fields the flight tests, read once and together (a lone
-    // lane would otherwise wait for each read behind its own branch); the
-    // collision gets the face base and the pore from here rather than read
-    // them again behind the tally's LDS atomics
+    // lane would otherwise wait for each read behind its own branch)
     const int32_t s_box = S.box, s_pore = S.pore, s_pbeg = S.pbeg;
     const F s_eps = S.eps;
     pbeg_out = s_pbeg;
@@ -1094,10 +1102,9 @@ __device__ __forceinline__ int flight_step(const KParams<F>& K, const View<F>& V
     }
     L.scat_next -= dmin;
     if (L.scat_next < dev::Real<F>::kMin) L.scat_next = F(0);
-    const dev::V3<F> pre = L.pos;
+    pre = L.pos;
     L.pos = dev::V3<F>{pre.x + dmin * L.dir.x, pre.y + dmin * L.dir.y, pre.z + dmin * L.dir.z};
     L.nstep++;
-    apos = L.pos;
     dmin_out = dmin;
     // kill test (subdomain.cpp:186-190): outside any face by more than eps
     bool outside;
@@ -1127,27 +1134,51 @@ __device__ __forceinline__ int flight_step(const KParams<F>& K, const View<F>& V
     } else {
         outside = !inside(V.planes, S, V.pores, L.pos);
     }
-    if ((dmin < -s_eps) | outside) {
-        fate = MCG_ESCAPED;
-    } else {
-        // tally (problem.cpp:414-416 with the kinds of problem.cpp:473-637);
-        // each amount is a sign times an F value, exact in F and in FP64
-        const F sg = F(L.sign);
-        const F dt = sg * dev::Real<F>::div(dmin, vel);
-        const F dx = sg * (L.pos.x - pre.x);
-        const F dy = sg * (L.pos.y - pre.y);
-        const F dz = sg * (L.pos.z - pre.z);
-        const int tk = K.tally;
-        const bool with_t = tk == MCG_TEMP || tk == MCG_MULTI || tk == MCG_CUMTEMP;
-        const F amt[kMaxRows] = {with_t ? dt : dx, with_t ? dx : dy, with_t ? dy : dz, dz};
-        const int nv = tk == MCG_MULTI ? 4 : (with_t ? 1 : 3);
-        int r0 = 0;
-        if (tk >= MCG_CUMTEMP) {
-            const int bin = int((int64_t(L.nscat) + K.step_cum - 1) / K.step_cum);
-            r0 = tk == MCG_CUMTEMP ? bin : 3 * bin;
-        }
-        walking = accumulate<F, kDefer>(S, sink, pre, L.pos, r0, nv, amt, W);
+    if ((dmin < -s_eps) | outside) fate = MCG_ESCAPED;
+    return hit;
+}
+
+// The tally of a flight pre -> pos of length dmin in cell S (problem.cpp:414-416
+// with the kinds of problem.cpp:473-637); each amount is a sign times an F
+// value, exact in F and in FP64.  Returns true when a 2-D / 3-D walk was set up
+// in W (kDefer).
+template <typename F, int kDefer>
+__device__ __forceinline__ bool tally_step(const KParams<F>& K, const DevSdom<F>& S, const Sink& sink,
+                                           const dev::V3<F>& pre, const dev::V3<F>& pos, F dmin, F vel, int32_t sign,
+                                           uint32_t nscat, WalkOf<F, kDefer>& W) {
+    const F sg = F(sign);
+    const F dt = sg * dev::Real<F>::div(dmin, vel);
+    const F dx = sg * (pos.x - pre.x);
+    const F dy = sg * (pos.y - pre.y);
+    const F dz = sg * (pos.z - pre.z);
+    const int tk = K.tally;
+    const bool with_t = tk == MCG_TEMP || tk == MCG_MULTI || tk == MCG_CUMTEMP;
+    const F amt[kMaxRows] = {with_t ? dt : dx, with_t ? dx : dy, with_t ? dy : dz, dz};
+    const int nv = tk == MCG_MULTI ? 4 : (with_t ? 1 : 3);
+    int r0 = 0;
+    if (tk >= MCG_CUMTEMP) {
+        const int bin = int((int64_t(nscat) + K.step_cum - 1) / K.step_cum);
+        r0 = tk == MCG_CUMTEMP ? bin : 3 * bin;
     }
+    return accumulate<F, kDefer>(S, sink, pre, pos, r0, nv, amt, W);
+}
+
+// The flight half of a scatter-step: advect_step and the tally.  `walking` is
+// set when the flight's 2-D / 3-D tally walk was deferred to W; apos receives
+// the position after the flight.
+template <typename F, int kDefer>
+__device__ __forceinline__ int flight_step(const KParams<F>& K, const View<F>& V, const Sink& sink,
+                                           Lane<F>& L, WalkOf<F, kDefer>& W, bool& walking, uint32_t& fate,
+                                           F& dmin_out, dev::V3<F>& apos, int32_t& pbeg_out,
+                                           int32_t& pore_out) {
+    walking = false;
+    const F vel = V.vel[L.mode];
+    const DevSdom<F>& S = V.sdoms[L.sdom];
+    dev::V3<F> pre;
+    const int hit = advect_step<F>(V, L, fate, dmin_out, pre, pbeg_out, pore_out);
+    apos = L.pos;
+    if (fate == 0xFFFFFFFFu)
+        walking = tally_step<F, kDefer>(K, S, sink, pre, L.pos, dmin_out, vel, L.sign, L.nscat, W);
     return hit;
 }
 
@@ -1214,18 +1245,7 @@ __device__ __forceinline__ void collide_step(const KParams<F>& K, const View<F>&
                         break;
                     }
                     default: {       // MCG_INTER, boundary.cpp:349-359
-                        int target = -1;
-                        if (P.icnt == 1) {
-                            target = P.target;
-                        } else {
-                            for (int q = 0; q < P.icnt; ++q) {
-                                const int cand = K.inter_list[P.ibeg + q];
-                                if (inside(V.planes, V.sdoms[cand], V.pores, L.pos)) {
-                                    target = cand;
-                                    break;
-                                }
-                            }
-                        }
+                        const int target = inter_target<F>(K, V, P, L.pos);
                         if (target < 0) fate = MCG_ESCAPED;
                         else L.sdom = target;
                         break;
@@ -1368,6 +1388,7 @@ __device__ __forceinline__ int64_t claim(bool need, int lane, uint64_t lt_mask, 
 }
 
 #include "mcg_box.h"
+#include "mcg_drain.h"
 
 // Single solve: persistent grid, every lane refilled from the solve's global
 // bundle counter until the range [first, first + count) is exhausted.
@@ -1428,9 +1449,16 @@ __global__ void __launch_bounds__(1024) trajectory_kernel(KParams<F> K) {
                 }
             }
             if (__ballot(active || walking || full || !drained) == 0ull) break;
+            if (__builtin_expect_with_probability(__ballot(drained) != 0ull, 0, kDrainRare) && __ballot(full) == 0ull &&
+                popc(__ballot(active)) <= kDrainLanes && K.trace_id < 0) {
+                if constexpr (kDefer != 0)
+                    while (__ballot(walking) != 0ull) walk_some<kWalkUnroll>(W, walking, sink);
+                general_drain<F, kDefer>(K, V, sink, lane, lt_mask, L, active, st);
+                break;
+            }
             if (active && !walking) {
                 const uint32_t fate = scatter_step<F, kDefer>(K, V, sink, L, W, walking);
-                if (fate != 0xFFFFFFFFu) {
+                if (fate != kAlive) {
                     st.add(fate, L.nstep);
                     active = false;
                 }
@@ -1453,9 +1481,15 @@ __global__ void __launch_bounds__(1024) trajectory_kernel(KParams<F> K) {
                 }
             }
             if (__ballot(active || walking) == 0ull) break;
+            if (__ballot(finished) != 0ull && popc(__ballot(active)) <= kDrainLanes && K.trace_id < 0) {
+                if constexpr (kDefer != 0)
+                    while (__ballot(walking) != 0ull) walk_some<kWalkUnroll>(W, walking, sink);
+                general_drain<F, kDefer>(K, V, sink, lane, lt_mask, L, active, st);
+                break;
+            }
             if (active && !walking) {
                 const uint32_t fate = scatter_step<F, kDefer>(K, V, sink, L, W, walking);
-                if (fate != 0xFFFFFFFFu) {
+                if (fate != kAlive) {
                     st.add(fate, L.nstep);
                     active = false;
                 }
