@@ -2405,12 +2405,25 @@ int launch_box(mcg_scene* sc, const HostProblem& p, KParams<F>& K, BoxCell<F>& c
                hipStream_t stream) {
     HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
     int per_cu = std::max<int>(1, int(sc->lds_limit / lds));
-    const int block = sc->tune.block > 0 ? sc->tune.block : (per_cu == 1 ? 1024 : 512);
+    int block = sc->tune.block > 0 ? sc->tune.block : (per_cu == 1 ? 1024 : 512);
     per_cu = std::min(per_cu, std::max(1, 2048 / block));
     if (sc->tune.blocks_per_cu > 0) per_cu = std::min(per_cu, int(sc->tune.blocks_per_cu));
     // each part of the tally takes the same share of the workgroups
-    const int64_t needed = (p.count + block - 1) / block;
     const int64_t share = std::max<int64_t>(1, int64_t(sc->num_cu) * per_cu / cell.parts);
+    if (sc->tune.block <= 0) {
+        // A small solve takes smaller workgroups on all CUs rather than a few
+        // full ones: enough lanes for kPerLane bundles each, so that lanes
+        // refill while the longest bundles run and fewer wavefronts share a
+        // SIMD in the drain (FP64, whose steps are long and whose lanes hold
+        // no bundle in reserve, gains more).  Default against this: slab 1e5
+        // FP64 273 -> 242 us, bar 3e5 FP64 1393 -> 1326 us, 1e6 FP64 1945 ->
+        // 1808 us, bar 3e4 FP32 649 -> 627 us, porous film 2e4 FP32 2259 ->
+        // 1270 us; bar 1e6 FP32 keeps 512 threads (1222 us; 384: 1337).
+        constexpr int64_t kPerLane = sizeof(F) == 8 ? 6 : 2;
+        const int64_t lanes = (p.count + kPerLane * share - 1) / (kPerLane * share);
+        block = int(std::min<int64_t>(block, std::max<int64_t>(128, (lanes + 63) / 64 * 64)));
+    }
+    const int64_t needed = (p.count + block - 1) / block;
     const int grid = int(std::max<int64_t>(1, std::min(share, needed)));
     K.tail = int64_t(MCG_TAIL_LANES) * grid * block;
     void* args[] = {&K, &cell};
