@@ -131,9 +131,13 @@ struct BoxWalk {
     F prev;
     double amt[kMaxRows];
 };
+// Without a grid: the share of the last flight in its last cell, kept back (the
+// next flight of the bundle starts in that cell) until the lane leaves it.
 template <typename F>
 struct BoxWalk<F, 0> {
-    int32_t left;
+    int32_t left;            // no walk: always 0
+    int32_t cell;            // the cell, -1 for none
+    double held[kMaxRows];
 };
 
 template <typename F>
@@ -304,9 +308,21 @@ __device__ __forceinline__ void add_row(const Span<F>& s, F amt, F ca) {
     }
 }
 
+// Adds what a lane holds back of its last cell.
+template <int kRows, typename F>
+__device__ __forceinline__ void box_release(BoxWalk<F, 0>& W, const BoxCell<F>& B, double* tally) {
+    if (W.cell >= 0) {
+#pragma unroll
+        for (int j = 0; j < kMaxRows; ++j)
+            if (kRows == kMaxRows || B.rowmask >> j & 1) unsafeAtomicAdd(tally + W.cell + j * kBoxCols, W.held[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < kMaxRows; ++j) W.held[j] = 0.0;
+}
+
 // The tally of a flight pre -> L.pos of length dmin: added at once along one
 // axis, set up in W for a grid.
-template <typename F, int kAxes, int kRows>
+template <typename F, int kAxes, int kRows, bool kHold = false>
 __device__ __forceinline__ void box_tally(const BoxCell<F>& B, const BoxView<F>& V, const BoxLane<F>& L,
                                           const dev::V3<F>& pre, F dmin, BoxWalk<F, kAxes>& W) {
     F dt;
@@ -323,6 +339,54 @@ __device__ __forceinline__ void box_tally(const BoxCell<F>& B, const BoxView<F>&
         const int ee = min(max(int(floor(e)), 0), B.last[0]);
         const bool up = bb < ee;
         const int lo = min(bb, ee) + 1, hi = max(bb, ee);
+        if constexpr (kHold) {
+            // What bounds a 1-D FP32 solve with full wavefronts is the LDS (an
+            // FP64 add of 64 lanes takes 20 cycles; 16 of them a flight, the
+            // LDS active 92 % of the time outside the drain): a flight's last
+            // share waits in registers for the next flight's first, and
+            // flights inside one cell add nothing.  Bar 1e7 4.31 -> 3.90 ms,
+            // 256 slabs 13.0 -> 12.4 ms.  FP64, whose steps are twice as
+            // long, adds at once (bar 1e6 held back: 1.98 -> 1.99 ms).
+            F ca[kMaxRows];
+            const F amt[kMaxRows] = {dt, dx, dy, dz};
+            if constexpr (sizeof(F) == 4) {
+                const F rad = __builtin_amdgcn_rcpf(fabsf(e - b));
+#pragma unroll
+                for (int j = 0; j < kMaxRows; ++j) ca[j] = amt[j] * rad;
+            } else {
+                const Quotient q(fabs(e - b));
+#pragma unroll
+                for (int j = 0; j < kMaxRows; ++j) ca[j] = q(amt[j]);
+            }
+            if (bb != W.cell) {   // another bundle, or moved by a periodic face
+                box_release<kRows>(W, B, V.tally);
+                W.cell = bb;
+            }
+            const bool one = bb == ee;
+            const F fb = up ? F(1 + bb) - b : b - F(bb);
+            const F fe = up ? e - F(ee) : F(1 + ee) - e;
+            double *const first = V.tally + bb, *const beg = V.tally + kMaxRows * kBoxCols + lo,
+                           *const end = V.tally + kMaxRows * kBoxCols + hi;
+#pragma unroll
+            for (int j = 0; j < kMaxRows; ++j) W.held[j] += double(one ? amt[j] : ca[j] * fb);
+            if (!one) {
+#pragma unroll
+                for (int j = 0; j < kMaxRows; ++j)
+                    if (kRows == kMaxRows || B.rowmask >> j & 1) unsafeAtomicAdd(first + j * kBoxCols, W.held[j]);
+#pragma unroll
+                for (int j = 0; j < kMaxRows; ++j) W.held[j] = double(ca[j] * fe);
+                W.cell = ee;
+                if (lo < hi) {
+#pragma unroll
+                    for (int j = 0; j < kMaxRows; ++j)
+                        if (kRows == kMaxRows || B.rowmask >> j & 1) {
+                            unsafeAtomicAdd(beg + j * kBoxCols, double(ca[j]));
+                            unsafeAtomicAdd(end + j * kBoxCols, -double(ca[j]));
+                        }
+                }
+            }
+            return;
+        }
         Span<F> s;
         s.one = bb == ee;
         s.range = lo < hi;
@@ -605,7 +669,7 @@ __device__ __forceinline__ uint32_t box_step(const BoxCell<F>& B, const BoxView<
     const uint32_t hit = box_flight(B, L, pre, dmin, outside);
     uint32_t fate = MCG_ESCAPED;
     if (!outside) {
-        box_tally<F, kAxes, kRows>(B, V, L, pre, dmin, W);
+        box_tally<F, kAxes, kRows, sizeof(F) == 4>(B, V, L, pre, dmin, W);
         fate = box_event<F, kLdsTables, false>(B, V, hit, L, Draws<F>{});
     }
     return fate;
@@ -911,6 +975,10 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
     BoxLane<F> L, N;
     BoxWalk<F, kAxes> W;
     W.left = 0;
+    if constexpr (kAxes == 0) {
+        W.cell = -1;
+        for (int j = 0; j < kMaxRows; ++j) W.held[j] = 0.0;
+    }
     BoxStats st;
     uint64_t busy = ~0ull, last_busy = 0ull;
     for (;;) {
@@ -965,8 +1033,12 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
             last_busy = __ballot(active || walking);
             // no id left (one lane found none) and few bundles: the drain
             if (__ballot(drained) != 0ull && __ballot(full) == 0ull && popc(__ballot(active)) <= kDrainLanes) {
-                if constexpr (kAxes != 0)
+                if constexpr (kAxes != 0) {
                     while (__ballot(W.left > 0) != 0ull) box_walk_some<kWalkUnroll, kRows>(W, B, V.tally);
+                } else if constexpr (sizeof(F) == 4) {
+                    box_release<kRows>(W, B, V.tally);
+                    W.cell = -1;
+                }
                 box_drain<F, kLdsTables, kAxes, kRows>(B, kp, V, lane, lt_mask, L, active, st);
                 break;
             }
@@ -987,6 +1059,7 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
         }
         busy = __ballot(active || W.left > 0);
     }
+    if constexpr (kAxes == 0 && sizeof(F) == 4) box_release<kRows>(W, B, V.tally);
     if (lane == 0 && st.ended != 0 && B.part == 0) {
         unsigned long long* const c = in_global(params_here<F>(kp)->counters);
         atomicAdd(c + C_STEPS, st.steps);
