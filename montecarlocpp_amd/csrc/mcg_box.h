@@ -152,7 +152,10 @@ struct BoxView {
 template <typename F>
 __device__ __forceinline__ dev::V3<F> unit_of(const dev::V3<F>& v) {
     if constexpr (sizeof(F) == 4) {
-        return dev::normalized(v);
+        // the directions normalised here have length one up to rounding, so
+        // normalized()'s test for the zero vector is left out
+        const F s = __builtin_amdgcn_rsqf(v.x * v.x + v.y * v.y + v.z * v.z);
+        return dev::V3<F>{v.x * s, v.y * s, v.z * s};
     } else {
         const F n2 = v.x * v.x + v.y * v.y + v.z * v.z;
         const Quotient q(sqrt(n2));
@@ -168,7 +171,7 @@ __device__ __forceinline__ dev::V3<F> box_wall_normal(const BoxCell<F>& B, const
         const Quotient q(B.r);
         return unit_of(dev::V3<F>{q(p.x - B.cx), q(p.y - B.cy), F(0)});
     } else {
-        return unit_of(dev::V3<F>{p.x - B.cx, p.y - B.cy, F(0)});
+        return dev::normalized(dev::V3<F>{p.x - B.cx, p.y - B.cy, F(0)});
     }
 }
 
@@ -212,6 +215,14 @@ __device__ __forceinline__ void box_pin(BoxCell<F>& B) {
         in_vector(B.last[q]);
     }
 }
+
+// floor(x) as an int (the hardware's one instruction in FP32).
+__device__ __forceinline__ int cell_of(float x) {
+    int i;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(i) : "v"(x));
+    return i;
+}
+__device__ __forceinline__ int cell_of(double x) { return int(floor(x)); }
 
 // The component of v a tally axis runs along: the masks are all ones for it
 // and zero for the others.
@@ -335,11 +346,12 @@ __device__ __forceinline__ void box_tally(const BoxCell<F>& B, const BoxView<F>&
         if (B.tally == 0) return;
         const F b = B.div[0] * (B.inv[0] * (pick3(B.comp[0], pre) - B.o[0]));
         const F e = B.div[0] * (B.inv[0] * (pick3(B.comp[0], L.pos) - B.o[0]));
-        const int bb = min(max(int(floor(b)), 0), B.last[0]);
-        const int ee = min(max(int(floor(e)), 0), B.last[0]);
+        const int bb = min(max(cell_of(b), 0), B.last[0]);
+        const int ee = min(max(cell_of(e), 0), B.last[0]);
         const bool up = bb < ee;
         const int lo = min(bb, ee) + 1, hi = max(bb, ee);
         if constexpr (kHold) {
+            static_assert(sizeof(F) == 4, "FP32 only");
             // What bounds a 1-D FP32 solve with full wavefronts is the LDS (an
             // FP64 add of 64 lanes takes 20 cycles; 16 of them a flight, the
             // LDS active 92 % of the time outside the drain): a flight's last
@@ -347,28 +359,21 @@ __device__ __forceinline__ void box_tally(const BoxCell<F>& B, const BoxView<F>&
             // flights inside one cell add nothing.  Bar 1e7 4.31 -> 3.90 ms,
             // 256 slabs 13.0 -> 12.4 ms.  FP64, whose steps are twice as
             // long, adds at once (bar 1e6 held back: 1.98 -> 1.99 ms).
-            F ca[kMaxRows];
-            const F amt[kMaxRows] = {dt, dx, dy, dz};
-            if constexpr (sizeof(F) == 4) {
-                const F rad = __builtin_amdgcn_rcpf(fabsf(e - b));
-#pragma unroll
-                for (int j = 0; j < kMaxRows; ++j) ca[j] = amt[j] * rad;
-            } else {
-                const Quotient q(fabs(e - b));
-#pragma unroll
-                for (int j = 0; j < kMaxRows; ++j) ca[j] = q(amt[j]);
-            }
+            const bool one = bb == ee;
+            const F fbb = F(bb), fee = F(ee);
+            const F db = (up ? fbb + F(1) : fbb) - b, de = e - (up ? fee : fee + F(1));
+            // a flight inside one cell: its whole amounts to that cell
+            const F rad = one ? F(1) : __builtin_amdgcn_rcpf(fabsf(e - b));
+            const F fb = one ? F(1) : (up ? db : -db), fe = up ? de : -de;
+            const F ca[kMaxRows] = {dt * rad, dx * rad, dy * rad, dz * rad};
             if (bb != W.cell) {   // another bundle, or moved by a periodic face
                 box_release<kRows>(W, B, V.tally);
                 W.cell = bb;
             }
-            const bool one = bb == ee;
-            const F fb = up ? F(1 + bb) - b : b - F(bb);
-            const F fe = up ? e - F(ee) : F(1 + ee) - e;
             double *const first = V.tally + bb, *const beg = V.tally + kMaxRows * kBoxCols + lo,
                            *const end = V.tally + kMaxRows * kBoxCols + hi;
 #pragma unroll
-            for (int j = 0; j < kMaxRows; ++j) W.held[j] += double(one ? amt[j] : ca[j] * fb);
+            for (int j = 0; j < kMaxRows; ++j) W.held[j] += double(ca[j] * fb);
             if (!one) {
 #pragma unroll
                 for (int j = 0; j < kMaxRows; ++j)
@@ -419,8 +424,8 @@ __device__ __forceinline__ void box_tally(const BoxCell<F>& B, const BoxView<F>&
         for (int q = 0; q < kAxes; ++q) {
             const F b = B.div[q] * (B.inv[q] * (pick3(B.comp[q], pre) - B.o[q]));
             const F e = B.div[q] * (B.inv[q] * (pick3(B.comp[q], L.pos) - B.o[q]));
-            const int bk = min(max(int(floor(b)), 0), B.last[q]);
-            const int ek = min(max(int(floor(e)), 0), B.last[q]);
+            const int bk = min(max(cell_of(b), 0), B.last[q]);
+            const int ek = min(max(cell_of(e), 0), B.last[q]);
             const F dc = e - b;
             const bool up = bk < ek;
             idx += bk * B.stride[q];
@@ -471,7 +476,7 @@ __device__ __forceinline__ uint32_t box_flight(const BoxCell<F>& B, BoxLane<F>& 
         if constexpr (sizeof(F) == 4) {
             // a face that rounding left just behind is met where the bundle stands
             const F ta = ((up ? B.hi[a] : B.lo[a]) - p[a]) * __builtin_amdgcn_rcpf(u[a]);
-            const F t = ta < F(0) ? F(0) : ta;
+            const F t = fmaxf(ta, F(0));
             const bool take = (u[a] != F(0)) & (t < dmin);
             dmin = take ? t : dmin;
             hit = take ? code : hit;
@@ -559,10 +564,10 @@ __device__ __forceinline__ Draws<F> box_draws(const BoxCell<F>& B, const BoxView
     D.spec = b1.w;
     if constexpr (sizeof(F) == 4)
         if (B.partial) D.spec = ev.block(1).w;
-    const F r = dev::Real<F>::uniform(b0.x, b1.x) * F(2) + F(-1);
+    const F r = dev::Real<F>::symmetric(b0.x, b1.x);
     const F ar = r < F(0) ? -r : r;
     const F si = dev::Real<F>::sqrt_(F(1) - r * r), sl = dev::Real<F>::sqrt_(ar);
-    const F q = dev::Real<F>::uniform(b0.y, b1.y) * F(2) + F(-1);
+    const F q = dev::Real<F>::symmetric(b0.y, b1.y);
     F sq, cq;
     dev::Real<F>::sincos_pi(q, sq, cq);
     D.iso = dev::V3<F>{si * cq, si * sq, r};
@@ -596,7 +601,7 @@ __device__ __forceinline__ uint32_t box_event(const BoxCell<F>& B, const BoxView
             kind = w < (pore ? B.pore_thr : P.spec_thr) ? uint32_t(MCG_SPEC) : uint32_t(MCG_DIFF);
         }
     }
-    L.nbdry += intr ? 0u : 1u;
+    if (sizeof(F) == 8 || B.counts) L.nbdry += intr ? 0u : 1u;
     dev::V3<F> d = L.dir;
     if (intr | (kind == MCG_DIFF)) {
         // isotropic cos(theta) = r or Lambertian sin^2(theta) = |r| about z,
@@ -609,11 +614,11 @@ __device__ __forceinline__ uint32_t box_event(const BoxCell<F>& B, const BoxView
             vel = ahead.vel;
         } else {
             const uint4 b0 = ev.block(0), b1 = low_block<F>(ev, 1);
-            const F r = dev::Real<F>::uniform(b0.x, b1.x) * F(2) + F(-1);
+            const F r = dev::Real<F>::symmetric(b0.x, b1.x);
             const F ar = r < F(0) ? -r : r;
             const F sinT = dev::Real<F>::sqrt_(intr ? F(1) - r * r : ar);
             const F cosT = intr ? r : dev::Real<F>::sqrt_(F(1) - ar);
-            const F q = dev::Real<F>::uniform(b0.y, b1.y) * F(2) + F(-1);
+            const F q = dev::Real<F>::symmetric(b0.y, b1.y);
             F sq, cq;
             dev::Real<F>::sincos_pi(q, sq, cq);
             d = dev::V3<F>{sinT * cq, sinT * sq, cosT};

@@ -73,6 +73,9 @@ struct Real<double> {
     __device__ static __forceinline__ double uniform(uint32_t a, uint32_t b) {
         return (double(a >> 5) * 67108864.0 + double(b >> 6)) * (1.0 / 9007199254740992.0);
     }
+    __device__ static __forceinline__ double symmetric(uint32_t a, uint32_t b) {   // 2 u - 1
+        return uniform(a, b) * 2.0 + -1.0;
+    }
     __device__ static __forceinline__ double sqrt_(double x) { return sqrt(x); }
     // sin(pi r), cos(pi r) and log from the portable header, bit-identical
     // to the CPU checker's evaluation
@@ -94,6 +97,10 @@ struct Real<float> {
     // leading bits, so both precisions take the same decisions)
     __device__ static __forceinline__ float uniform(uint32_t a, uint32_t) {
         return float(a >> 8) * 5.9604644775390625e-8f;
+    }
+    // 2 u - 1 (the scaling is exact, so the fused form rounds as the separate one)
+    __device__ static __forceinline__ float symmetric(uint32_t a, uint32_t) {
+        return __builtin_fmaf(float(a >> 8), 1.1920928955078125e-7f, -1.0f);
     }
     // FP32 flight is compared statistically, so it uses the hardware's
     // one-instruction approximations: v_sqrt_f32, v_rcp_f32 (1 ulp) and
