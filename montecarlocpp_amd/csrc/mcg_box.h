@@ -47,6 +47,24 @@ enum : uint32_t { kCodeIntrinsic = 24, kCodePore = 28 };
 // 20 / 28 / 36 / 44: 9.6 / 9.8 / 10.2 / 11.3 ms.
 constexpr int kBoxWalkQuorum4 = 36;
 
+// Threads of a box kernel's workgroup at most (kThreads).  The FP64 kernels of
+// grids hold a walk besides a bundle (and the drain its draws and a flight): two
+// wavefronts a SIMD with 256 registers each run them without spills, four with
+// 128 spill 50 to 100.  A lone bundle's step takes 1.21 us with two and 1.52 us
+// with four (12 x 6 film), so solves whose longest bundles bound them take two:
+// up to kNarrowPerLane bundles a lane of four (a batch, whose solves end
+// together, kNarrowBatch).  Film 1e5 8.1 -> 5.6 ms, 1e6 28.2
+// -> 22.9 ms, its 3-D grid 1e6 36.9 -> 25.0 ms, porous film 1e5 8.2 -> 7.2 ms,
+// 1e6 20.0 -> 18.6 ms, 16 porous films of 3e3 in a batch 14.2 -> 10.5 ms; beyond,
+// four hide each other's waits better: porous film 4e6 56 ms (two: 62), 1e7 127
+// ms (147), 16 of 5e4 in a batch 18.3 ms (19.2).  1-D tallies keep four
+// throughout (bar 1e7 FP64: 7.5 ms, two 8.5).
+constexpr int kNarrowThreads = 512, kNarrowPerLane = 5, kNarrowBatch = 1;
+template <typename F>
+bool box_narrow(int axes, double bundles, int cus, int per_lane) {
+    return sizeof(F) == 8 && axes != 0 && bundles <= per_lane * 1024.0 * cus;
+}
+
 
 // LDS row stride of a 1-D tally and of its difference array, in doubles: a
 // compile-time stride puts the rows of one column at immediate offsets of one
@@ -1110,8 +1128,8 @@ __host__ __device__ inline void box_part(BoxCell<F>& B, uint32_t w) {
 
 // A solve of a one-box scene (the kernel parameters come first: params_here
 // reads them through the kernel-argument segment).
-template <typename F, bool kLdsTables, int kAxes, int kRows>
-__global__ void __launch_bounds__(1024) box_kernel(KParams<F> Karg, BoxCell<F> Barg) {
+template <typename F, bool kLdsTables, int kAxes, int kRows, int kThreads = 1024>
+__global__ void __launch_bounds__(kThreads) box_kernel(KParams<F> Karg, BoxCell<F> Barg) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int tid = threadIdx.x;
     const ParamPtr<F> kp = (ParamPtr<F>)__builtin_amdgcn_kernarg_segment_ptr();
@@ -1195,8 +1213,8 @@ __device__ int box_pick(const BoxSolve<F>* solves, int n, unsigned char* lds, in
 }
 
 // kAxes: axes of the grids among the solves (0 when all tallies are 1-D).
-template <typename F, int kAxes>
-__global__ void __launch_bounds__(1024) box_batch_kernel(const BoxSolve<F>* solves, int n) {
+template <typename F, int kAxes, int kThreads = 1024>
+__global__ void __launch_bounds__(kThreads) box_batch_kernel(const BoxSolve<F>* solves, int n) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int tid = threadIdx.x, nthreads = blockDim.x;
     // the solve this workgroup's share of the work starts in: the last one

@@ -2314,21 +2314,26 @@ bool box_cell(const HostScene& h, const HostProblem& p, BoxCell<F>& B) {
 // Multi rows, one, or any) and of tables staged in LDS or read from global
 // memory.
 template <typename F, int kAxes, int kRows>
-const void* pick_box_kernel(bool tables) {
+const void* pick_box_kernel(bool tables, bool narrow) {
+    if constexpr (sizeof(F) == 8 && kAxes != 0)
+        if (narrow)
+            return tables ? reinterpret_cast<const void*>(box_kernel<F, true, kAxes, kRows, kNarrowThreads>)
+                          : reinterpret_cast<const void*>(box_kernel<F, false, kAxes, kRows, kNarrowThreads>);
     return tables ? reinterpret_cast<const void*>(box_kernel<F, true, kAxes, kRows>)
                   : reinterpret_cast<const void*>(box_kernel<F, false, kAxes, kRows>);
 }
 template <typename F, int kAxes>
-const void* pick_box_kernel(bool tables, int rows) {
-    if (rows == kMaxRows) return pick_box_kernel<F, kAxes, kMaxRows>(tables);
+const void* pick_box_kernel(bool tables, int rows, bool narrow) {
+    if (rows == kMaxRows) return pick_box_kernel<F, kAxes, kMaxRows>(tables, narrow);
     if constexpr (kAxes != 0)
-        if (rows == 1) return pick_box_kernel<F, kAxes, 1>(tables);
-    return pick_box_kernel<F, kAxes, 0>(tables);
+        if (rows == 1) return pick_box_kernel<F, kAxes, 1>(tables, narrow);
+    return pick_box_kernel<F, kAxes, 0>(tables, narrow);
 }
 template <typename F>
-const void* pick_box_kernel(bool tables, int rows, int axes) {
-    return axes == 0 ? pick_box_kernel<F, 0>(tables, rows == 1 ? 0 : rows)
-                     : (axes == 2 ? pick_box_kernel<F, 2>(tables, rows) : pick_box_kernel<F, 3>(tables, rows));
+const void* pick_box_kernel(bool tables, int rows, int axes, bool narrow) {
+    return axes == 0 ? pick_box_kernel<F, 0>(tables, rows == 1 ? 0 : rows, false)
+                     : (axes == 2 ? pick_box_kernel<F, 2>(tables, rows, narrow)
+                                  : pick_box_kernel<F, 3>(tables, rows, narrow));
 }
 
 // Parts a map may be split into.  Past this the repeated steps cost more than
@@ -2401,12 +2406,13 @@ constexpr int kTallyCopies = 8;
 
 // Launch of a one-box solve.
 template <typename F>
-int launch_box(mcg_scene* sc, const HostProblem& p, KParams<F>& K, BoxCell<F>& cell, const void* fn, size_t lds,
-               hipStream_t stream) {
+int launch_box(mcg_scene* sc, const HostProblem& p, KParams<F>& K, BoxCell<F>& cell, const void* fn, bool narrow,
+               size_t lds, hipStream_t stream) {
     HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
     int per_cu = std::max<int>(1, int(sc->lds_limit / lds));
-    int block = sc->tune.block > 0 ? sc->tune.block : (per_cu == 1 ? 1024 : 512);
-    per_cu = std::min(per_cu, std::max(1, 2048 / block));
+    const int most = narrow ? kNarrowThreads : 1024;
+    int block = std::min(most, sc->tune.block > 0 ? sc->tune.block : (per_cu == 1 ? 1024 : 512));
+    per_cu = std::min(per_cu, std::max(1, (narrow ? kNarrowThreads : 2048) / block));
     if (sc->tune.blocks_per_cu > 0) per_cu = std::min(per_cu, int(sc->tune.blocks_per_cu));
     // each part of the tally takes the same share of the workgroups
     const int64_t share = std::max<int64_t>(1, int64_t(sc->num_cu) * per_cu / cell.parts);
@@ -2446,7 +2452,9 @@ int launch_solve(mcg_scene* sc, const HostProblem& p, KParams<F>& K, hipStream_t
         box_lds_plan<F>(cell, K.part_next != nullptr, sc->tune.lds_tables >= 0, sc->lds_limit, box_tables, box_lds)) {
         cell.counts = K.c_nscat != nullptr;
         const int axes = cell.tally == 2 ? (h.grid_2d ? 2 : 3) : 0;
-        return launch_box<F>(sc, p, K, cell, pick_box_kernel<F>(box_tables, cell.rows, axes), box_lds, stream);
+        const bool narrow = box_narrow<F>(axes, double(p.count) * cell.parts, sc->num_cu, kNarrowPerLane);
+        return launch_box<F>(sc, p, K, cell, pick_box_kernel<F>(box_tables, cell.rows, axes, narrow), narrow, box_lds,
+                             stream);
     }
     const size_t geo = lds_bytes<F>(h, rows, false, false);
     const LdsPlan lp = plan_lds(geo, lds_bytes<F>(h, rows, true, false) - geo,
@@ -3068,6 +3076,7 @@ struct BatchWork {
     std::vector<int> box_of;             // the entry's solve
     size_t box_lds = 0;
     int box_block = 0, box_grid = 0, box_axes = 0, box_chunk = kChunk;
+    bool box_slim = false;               // the kernel with kNarrowThreads
     size_t words = 0;                    // claim counters of parts and visitor counts (8-byte words, cleared per launch)
 
     // Splits the solves and plans both launches.
@@ -3137,7 +3146,11 @@ struct BatchWork {
             box_block = tune && tune->block ? tune->block : (per_cu == 1 ? 1024 : 512);
             if (box_block < 64 || box_block > 1024 || box_block % 64 != 0)
                 return set_error(MCG_EINVAL, "block must be a multiple of 64 from 64 to 1024");
-            per_cu = std::min(per_cu, std::max(1, 2048 / box_block));
+            double bundles = 0.0;
+            for (int i : box_of) bundles += double(P[i].count);
+            box_slim = box_narrow<F>(box_axes, bundles, sc[0]->num_cu, kNarrowBatch);
+            if (box_slim) box_block = std::min(box_block, kNarrowThreads);
+            per_cu = std::min(per_cu, std::max(1, (box_slim ? kNarrowThreads : 2048) / box_block));
             if (tune && tune->blocks_per_cu > 0) per_cu = std::min(per_cu, int(tune->blocks_per_cu));
             box_grid = sc[0]->num_cu * per_cu;
             box_chunk = tune && tune->chunk > 0 ? tune->chunk : kChunk;
@@ -3213,6 +3226,10 @@ struct BatchWork {
         return MCG_OK;
     }
     const void* box_kernel_fn() const {
+        if constexpr (sizeof(F) == 8)
+            if (box_slim)
+                return box_axes == 2 ? reinterpret_cast<const void*>(box_batch_kernel<F, 2, kNarrowThreads>)
+                                     : reinterpret_cast<const void*>(box_batch_kernel<F, 3, kNarrowThreads>);
         return box_axes == 0 ? reinterpret_cast<const void*>(box_batch_kernel<F, 0>)
                              : (box_axes == 2 ? reinterpret_cast<const void*>(box_batch_kernel<F, 2>)
                                               : reinterpret_cast<const void*>(box_batch_kernel<F, 3>));

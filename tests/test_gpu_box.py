@@ -149,3 +149,26 @@ def test_batch_of_one_tiny_solve():
         fb, sb = engine.batch_solve([sc], [prob])
     assert sa["steps"] == sb[0]["steps"]
     close(fb[0], fa, 1e-9)
+
+
+@pytest.mark.parametrize("block", [0, 64, 1024])
+@pytest.mark.parametrize("name,n", [("grid_3d", 5003), ("parts_rows", 5003), ("grid_2x2", 1 << 21)])
+def test_fp64_grid_launch_shapes(name, n, block):
+    """FP64 grids, single and in a batch: a small solve's kernel of at most 512
+    threads (launched with those where the tuning says more) and, at the last
+    size, a large solve's of up to 1024, against the event engine: counts
+    exactly, tallies to 1e-9 (other summation orders)."""
+    dom, tally = CASES[name]
+    mat, dom = materials.si_like(300.0), dom()
+    prob = scenes.problem(n, tally=tally, maxscat=20, seed=14, precision=abi.FP64)
+    with engine.Scene(mat, dom) as sc:
+        sc.set_tune(abi.Tune(engine=abi.ENGINE_EVENT))
+        fa, sa, ca = solved(sc, prob)
+        sc.set_tune(abi.Tune(block=block))
+        fb, sb, cb = solved(sc, prob)
+        fc, stats = engine.batch_solve([sc], [prob], tune=abi.Tune(block=block))
+    for k in COUNTS:
+        np.testing.assert_array_equal(cb[k], ca[k], err_msg=k)
+    assert sb["steps"] == sa["steps"] == stats[0]["steps"]
+    close(fb, fa, 1e-9)
+    close(fc[0], fa, 1e-9)
