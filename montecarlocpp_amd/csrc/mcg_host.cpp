@@ -514,7 +514,7 @@ int build_domain(const mcg_domain_spec* spec, HostScene& s) {
             s.grid_cells = std::max<int64_t>(s.grid_cells, int64_t(std::min(cells, 1e18)));
             int g = 0;
             for (int k = 0; k < 3; ++k)
-                if (div[k] > 0 && g < 2) d.gax[g++] = k;
+                if (div[k] > 0 && g < 2) d.gax |= k << (2 * g++);
         }
         for (int k = 0; k < 3; ++k) {
             if (shapes[si][k] > (1ll << 30)) return set_error(MCG_ERANGE, "too many tally divisions");
@@ -556,7 +556,6 @@ int build_domain(const mcg_domain_spec* spec, HostScene& s) {
             rotation_to(n, P.rot);
             reflection(n, P.refl);
             P.kind = fs.kind;
-            P.sdom = si;
             P.target = si;
             P.ibeg = P.icnt = 0;
             if (fs.kind == MCG_PARTIAL) {
@@ -646,16 +645,16 @@ int build_domain(const mcg_domain_spec* spec, HostScene& s) {
                 a.pt[i] = t[i];
                 b.pt[i] = tb[i];
             }
-            a.target = b.sdom;
-            b.target = a.sdom;
+            a.target = ps.sdom_b;
+            b.target = ps.sdom_a;
             peri_pair[ia] = ib;
             peri_pair[ib] = ia;
         } else if (a.kind == MCG_INTER && b.kind == MCG_INTER) {
             if (!approx_vec(na, times(-1.0, nb)))
                 return set_error(MCG_EINVAL, "Boundary normals not antiparallel");
             if (!approx_scalar(a.c, -b.c)) return set_error(MCG_EINVAL, "Boundaries planes not the same");
-            inter_pairs[ia].push_back(b.sdom);
-            inter_pairs[ib].push_back(a.sdom);
+            inter_pairs[ia].push_back(ps.sdom_b);
+            inter_pairs[ib].push_back(ps.sdom_a);
         } else {
             return set_error(MCG_EINVAL, "pair joins faces that are not both Peri or both Inter");
         }

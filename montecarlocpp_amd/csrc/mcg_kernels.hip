@@ -184,12 +184,34 @@ __device__ __forceinline__ bool outside_pore(const DevPore<F>& Q, const dev::V3<
     return !(dx * dx + dy * dy < rr * rr);
 }
 
+// Whether p is in the cell, to its tolerance.  FP32 (Inter faces with several
+// partners) evaluates a cell's first kMaxFaces faces together, one LDS round
+// trip, rather than one behind the other's branch; a slot past its last face
+// repeats the first.  Octet truss, 1e6 bundles 4.40 -> 4.22 ms.  FP64, whose
+// flight tests it too, leaves at the first face missed: without that it spills
+// (octet FP64 1e6 9.6 -> 12.3 ms).
 template <typename F>
 __device__ __forceinline__ bool inside(const DevPlane<F>* planes, const DevSdom<F>& S,
                                        const DevPore<F>* pores, const dev::V3<F>& p) {
-    for (int b = S.pbeg; b < S.pend; ++b) {
-        const DevPlane<F>& P = planes[b];
-        if (dev::dot3(P.n, p) + P.c < -S.eps) return false;
+    if constexpr (sizeof(F) == 4) {
+        const int pbeg = S.pbeg, pend = S.pend;
+        const F lost = -S.eps;
+        bool out = false;
+#pragma unroll
+        for (int i = 0; i < kMaxFaces; ++i) {
+            const DevPlane<F>& P = planes[pbeg + i < pend ? pbeg + i : pbeg];
+            out |= dev::dot3(P.n, p) + P.c < lost;
+        }
+        for (int b = pbeg + kMaxFaces; b < pend; ++b) {
+            const DevPlane<F>& P = planes[b];
+            out |= dev::dot3(P.n, p) + P.c < lost;
+        }
+        if (out) return false;
+    } else {
+        for (int b = S.pbeg; b < S.pend; ++b) {
+            const DevPlane<F>& P = planes[b];
+            if (dev::dot3(P.n, p) + P.c < -S.eps) return false;
+        }
     }
     return S.pore < 0 || outside_pore(pores[S.pore], p);
 }
@@ -558,7 +580,7 @@ __device__ __forceinline__ bool accumulate(const DevSdom<F>& S, const Sink& sink
         for (int k = 0; k < 3; ++k) col += bi[k] * S.stride[k];
 #pragma unroll
         for (int q = 0; q < kDefer; ++q) {
-            const int k = kDefer == 3 ? q : S.gax[q];
+            const int k = kDefer == 3 ? q : (S.gax >> (2 * q)) & 3;
             const F b0 = k == 0 ? bc[0] : (k == 1 ? bc[1] : bc[2]);
             const F e0 = k == 0 ? ec[0] : (k == 1 ? ec[1] : ec[2]);
             const int bk = k == 0 ? bi[0] : (k == 1 ? bi[1] : bi[2]);
@@ -2035,7 +2057,7 @@ void convert_plane(const DevPlane<double>& s, DevPlane<F>& d) {
     for (int i = 0; i < 3; ++i) { d.n[i] = F(s.n[i]); d.pt[i] = F(s.pt[i]); }
     d.c = F(s.c);
     for (int i = 0; i < 9; ++i) { d.rot[i] = F(s.rot[i]); d.refl[i] = F(s.refl[i]); d.prot[i] = F(s.prot[i]); }
-    d.kind = s.kind; d.sdom = s.sdom; d.target = s.target; d.ibeg = s.ibeg; d.icnt = s.icnt; d.spec_thr = s.spec_thr;
+    d.kind = s.kind; d.target = s.target; d.ibeg = s.ibeg; d.icnt = s.icnt; d.spec_thr = s.spec_thr;
 }
 
 template <typename F>
@@ -2045,8 +2067,7 @@ void convert_sdom(const DevSdom<double>& s, DevSdom<F>& d, double eps_scale) {
     d.eps = F(s.eps * eps_scale);
     d.accum = s.accum; d.pbeg = s.pbeg; d.pend = s.pend; d.col_off = s.col_off; d.pore = s.pore;
     d.box = s.box;
-    d.gax[0] = s.gax[0];
-    d.gax[1] = s.gax[1];
+    d.gax = s.gax;
     for (int i = 0; i < 3; ++i) {
         d.bmin[i] = F(s.box ? s.bmin[i] : 0.0);
         d.bmax[i] = F(s.box ? s.bmax[i] : 0.0);
@@ -2269,8 +2290,8 @@ bool box_cell(const HostScene& h, const HostProblem& p, BoxCell<F>& B) {
     if (S.accum == -1) axes[na++] = 0;
     else if (S.accum >= 0 && S.accum < 3) axes[na++] = S.accum;
     else if (S.accum == 3) {
-        axes[na++] = S.gax[0];
-        axes[na++] = S.gax[1];
+        axes[na++] = S.gax & 3;
+        axes[na++] = S.gax >> 2;
     } else if (S.accum == 4) {
         for (int k = 0; k < 3; ++k) axes[na++] = k;
     }

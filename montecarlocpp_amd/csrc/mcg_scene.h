@@ -39,6 +39,11 @@ enum ShapeKind : int32_t { SHAPE_PAR = 0, SHAPE_TRI = 1, SHAPE_POLY = 2 };
 // Triangles of a polygon face's fan, or pieces of a prism / pyramid's volume
 constexpr int kMaxPieces = MCG_MAX_SIDES - 2;
 
+// A float DevPlane is 39 words and a float DevSdom 47: odd strides, so that lanes
+// in different cells read different LDS banks (at 40 and 48 the records started
+// in 8 and 4 of the 64 banks, and half of the octet truss's LDS cycles were bank
+// conflicts: 1e6 bundles 4.46 -> 4.40 ms).  The double ones are 37 and 38
+// 8-byte words.
 template <typename F>
 struct DevPlane {
     F n[3];
@@ -48,7 +53,6 @@ struct DevPlane {
     F prot[9];        // periodic map rotation (column-major)
     F pt[3];          // periodic map translation
     int32_t kind;     // mcg_bdry_kind
-    int32_t sdom;     // owning subdomain
     int32_t target;   // Peri: subdomain of the paired face; Inter with one partner: that partner
     int32_t ibeg;     // Inter: first candidate in the pair list
     int32_t icnt;     // Inter: number of candidates
@@ -68,11 +72,12 @@ struct DevSdom {
     int32_t stride[3];
     int32_t pore;     // index of the cylindrical pore or -1
     int32_t box;      // 1: six axis-aligned faces (the FP32 flight's box advect)
-    int32_t gax[2];   // 2-D grid (accum 3): its two divided axes
+    int32_t gax;      // 2-D grid (accum 3): its two divided axes, first | second << 2
     F bmin[3], bmax[3];        // box: the faces' positions on each axis
     F kmin[3], kmax[3];        // box: positions beyond which a bundle is lost (eps outside)
     int32_t fmin[3], fmax[3];  // box: plane offsets (from pbeg) of the low / high face
 };
+static_assert(sizeof(DevPlane<float>) == 4 * 39 && sizeof(DevSdom<float>) == 4 * 47, "odd strides");
 
 template <typename F>
 struct DevEmitter {
