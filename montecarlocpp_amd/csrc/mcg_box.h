@@ -53,12 +53,12 @@ constexpr int kBoxWalkQuorum4 = 36;
 // 128 spill 50 to 100.  A lone bundle's step takes 1.21 us with two and 1.52 us
 // with four (12 x 6 film), so solves whose longest bundles bound them take two:
 // up to kNarrowPerLane bundles a lane of four (a batch, whose solves end
-// together, kNarrowBatch).  Film 1e5 8.1 -> 5.6 ms, 1e6 28.2
-// -> 22.9 ms, its 3-D grid 1e6 36.9 -> 25.0 ms, porous film 1e5 8.2 -> 7.2 ms,
-// 1e6 20.0 -> 18.6 ms, 16 porous films of 3e3 in a batch 14.2 -> 10.5 ms; beyond,
-// four hide each other's waits better: porous film 4e6 56 ms (two: 62), 1e7 127
-// ms (147), 16 of 5e4 in a batch 18.3 ms (19.2).  1-D tallies keep four
-// throughout (bar 1e7 FP64: 7.5 ms, two 8.5).
+// together, kNarrowBatch).  Film 1e4 1.82 -> 1.26 ms, 1e5 4.3 -> 3.1 ms, 1e6 25.2
+// -> 21.5 ms, porous film 1e5 3.04 -> 2.76 ms (1e6 the other way, 15.4 -> 16.9
+// ms), 16 porous films of 3e3 in a batch 14.2 -> 10.4 ms; beyond, four hide
+// each other's waits better: porous film 4e6 56 ms (two: 62), 1e7 127 ms (147),
+// 16 of 5e4 in a batch 18.3 ms (19.2).  1-D tallies keep four throughout (bar
+// 1e7 FP64: 7.5 ms, two 8.5).
 constexpr int kNarrowThreads = 512, kNarrowPerLane = 5, kNarrowBatch = 1;
 template <typename F>
 bool box_narrow(int axes, double bundles, int cus, int per_lane) {
@@ -1022,7 +1022,7 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
                 if (me != 0ull && (popc(me) >= kSlotQuorum || popc(__ballot(empty && !active && !walking)) >= kEmitQuorum ||
                                    __ballot(active || walking) == 0ull)) {
                     const int64_t mine = claim(empty, lane, lt_mask, pool_base, pool_lim, next, k->chunk, count,
-                                               k->tail, &seen);
+                                               k->guide, k->tail, seen);
                     if (empty) {
                         if (mine < count) {
                             box_emit<F, kLdsTables>(k, B, V, k->first + mine, N);
@@ -1041,7 +1041,8 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
             } else {
                 const bool need = !active && !drained && !walking;
                 if (emit_now<kEmitQuorumFp64>(need, active || walking)) {
-                    const int64_t mine = claim(need, lane, lt_mask, pool_base, pool_lim, next, k->chunk);
+                    const int64_t mine = claim(need, lane, lt_mask, pool_base, pool_lim, next, k->chunk, count,
+                                               k->guide, 0, seen);
                     if (need) {
                         if (mine < count) {
                             box_emit<F, kLdsTables>(k, B, V, k->first + mine, L);

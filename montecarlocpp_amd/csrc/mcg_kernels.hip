@@ -43,7 +43,20 @@ namespace mcg {
 namespace {
 
 constexpr int kWave = 64;
-constexpr int kChunk = 256;            // bundle ids claimed per wavefront grab
+constexpr int kChunk = 256;            // bundle ids claimed per wavefront grab in a batch
+// A single solve's grabs (claim): the ids left over kGuide* times the
+// wavefronts, at most kChunk*.  Where faces absorb, bundles are short and the
+// claim counter bounds a large solve (20 ns a grab, one address): large grabs
+// spare it.  Elsewhere bundles run to the scatter cap, and fine grabs end the
+// wavefronts together.  Against grabs of 256 (in FP32 of 64 near the end):
+// slab FP32 1e7 2.65 -> 1.80 ms, bar 1.25e7 3.78 -> 3.65 ms, slab FP64 1e5 567
+// -> 550 us; octet FP32 1e6 4.23 -> 3.77 ms, tee FP64 1.5e5 33.9 -> 16.9 ms,
+// film FP64 1e4 4.3 -> 1.26 ms, porous film of 128 x 128 8.4 -> 5.9 ms (the
+// launch shapes of small solves below are part of the last four).  With 1 for
+// long bundles octet FP32 1e6 takes 4.9 ms, with 4 for short ones slab FP32
+// 1e6 0.59 instead of 0.48 ms.
+constexpr int kGuideShort = 1, kChunkShort = 1024;
+constexpr int kGuideLong = 4, kChunkLong = 256;
 constexpr int kMaxRows = 4;            // nonzero amount entries per step
 constexpr int kMaxFaces = 6;           // faces an FP32 step keeps in registers (the parallelepiped's)
 constexpr size_t kLdsTallyCap = 48 * 1024;
@@ -134,8 +147,9 @@ struct KParams {
     uint32_t* c_fate;
     int32_t lds_tally;
     int32_t lds_diff;      // the LDS tally holds the range-add difference array (1-D tallies)
-    int32_t chunk;         // bundle ids a wavefront claims at a time
-    int64_t tail;          // FP32 single solve: ids from the end where claims shrink (0: never)
+    int32_t chunk;         // bundle ids a wavefront claims at a time, at most
+    int64_t tail;          // FP32: ids from the end where only idle lanes take a next bundle (0: never)
+    float guide;           // share of the ids left that a wavefront claims at a time
     int64_t trace_id;      // bundle whose steps are recorded, -1 for none
     double* trace;         // MCG_TRACE_WIDTH doubles per step
     int64_t trace_cap;     // records available
@@ -1370,12 +1384,18 @@ __device__ __forceinline__ void walk_phase(WalkN<F, NA>& W, bool& walking, bool 
 }
 
 // Wave-level id pool: lanes whose bundle ended take the next ids of the pool,
-// refilled `chunk` ids at a time from *counter by one lane.  Returns the id
-// offset for lanes with `need` (all lanes call, the pool stays wave-uniform).
+// refilled from *counter by one lane.  In a single solve (guide > 0) a grab
+// takes a share `guide` of the ids left by this wavefront's last grab
+// (`seen`: the counter after it), from one id a lane to `chunk`, so that
+// grabs are few while much is left and the last ids spread over the
+// wavefronts.  In a batch, whose wavefronts come to a solve at any time, it
+// takes `chunk`, and no more than its lanes need (at least one id a lane)
+// within `tail` ids of the end.  Returns the id offset for lanes with `need`
+// (all lanes call, the pool and `seen` stay wave-uniform).
 template <typename Counter>
-__device__ __forceinline__ int64_t claim(bool need, int lane, uint64_t lt_mask, int64_t& base,
-                                         int64_t& lim, Counter* counter, int chunk, int64_t count = 0,
-                                         int64_t tail = 0, int64_t* seen = nullptr) {
+__device__ __forceinline__ int64_t claim(bool need, int lane, uint64_t lt_mask, int64_t& base, int64_t& lim,
+                                         Counter* counter, int chunk, int64_t count, float guide, int64_t tail,
+                                         int64_t& seen) {
     const uint64_t mask = __ballot(need);
     if (!mask) return 0;
     const int cnt = __popcll(mask);
@@ -1386,14 +1406,13 @@ __device__ __forceinline__ int64_t claim(bool need, int lane, uint64_t lt_mask, 
         mine = base + rank;
         base += cnt;
     } else {
-        // within `tail` ids of the end a wavefront takes no more than its
-        // lanes need (at least one id per lane), so the last bundles spread
-        // over the wavefronts instead of waiting in a few private pools
         const int leader = __ffsll((long long)mask) - 1;
         unsigned long long fresh = 0;
         int want = chunk;
+        if (guide > 0.0f)
+            want = max(int(fminf(float(count - seen) * guide, float(chunk))), max(cnt - int(avail), min(chunk, kWave)));
         if (lane == leader) {
-            if (tail > 0) {
+            if (guide <= 0.0f && tail > 0) {
                 const unsigned long long cur = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 if (int64_t(cur) + tail >= count) want = max(cnt - int(avail), min(chunk, kWave));
             }
@@ -1404,7 +1423,7 @@ __device__ __forceinline__ int64_t claim(bool need, int lane, uint64_t lt_mask, 
         mine = rank < avail ? base + rank : int64_t(fresh) + (rank - avail);
         base = int64_t(fresh) + (cnt - avail);
         lim = int64_t(fresh) + want;
-        if (seen) *seen = int64_t(fresh) + want;
+        seen = lim;
     }
     return mine;
 }
@@ -1455,7 +1474,7 @@ __global__ void __launch_bounds__(1024) trajectory_kernel(KParams<F> K) {
                 (__popcll(me) >= kSlotQuorum || __popcll(__ballot(empty && !active && !walking)) >= kEmitQuorum ||
                  __ballot(active || walking) == 0ull)) {
                 const int64_t mine = claim(empty, lane, lt_mask, pool_base, pool_lim, K.next, K.chunk, K.count,
-                                           K.tail, &seen);
+                                           K.guide, sizeof(F) == 4 ? K.tail : 0, seen);
                 if (empty) {
                     if (mine < K.count) {
                         emit<F>(K, K.flux_alias, V.mfp, K.first + mine, N);
@@ -1489,10 +1508,12 @@ __global__ void __launch_bounds__(1024) trajectory_kernel(KParams<F> K) {
         }
     } else {
         bool finished = false;
+        int64_t seen = 0;
         for (;;) {
             const bool need = !active && !finished && !walking;
             if (emit_now<kEmitQuorumFp64>(need, active || walking)) {
-                const int64_t mine = claim(need, lane, lt_mask, pool_base, pool_lim, K.next, K.chunk);
+                const int64_t mine = claim(need, lane, lt_mask, pool_base, pool_lim, K.next, K.chunk, K.count,
+                                           K.guide, sizeof(F) == 4 ? K.tail : 0, seen);
                 if (need) {
                     if (mine < K.count) {
                         emit<F>(K, K.flux_alias, V.mfp, K.first + mine, L);
@@ -1599,7 +1620,7 @@ __global__ void __launch_bounds__(1024) batch_kernel(const KParams<F>* __restric
         const View<F> V = stage<F, kLdsTables, kLdsTally>(K, lds, tid, blockDim.x);
         const Sink sink{V.direct, V.diff, K.cols};
         __syncthreads();
-        int64_t pool_base = 0, pool_lim = 0;
+        int64_t pool_base = 0, pool_lim = 0, seen = 0;
         bool active = false, finished = false, walking = false;
         Lane<F> L;
         WalkOf<F, kDefer> W;
@@ -1607,7 +1628,8 @@ __global__ void __launch_bounds__(1024) batch_kernel(const KParams<F>* __restric
         for (;;) {
             const bool need = !active && !finished && !walking;
             if (emit_now(need, active || walking)) {
-                const int64_t mine = claim(need, lane, lt_mask, pool_base, pool_lim, K.next, K.chunk);
+                const int64_t mine = claim(need, lane, lt_mask, pool_base, pool_lim, K.next, K.chunk, K.count,
+                                           K.guide, sizeof(F) == 4 ? K.tail : 0, seen);
                 if (need) {
                     if (mine < K.count) {
                         emit<F>(K, K.flux_alias, V.mfp, K.first + mine, L);
@@ -2202,6 +2224,8 @@ DevScene<F>& dev_scene(mcg_scene* sc) {
 }
 
 // Scene and problem fields of a solve's kernel parameters (buffers aside).
+bool absorbs(const HostScene& h);
+
 template <typename F>
 void fill_params(mcg_scene* sc, const HostProblem& p, KParams<F>& K) {
     const HostScene& h = sc->host;
@@ -2230,7 +2254,8 @@ void fill_params(mcg_scene* sc, const HostProblem& p, KParams<F>& K) {
     K.k1 = uint32_t(p.seed >> 32);
     K.first = p.first;
     K.count = p.count;
-    K.chunk = sc->tune.chunk > 0 ? sc->tune.chunk : kChunk;
+    K.chunk = sc->tune.chunk > 0 ? sc->tune.chunk : (absorbs(h) ? kChunkShort : kChunkLong);
+    K.guide = 0.0f;   // set with the launch's lanes
     K.lds_diff = h.has_1d ? 1 : 0;
     K.trace_id = -1;
 }
@@ -2425,6 +2450,18 @@ __global__ void fold_copies_kernel(double* a, size_t n, const double* priv, size
 // Private copies of a tally that stays in global memory (one per XCD)
 constexpr int kTallyCopies = 8;
 
+// Whether some face absorbs bundles (otherwise they end at the scatter cap).
+bool absorbs(const HostScene& h) {
+    for (const auto& p : h.planes)
+        if (p.kind == MCG_ISOT) return true;
+    return false;
+}
+
+// Share of the ids left that a grab takes in a single solve on `lanes` lanes.
+float claim_share(const HostScene& h, double lanes) {
+    return float(double(kWave) / ((absorbs(h) ? kGuideShort : kGuideLong) * lanes));
+}
+
 // Launch of a one-box solve.
 template <typename F>
 int launch_box(mcg_scene* sc, const HostProblem& p, KParams<F>& K, BoxCell<F>& cell, const void* fn, bool narrow,
@@ -2445,14 +2482,17 @@ int launch_box(mcg_scene* sc, const HostProblem& p, KParams<F>& K, BoxCell<F>& c
         // no bundle in reserve, gains more).  Default against this: slab 1e5
         // FP64 273 -> 242 us, bar 3e5 FP64 1393 -> 1326 us, 1e6 FP64 1945 ->
         // 1808 us, bar 3e4 FP32 649 -> 627 us, porous film 2e4 FP32 2259 ->
-        // 1270 us; bar 1e6 FP32 keeps 512 threads (1222 us; 384: 1337).
-        constexpr int64_t kPerLane = sizeof(F) == 8 ? 6 : 2;
+        // 1270 us; bar 1e6 FP32 keeps 512 threads (1222 us; 384: 1337).  Where
+        // nothing absorbs, FP64 bundles are long and of one length: one a
+        // lane (porous film 1e5 FP64 3.8 -> 2.7 ms against two, 6.4 with six).
+        const int64_t kPerLane = sizeof(F) == 4 ? 2 : (absorbs(sc->host) ? 6 : 1);
         const int64_t lanes = (p.count + kPerLane * share - 1) / (kPerLane * share);
         block = int(std::min<int64_t>(block, std::max<int64_t>(128, (lanes + 63) / 64 * 64)));
     }
     const int64_t needed = (p.count + block - 1) / block;
     const int grid = int(std::max<int64_t>(1, std::min(share, needed)));
     K.tail = int64_t(MCG_TAIL_LANES) * grid * block;
+    K.guide = claim_share(sc->host, double(grid) * block);
     void* args[] = {&K, &cell};
     HIP_TRY(hipLaunchKernel(fn, dim3(grid * cell.parts), dim3(block), args, lds, stream));
     HIP_TRY(hipGetLastError());
@@ -2491,12 +2531,21 @@ int launch_solve(mcg_scene* sc, const HostProblem& p, KParams<F>& K, hipStream_t
     HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
     int blocks_per_cu = std::max<int>(1, int(sc->lds_limit / std::max<size_t>(lds, 1)));
     // one workgroup per CU (a large LDS tally): give it the CU's 16 waves
-    const int block = sc->tune.block > 0 ? sc->tune.block : (blocks_per_cu == 1 ? 1024 : 512);
+    int block = sc->tune.block > 0 ? sc->tune.block : (blocks_per_cu == 1 ? 1024 : 512);
     blocks_per_cu = std::min(blocks_per_cu, std::max(1, 2048 / block));
     if (sc->tune.blocks_per_cu > 0) blocks_per_cu = std::min(blocks_per_cu, int(sc->tune.blocks_per_cu));
+    if (sc->tune.block <= 0) {
+        // A small solve's bundles, one a lane, spread over all CUs: fewer
+        // wavefronts a SIMD step faster.  Octet 1e5 FP32 1.10 -> 0.88 ms, 1e4
+        // 1.05 -> 0.79 ms; FP64 1e5 6.7 -> 1.7 ms with the finer grabs.
+        const int64_t share = int64_t(sc->num_cu) * blocks_per_cu;
+        const int64_t lanes = (p.count + share - 1) / share;
+        block = int(std::min<int64_t>(block, std::max<int64_t>(128, (lanes + 63) / 64 * 64)));
+    }
     const int64_t needed = (p.count + block - 1) / block;
     const int grid = int(std::max<int64_t>(1, std::min<int64_t>(int64_t(sc->num_cu) * blocks_per_cu, needed)));
     K.tail = int64_t(MCG_TAIL_LANES) * grid * block;
+    K.guide = claim_share(sc->host, double(grid) * block);
     // a tally left in global memory gets a private copy per XCD (a solve
     // that may allocate, whose direct and diff arrays are contiguous),
     // summed into the first after the launch
@@ -3145,9 +3194,7 @@ struct BatchWork {
             }
             // rough cost of a bundle: its steps (an absorber ends it after
             // some; otherwise the scatter cap does) and the cells they cross
-            bool absorbs = false;
-            for (const auto& pl : h.planes) absorbs = absorbs || pl.kind == MCG_ISOT;
-            double cost = absorbs ? 8.0 : 1.5 * double(std::min<int64_t>(p.maxscat, 1000));
+            double cost = absorbs(h) ? 8.0 : 1.5 * double(std::min<int64_t>(p.maxscat, 1000));
             if (c.tally == 2) cost *= 1.0 + double(c.last[0] + c.last[1] + c.last[2]) / 64.0;
             for (int q = 0; q < c.parts; ++q) {
                 BoxSolve<F> e{};
@@ -3197,6 +3244,8 @@ struct BatchWork {
         for (int i : general) {
             kparams.push_back(K[i]);
             kparams.back().chunk = plan.chunk;
+            kparams.back().guide = 0.0f;
+            kparams.back().tail = 0;
             kparams.back().lds_tally = plan.tally ? 1 : 0;
             total += K[i].count;
         }
@@ -3219,6 +3268,7 @@ struct BatchWork {
             // workgroups its share of the work brings
             const double wgs = work > 0.0 ? double(box_grid) * e.work * double(e.K.count) / work : 1.0;
             e.K.tail = int64_t(MCG_TAIL_LANES) * box_block * std::max<int64_t>(1, int64_t(wgs + 0.5));
+            e.K.guide = 0.0f;
             e.B.next = e.B.part == 0 ? e.K.next : ctl++;
             e.visitors = reinterpret_cast<uint32_t*>(ctl++);
         }
