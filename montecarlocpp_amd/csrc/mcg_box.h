@@ -18,10 +18,11 @@
 // the general step spends both on what one box does not need: LDS reads of the
 // cell (28 words) behind every step, address arithmetic per tally row, ~70
 // spilled scalars read back lane by lane, and per-step checks for traces.
-// Measured, general kernel against this one, same box: bar 1e7 bundles FP32
-// 5.68 -> 4.43 ms, 1e6 FP64 4.13 -> 3.17 ms, slab 1e5 FP64 562 -> 347 us, slab
-// 1e4 FP32 185 -> 122 us, porous film 1e7 64 x 64 85.3 -> 71.3 ms, film 1e6
-// (12 x 6 map, bundles of up to 10,000 steps) 26.8 -> 14.5 ms.
+// Measured, general kernel (before it had a drain of its own) against this one
+// with its drain, launch shapes and claims, a whole solve, same box: bar 1e7
+// bundles FP32 5.75 -> 3.73 ms, 1e6 FP64 4.20 -> 1.99 ms, slab 1e5 FP64 725 ->
+// 351 us, slab 1e4 FP32 295 -> 148 us, porous film 1e7 64 x 64 85.5 -> 66.1 ms,
+// film 1e6 (12 x 6 map, bundles of thousands of steps) 21.4 -> 8.0 ms.
 //
 // Results: FP32 flight takes the same rounded operations on every quantity a
 // trajectory depends on as the general step, and FP64 the checker's, so
@@ -55,10 +56,10 @@ constexpr int kBoxWalkQuorum4 = 36;
 // up to kNarrowPerLane bundles a lane of four (a batch, whose solves end
 // together, kNarrowBatch).  Film 1e4 1.82 -> 1.26 ms, 1e5 4.3 -> 3.1 ms, 1e6 25.2
 // -> 21.5 ms, porous film 1e5 3.04 -> 2.76 ms (1e6 the other way, 15.4 -> 16.9
-// ms), 16 porous films of 3e3 in a batch 14.2 -> 10.4 ms; beyond, four hide
-// each other's waits better: porous film 4e6 56 ms (two: 62), 1e7 127 ms (147),
-// 16 of 5e4 in a batch 18.3 ms (19.2).  1-D tallies keep four throughout (bar
-// 1e7 FP64: 7.5 ms, two 8.5).
+// ms), 16 porous films of 3e3 in a batch 14.2 -> 10.4 ms (with grabs of 256);
+// beyond, four hide each other's waits better: porous film 4e6 56 ms (two: 62),
+// 1e7 127 ms (147), 16 of 5e4 in a batch 18.3 ms (19.2).  1-D tallies keep four
+// throughout (bar 1e7 FP64: 7.5 ms, two 8.5).
 constexpr int kNarrowThreads = 512, kNarrowPerLane = 5, kNarrowBatch = 1;
 template <typename F>
 bool box_narrow(int axes, double bundles, int cus, int per_lane) {
@@ -1103,7 +1104,7 @@ __device__ __forceinline__ void box_run(const BoxCell<F>& B, ParamPtr<F> kp, con
 // LDS, 1.1e10 a second for the whole GPU, four per cell a flight crosses, so a
 // 128 x 128 map ran at 2e8 scatter-steps a second; running the bundles once per
 // part and adding in LDS costs parts / (parts running at once) more steps.
-// Porous film, 2e5 bundles, 128 x 128 Multi map (4 parts): 153 -> 9.7 ms.
+// Porous film, 2e5 bundles, 128 x 128 Multi map (4 parts): 153 -> 6.0 ms.
 template <typename F>
 __host__ __device__ inline void box_part(BoxCell<F>& B, uint32_t w) {
     if (B.parts == 1) return;
@@ -1162,7 +1163,7 @@ __global__ void __launch_bounds__(kThreads) box_kernel(KParams<F> Karg, BoxCell<
 // taken, and a visitor leaves only when nothing is unclaimed (a stale read of
 // a counter can only add a visit that finds nothing).
 // Every solve visited in turn by the general step, before, and this: 256 slabs
-// 17.3 -> 13.5 ms a call, 24 mixed solves replayed 19.7 -> 11.7 ms, same box.
+// 17.7 -> 12.1 ms a call, 24 mixed solves replayed 19.9 -> 10.3 ms, same box.
 template <typename F>
 struct BoxSolve {
     KParams<F> K;                  // first: box_run reads it through ParamPtr

@@ -3,10 +3,11 @@
 // One launch runs a whole field solve (FieldProblem::solve, problem.cpp:370-445)
 // for a bundle range.  The kernel is persistent and history-based: every lane
 // owns one live bundle in registers and, as soon as that bundle terminates,
-// takes the next bundle id from its wavefront's pool (refilled 256 ids at a
-// time with one global atomic), so lanes stay busy until the bundle set is
-// exhausted.  Each bundle's random numbers depend only on (seed, bundle id,
-// event index), which makes results independent of scheduling.
+// takes the next bundle id from its wavefront's pool (refilled with one global
+// atomic), so lanes stay busy until the bundle set is exhausted.  Scenes of one
+// axis-aligned box run the kernels of mcg_box.h, others trajectory_kernel.
+// Each bundle's random numbers depend only on (seed, bundle id, event index),
+// which makes results independent of scheduling.
 //
 // Per workgroup, the scatter sampling table and the per-mode velocity and mean
 // free path live in LDS, as do the subdomain planes and, when small enough,
@@ -43,13 +44,12 @@ namespace mcg {
 namespace {
 
 constexpr int kWave = 64;
-constexpr int kChunk = 256;            // bundle ids claimed per wavefront grab in a batch
 // A single solve's grabs (claim): the ids left over kGuide* times the
 // wavefronts, at most kChunk*.  Where faces absorb, bundles are short and the
 // claim counter bounds a large solve (20 ns a grab, one address): large grabs
 // spare it.  Elsewhere bundles run to the scatter cap, and fine grabs end the
 // wavefronts together.  Against grabs of 256 (in FP32 of 64 near the end):
-// slab FP32 1e7 2.65 -> 1.80 ms, bar 1.25e7 3.78 -> 3.65 ms, slab FP64 1e5 567
+// slab FP32 1e7 2.65 -> 1.80 ms, bar 1e7 3.78 -> 3.65 ms, slab FP64 1e5 567
 // -> 550 us; octet FP32 1e6 4.23 -> 3.77 ms, tee FP64 1.5e5 33.9 -> 16.9 ms,
 // film FP64 1e4 4.3 -> 1.26 ms, porous film of 128 x 128 8.4 -> 5.9 ms (the
 // launch shapes of small solves below are part of the last four).  With 1 for
@@ -57,6 +57,10 @@ constexpr int kChunk = 256;            // bundle ids claimed per wavefront grab 
 // 1e6 0.59 instead of 0.48 ms.
 constexpr int kGuideShort = 1, kChunkShort = 1024;
 constexpr int kGuideLong = 4, kChunkLong = 256;
+// A batch's grabs, by the same reasons: against 256 throughout, 24 mixed FP32
+// solves replayed 10.33 -> 9.97 ms, 16 FP64 films of 3e3 bundles 7.85 -> 3.01 ms,
+// 16 FP64 porous films of 3e3 10.5 -> 4.5 ms, of 5e4 18.2 -> 13.9 ms.
+constexpr int kChunk = 256, kChunkBatchLong = 64;
 constexpr int kMaxRows = 4;            // nonzero amount entries per step
 constexpr int kMaxFaces = 6;           // faces an FP32 step keeps in registers (the parallelepiped's)
 constexpr size_t kLdsTallyCap = 48 * 1024;
@@ -3063,7 +3067,7 @@ struct BatchPlan {
     size_t lds = 0;
     bool tables = true, tally = true;
     int walk = 0;              // axes of deferred tally walks (walk_axes)
-    int block = 256, grid = 0, chunk = kChunk;
+    int block = 256, grid = 0;
 };
 
 // LDS layout, block size and grid of a batch launch over these solves.
@@ -3102,7 +3106,6 @@ int plan_shape(int n, mcg_scene* const* scenes, const HostProblem* P, const mcg_
     per_cu = std::min(per_cu, std::max(1, 2048 / B.block));
     if (tune && tune->blocks_per_cu > 0) per_cu = std::min(per_cu, int(tune->blocks_per_cu));
     B.grid = s0->num_cu * per_cu;
-    B.chunk = (tune && tune->chunk > 0) ? tune->chunk : kChunk;
     return MCG_OK;
 }
 
@@ -3145,12 +3148,16 @@ struct BatchWork {
     std::vector<BoxSolve<F>> box;        // one entry per one-box solve and part of its map
     std::vector<int> box_of;             // the entry's solve
     size_t box_lds = 0;
-    int box_block = 0, box_grid = 0, box_axes = 0, box_chunk = kChunk;
+    int box_block = 0, box_grid = 0, box_axes = 0;
     bool box_slim = false;               // the kernel with kNarrowThreads
+    std::vector<int> grab;               // bundle ids a wavefront claims at a time, per solve
     size_t words = 0;                    // claim counters of parts and visitor counts (8-byte words, cleared per launch)
 
     // Splits the solves and plans both launches.
     int make(int n, mcg_scene* const* sc, const HostProblem* P, const mcg_tune* tune) {
+        grab.clear();
+        for (int i = 0; i < n; ++i)
+            grab.push_back(tune && tune->chunk > 0 ? tune->chunk : (absorbs(sc[i]->host) ? kChunk : kChunkBatchLong));
         general.clear();
         box.clear();
         box_of.clear();
@@ -3221,7 +3228,6 @@ struct BatchWork {
             per_cu = std::min(per_cu, std::max(1, (box_slim ? kNarrowThreads : 2048) / box_block));
             if (tune && tune->blocks_per_cu > 0) per_cu = std::min(per_cu, int(tune->blocks_per_cu));
             box_grid = sc[0]->num_cu * per_cu;
-            box_chunk = tune && tune->chunk > 0 ? tune->chunk : kChunk;
         }
         if (!general.empty()) {
             std::vector<mcg_scene*> gs;
@@ -3243,7 +3249,7 @@ struct BatchWork {
         kparams.clear();
         for (int i : general) {
             kparams.push_back(K[i]);
-            kparams.back().chunk = plan.chunk;
+            kparams.back().chunk = grab[i];
             kparams.back().guide = 0.0f;
             kparams.back().tail = 0;
             kparams.back().lds_tally = plan.tally ? 1 : 0;
@@ -3263,7 +3269,7 @@ struct BatchWork {
         for (size_t j = 0; j < box.size(); ++j) {
             BoxSolve<F>& e = box[j];
             e.K = K[box_of[j]];
-            e.K.chunk = box_chunk;
+            e.K.chunk = grab[box_of[j]];
             // claims shrink within kTailLanes bundles per lane of the
             // workgroups its share of the work brings
             const double wgs = work > 0.0 ? double(box_grid) * e.work * double(e.K.count) / work : 1.0;
