@@ -62,7 +62,7 @@ BYTES_PER_STEP_FP32 = 96   # 48 B SoA bundle state read + written per scatter-st
 BYTES_PER_STEP_FP64 = 152  # 76 B state in FP64
 NBUNDLES = 10_000_000
 CPU_REPS = 3
-KERNEL_NAME = "trajectory_kernel<float, true, true, 0>"   # <F, tables in LDS, tally in LDS, walk axes>
+KERNEL_NAME = "box_kernel<float, true, 0, 4, 1024>"   # <F, tables in LDS, grid axes, tally rows, threads at most>
 
 
 def workload():
@@ -119,7 +119,7 @@ def main():
     ap.add_argument("--copy-probe", action="store_true",
                     help="run a 1 GiB device copy for counter calibration and exit")
     ap.add_argument("--traffic-json",
-                    default=os.path.join(ROOT, "profiles", "trajectory_kernel_bar1e7_fp32_traffic.json"),
+                    default=os.path.join(ROOT, "profiles", "box_kernel_bar1e7_fp32_traffic.json"),
                     help="counter-measured HBM bytes per launch of the kernel (rocprofv3 --pmc "
                          "FETCH_SIZE / WRITE_SIZE, scaled by the copy-probe calibration)")
     ap.add_argument("--quick", action="store_true",

@@ -305,7 +305,8 @@ int mcg_trace_from(mcg_scene* scene, const mcg_problem_spec* prob, int64_t prop_
                    const double pos[3], const double* dir, double* rec, int64_t cap, int64_t* nrec);
 
 /* --------------------------------------------------------------- batching
- * Many independent solves in one persistent launch.  Each solve has its
+ * Many independent solves in one persistent launch (two when scenes of one
+ * axis-aligned box and others are mixed).  Each solve has its
  * own scene, problem and output; results equal those of mcg_solve. */
 enum mcg_engine {
     MCG_ENGINE_HISTORY = 0,    /* persistent kernel, a bundle per lane for its
@@ -316,11 +317,15 @@ enum mcg_engine {
 };
 
 struct mcg_tune {
-    int32_t block;             /* threads per block: a multiple of 64 up to 1024 (0 = auto) */
+    int32_t block;             /* threads per block: a multiple of 64 up to 1024 (0 = auto);
+                                  small FP64 solves of one-box grid scenes run
+                                  with at most 512                             */
     int32_t per_thread;        /* event engine: bundles per thread per round
                                   launch, 1, 2, 4 or 8 (0 = 1); the history
                                   engine carries one bundle per lane          */
-    int32_t chunk;             /* history: bundle ids per wavefront grab         */
+    int32_t chunk;             /* history: bundle ids per wavefront grab (in a
+                                  single solve the most: a grab takes a share
+                                  of the ids left); at least 64, 0 = auto      */
     int32_t blocks_per_cu;     /* occupancy target (0 = auto)                   */
     int32_t lds_tables;        /* sampling tables in LDS: 1 yes, -1 no, 0 auto  */
     int32_t engine;            /* mcg_engine (single solves, mcg_solve)         */
@@ -329,10 +334,11 @@ struct mcg_tune {
     int32_t defer_walks;       /* history engine, scenes with 2-D / 3-D tally
                                   grids: a step's crossing walk deferred to the
                                   wavefront's walk phase, 1 yes, -1 no (walked
-                                  inside the step), 0 auto (yes when some grid
-                                  has at least 32 cells).  FP64 defers only in
-                                  single solves.  Results differ by rounding
-                                  only.                                       */
+                                  inside the step, general kernel), 0 auto:
+                                  scenes of one axis-aligned box defer, others
+                                  when some grid has at least 32 cells (FP64
+                                  only in single solves).  Results differ by
+                                  rounding only.                               */
     int64_t live;              /* event engine: bundles in flight (0 = auto)    */
 };
 
