@@ -25,7 +25,7 @@
 // film 1e6 (12 x 6 map, bundles of thousands of steps) 21.4 -> 8.0 ms.
 //
 // Results: FP32 flight takes the same rounded operations on every quantity a
-// trajectory depends on as the general step, and FP64 the checker's, so
+// trajectory depends on as the general step, and FP64 the oracle's, so
 // bundles take the same events bundle for bundle; the places where an
 // operation of the general step is left out (products with exact zeros and
 // ones) are noted where they are.
@@ -183,7 +183,7 @@ __device__ __forceinline__ dev::V3<F> unit_of(const dev::V3<F>& v) {
 }
 
 // The pore wall's normal at p, away from the axis (FP64 divides by the radius
-// as the checker does).
+// as the oracle does).
 template <typename F>
 __device__ __forceinline__ dev::V3<F> box_wall_normal(const BoxCell<F>& B, const dev::V3<F>& p) {
     if constexpr (sizeof(F) == 8) {
@@ -500,7 +500,7 @@ __device__ __forceinline__ uint32_t box_flight(const BoxCell<F>& B, BoxLane<F>& 
             dmin = take ? t : dmin;
             hit = take ? code : hit;
         } else {
-            // -(c + n.p) / (n.u) of the checker's face loop: the normal's
+            // -(c + n.p) / (n.u) of the oracle's face loop: the normal's
             // other components are zeros and its sign cancels.  Equal
             // parameters keep the lower face number.
             const F t = Quotient(u[a])((up ? B.hi[a] : B.lo[a]) - p[a]);

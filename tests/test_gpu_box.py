@@ -4,7 +4,7 @@ single cell, no tally, 2-D and 3-D maps, maps larger than the LDS (in parts
 of several rows, one row, or a range of columns, and past the most parts), each tally kind, every face kind it
 takes, a box away from the origin, a pore of each kind of wall.
 
-FP64 is compared with the checker: per-bundle counts exactly, tallies to 1e-9
+FP64 is compared with the oracle: per-bundle counts exactly, tallies to 1e-9
 (sums of at most 1e6 terms in another order: about 1e6 * 2^-53 = 1e-10 of the
 largest partial sum).  FP32 flight is compared with the event engine, which
 takes the general kernel's steps: counts exactly, tallies to 1e-5 (a grid
@@ -84,7 +84,7 @@ def close(a, b, tol):
 
 
 @pytest.mark.parametrize("name", sorted(CASES))
-def test_fp64_matches_checker(name):
+def test_fp64_matches_oracle(name):
     from oracle import oracle
     dom, tally = CASES[name]
     mat, dom = materials.si_like(300.0), dom()
