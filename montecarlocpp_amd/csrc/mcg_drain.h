@@ -6,9 +6,9 @@
 // its idle lanes the work that does not depend on the bundles' paths: the
 // draws of their next events, and the tallies of their flights.
 // Measured, before and now, same box: tee of four boxes, 1.5e5 bundles of up to
-// 20,000 steps, FP64 CumFlux 44.1 -> 31.0 ms; octet truss 1e6 FP32 4.50 -> 4.48
-// ms; a lone bundle's step in the tee, FP32 / FP64, 2.86 / 3.94 -> 1.37 / 2.04
-// us.
+// 20,000 steps, FP64 CumFlux 44.1 -> 31.0 ms (16.9 since grabs are finer);
+// octet truss 1e6 FP32 4.50 -> 4.48 ms; a lone bundle's step in the tee, FP32 /
+// FP64, 2.86 / 3.94 -> 1.37 / 2.04 us.
 #pragma once
 
 // FP32: how rarely a wavefront's iteration finds the ids spent, for the register
