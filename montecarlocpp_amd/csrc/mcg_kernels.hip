@@ -2487,9 +2487,11 @@ int launch_box(mcg_scene* sc, const HostProblem& p, KParams<F>& K, BoxCell<F>& c
         // FP64 273 -> 242 us, bar 3e5 FP64 1393 -> 1326 us, 1e6 FP64 1945 ->
         // 1808 us, bar 3e4 FP32 649 -> 627 us, porous film 2e4 FP32 2259 ->
         // 1270 us; bar 1e6 FP32 keeps 512 threads (1222 us; 384: 1337).  Where
-        // nothing absorbs, FP64 bundles are long and of one length: one a
-        // lane (porous film 1e5 FP64 3.8 -> 2.7 ms against two, 6.4 with six).
-        const int64_t kPerLane = sizeof(F) == 4 ? 2 : (absorbs(sc->host) ? 6 : 1);
+        // nothing absorbs, bundles are long and of one length: one a lane, so
+        // that none waits for another's end (porous film 5e4 FP32 2.13 -> 1.10
+        // ms, 1e5 2.15 -> 1.44 ms, 4e5 3.76 -> 3.63 ms against two; 1e5 FP64 3.8
+        // -> 2.7 ms, 6.4 ms with six).
+        const int64_t kPerLane = absorbs(sc->host) ? (sizeof(F) == 4 ? 2 : 6) : 1;
         const int64_t lanes = (p.count + kPerLane * share - 1) / (kPerLane * share);
         block = int(std::min<int64_t>(block, std::max<int64_t>(128, (lanes + 63) / 64 * 64)));
     }
