@@ -323,9 +323,11 @@ struct mcg_tune {
     int32_t per_thread;        /* event engine: bundles per thread per round
                                   launch, 1, 2, 4 or 8 (0 = 1); the history
                                   engine carries one bundle per lane          */
-    int32_t chunk;             /* history: bundle ids per wavefront grab (in a
-                                  single solve the most: a grab takes a share
-                                  of the ids left); at least 64, 0 = auto      */
+    int32_t chunk;             /* history: bundle ids per wavefront grab, 0 =
+                                  auto (in a single solve the most, at least
+                                  64: a grab takes a share of the ids left; in
+                                  a batch or server a grab below what the
+                                  wavefront's lanes need takes that many)      */
     int32_t blocks_per_cu;     /* occupancy target (0 = auto)                   */
     int32_t lds_tables;        /* sampling tables in LDS: 1 yes, -1 no, 0 auto  */
     int32_t engine;            /* mcg_engine (single solves, mcg_solve)         */

@@ -1412,7 +1412,8 @@ __device__ __forceinline__ int64_t claim(bool need, int lane, uint64_t lt_mask, 
     } else {
         const int leader = __ffsll((long long)mask) - 1;
         unsigned long long fresh = 0;
-        int want = chunk;
+        // never fewer ids than are handed out here (a batch may ask for smaller grabs)
+        int want = max(chunk, cnt - int(avail));
         if (guide > 0.0f)
             want = max(int(fminf(float(count - seen) * guide, float(chunk))), max(cnt - int(avail), min(chunk, kWave)));
         if (lane == leader) {
