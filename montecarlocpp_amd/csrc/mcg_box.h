@@ -139,16 +139,50 @@ struct BoxLane {
     int64_t id;
 };
 
+// Parameter along a flight, 0 to 1, of a walk.  An axis's crossings follow one
+// another by a fixed step; FP64 adds up steps in fixed point, 2^-62 a unit,
+// where adding them up in double puts the flight's last shares off by an ulp
+// per crossing.  Largest error of a share at 64 / 160 cells, against extended
+// precision: double steps 1.8e-15 / 4.4e-15, a quotient per crossing 1.3e-16 /
+// 2.7e-16, fixed point 8.3e-17 / 1.3e-16.  It costs 2 to 8 % of an FP64 map's
+// time (porous film 64 x 64, 1e6 bundles 17.0 -> 17.6 ms, 4e6 54.1 -> 58.4;
+// film 1e6 12.2 -> 12.5 ms).
+template <typename F>
+struct BoxParam {
+    using T = F;
+    static constexpr F kOne = F(1), kNone = F(2);   // kNone: no crossing left
+    __device__ static __forceinline__ F of(F x) { return x; }
+    __device__ static __forceinline__ double length(F to, F from) { return double(to - from); }
+    static constexpr double kUnit = 1.0;            // length() of a whole flight is 1 / kUnit
+};
+template <>
+struct BoxParam<double> {
+    using T = uint64_t;
+    static constexpr uint64_t kOne = 1ull << 62, kNone = ~0ull;
+    static constexpr double kUnit = 0x1p-62;
+    // x in [0, 1], or below for a step
+    __device__ static __forceinline__ uint64_t of(double x) {
+        const double s = x * 0x1p30, h = floor(s);
+        return (uint64_t(uint32_t(h)) << 32) | uint32_t((s - h) * 0x1p32);
+    }
+    // the difference, which rounding of the steps may leave just below zero
+    __device__ static __forceinline__ double length(uint64_t to, uint64_t from) {
+        const uint64_t d = to - from;
+        return __builtin_fma(double(int32_t(d >> 32)), 0x1p32, double(uint32_t(d)));
+    }
+};
+
 // A grid walk in progress (see WalkN).  `left` counts the entries still to
 // add (crossings and the last segment): the lane walks while it is positive.
 template <typename F, int NA>
 struct BoxWalk {
-    F t[NA], dt[NA];         // next crossing parameter per axis (2: none left) and the step between crossings
+    using T = typename BoxParam<F>::T;
+    T t[NA], dt[NA];         // next crossing parameter per axis and the step between crossings
     int32_t n[NA], dcol[NA];
     int32_t left;
     int32_t idx;
-    F prev;
-    double amt[kMaxRows];
+    T prev;
+    double amt[kMaxRows];    // per unit of BoxParam::length
 };
 // Without a grid: the share of the last flight in its last cell, kept back (the
 // next flight of the bundle starts in that cell) until the lane leaves it.
@@ -263,7 +297,8 @@ __device__ __forceinline__ double pick3(const uint32_t (&m)[3], const dev::V3<do
 // nothing that is read again.
 template <int kRows, typename F, int NA>
 __device__ __forceinline__ void box_walk_next(BoxWalk<F, NA>& W, const BoxCell<F>& B, double* tally) {
-    F tm = W.t[0], dt = W.dt[0];
+    using P = BoxParam<F>;
+    typename P::T tm = W.t[0], dt = W.dt[0];
     int32_t n = W.n[0], dcol = W.dcol[0];
     bool later[NA];   // the crossing is of axis q or a later one
     later[0] = true;
@@ -275,7 +310,7 @@ __device__ __forceinline__ void box_walk_next(BoxWalk<F, NA>& W, const BoxCell<F
         n = later[q] ? W.n[q] : n;
         dcol = later[q] ? W.dcol[q] : dcol;
     }
-    const double seg = double((W.left == 1 ? F(1) : tm) - W.prev);
+    const double seg = P::length(W.left == 1 ? P::kOne : tm, W.prev);
     double* p = tally + W.idx;
     if constexpr (kRows == kMaxRows) {
 #pragma unroll
@@ -300,7 +335,7 @@ __device__ __forceinline__ void box_walk_next(BoxWalk<F, NA>& W, const BoxCell<F
     W.prev = tm;
     W.idx += dcol;
     n--;
-    const F t = n > 0 ? tm + dt : F(2);
+    const typename P::T t = n > 0 ? tm + dt : P::kNone;
 #pragma unroll
     for (int q = 0; q < NA; ++q) {
         bool mine = later[q];
@@ -451,30 +486,34 @@ __device__ __forceinline__ void box_tally(const BoxCell<F>& B, const BoxView<F>&
             const F first = F(up ? bk + 1 : bk) - b;
             const int n = up ? ek - bk : bk - ek;
             bool none;
-            F t;
             if constexpr (sizeof(F) == 4) {
                 none = (fabsf(dc) < FLT_MIN) | (n == 0);
                 const F r = __builtin_amdgcn_rcpf(dc);
-                t = first * r;
                 W.dt[q] = fabsf(r);
+                W.t[q] = none ? F(2) : first * r;
             } else {
                 none = (fabs(dc) < DBL_MIN) | (n == 0);
                 const Quotient d(none ? F(1) : dc);
-                t = d(first);
-                W.dt[q] = fabs(d(F(1)));
+                // the step is used from two crossings on, where it is below
+                // one: 1 / |dc| and, to the fixed point's last bits, the
+                // remainder of that reciprocal
+                const double rest = __builtin_fma(-d.b, d.r, 1.0) * d.r * 0x1p62;
+                const int64_t dt = int64_t(BoxParam<F>::of(fabs(d.r))) + int32_t(dc < F(0) ? -rest : rest);
+                W.dt[q] = uint64_t(dt);
+                W.t[q] = none ? BoxParam<F>::kNone : BoxParam<F>::of(d(first));
             }
-            W.t[q] = none ? F(2) : t;
             W.n[q] = none ? 0 : n;
             left += none ? 0 : n;
             W.dcol[q] = up ? B.stride[q] : -B.stride[q];
         }
         W.idx = kRows == kMaxRows ? idx : idx - B.col0;
-        W.prev = F(0);
+        W.prev = 0;
         W.left = left;
-        W.amt[0] = double(kRows == 1 ? only : dt);
-        W.amt[1] = double(dx);
-        W.amt[2] = double(dy);
-        W.amt[3] = double(dz);
+        constexpr double kUnit = BoxParam<F>::kUnit;   // a power of two: exact
+        W.amt[0] = kUnit * double(kRows == 1 ? only : dt);
+        W.amt[1] = kUnit * double(dx);
+        W.amt[2] = kUnit * double(dy);
+        W.amt[3] = kUnit * double(dz);
     }
 }
 
