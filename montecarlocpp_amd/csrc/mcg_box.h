@@ -151,7 +151,6 @@ template <typename F>
 struct BoxParam {
     using T = F;
     static constexpr F kOne = F(1), kNone = F(2);   // kNone: no crossing left
-    __device__ static __forceinline__ F of(F x) { return x; }
     __device__ static __forceinline__ double length(F to, F from) { return double(to - from); }
     static constexpr double kUnit = 1.0;            // length() of a whole flight is 1 / kUnit
 };

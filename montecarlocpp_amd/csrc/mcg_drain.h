@@ -5,17 +5,25 @@
 // A wavefront left with at most kDrainLanes bundles and no id to claim gives
 // its idle lanes the work that does not depend on the bundles' paths: the
 // draws of their next events, and the tallies of their flights.
-// Measured, before and now, same box: tee of four boxes, 1.5e5 bundles of up to
-// 20,000 steps, FP64 CumFlux 44.1 -> 31.0 ms (16.9 since grabs are finer);
-// octet truss 1e6 FP32 4.50 -> 4.48 ms; a lone bundle's step in the tee, FP32 /
-// FP64, 2.86 / 3.94 -> 1.37 / 2.04 us.
+// It is a function of its own, called at most once by a wavefront: inlined, its
+// values took registers from the step loop, which spilled 18 to 322 vector
+// registers in FP32 and 54 to 317 in FP64 and now spills none and at most 16.
+// It publishes the wavefront's statistics (a second round of atomics on the
+// same counters cost 40 us a launch).
+// Measured, without a drain / inlined / called, same box: tee with 6 x 6 maps
+// 1e6 bundles FP32 18.0 / 18.0 / 16.1 ms, FP64 23.2 / 26.0 / 16.8; with 6 x 6 x 2
+// maps FP64 24.3 / 49.8 / 18.1; octet truss of finer struts 1e6 FP64 7.8 / 14.5 /
+// 6.0; octet 1e6 FP32 2.39 / 2.03 / 1.92; porous film, CumTemp 3e6 FP64 15.6 /
+// 23.2 / 15.5; two boxes 1e5 FP32 0.24 / 0.19 / 0.16.
 #pragma once
 
-// FP32: how rarely a wavefront's iteration finds the ids spent, for the register
-// allocation: the drain's values must not displace the main loop's (octet truss
-// 4.68 ms without it, 4.45 with it).  FP64 has no registers to spare in either,
-// and spills in the drain cost more there.
-constexpr double kDrainRare = 0.9999;
+// The kernel's parameters and its LDS as plain numbers, to hand to the drain.
+__device__ __forceinline__ uint64_t kernarg_address() {
+    return (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+}
+__device__ __forceinline__ uint32_t lds_offset(unsigned char* lds) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
+}
 
 // What an event may draw, for any kind of cell.
 template <typename F>
@@ -89,9 +97,19 @@ __device__ __forceinline__ void collide_drawn(const KParams<F>& K, const View<F>
     }
 }
 
-template <typename F, int kDefer>
-__device__ __forceinline__ void general_drain(const KParams<F>& K, const View<F>& V, const Sink& sink, int lane,
-                                              uint64_t lt_mask, Lane<F>& L, bool active, LaneStats& st) {
+template <typename F, bool kLdsTables, bool kLdsTally, int kDefer>
+__device__ __attribute__((noinline)) void general_drain(uint64_t params, uint32_t lds_at, int lane, Lane<F> L,
+                                                        bool active, LaneStats st) {
+    // arguments arrive in vector registers: the parameters' and LDS addresses
+    // are the same in all lanes
+    const uint64_t at_params = (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(params >> 32)))) << 32) |
+                               uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(params))));
+    const KParams<F>& K = *(const KParams<F>*)(ParamPtr<F>)at_params;
+    unsigned char* const lds = (unsigned char*)(__attribute__((address_space(3))) unsigned char*)(uintptr_t)
+        __builtin_amdgcn_readfirstlane(int(lds_at));
+    const View<F> V = view_of<F, kLdsTables, kLdsTally>(K, lds);
+    const Sink sink{V.direct, V.diff, K.cols};
+    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
     int span = 2 * kDrainLanes, shift = 0;
     int at = 0, ahead = 0, slot = 0;
     EventDraws<F> D;
@@ -113,7 +131,7 @@ __device__ __forceinline__ void general_drain(const KParams<F>& K, const View<F>
             pending = false;
             slot = 0;
         }
-        if (live == 0ull) return;
+        if (live == 0ull) break;
         const int n = popc(live);
         if (2 * n <= span) {
             const int to = active ? popc(live & lt_mask) : n + popc(~live & lt_mask);
@@ -190,4 +208,5 @@ __device__ __forceinline__ void general_drain(const KParams<F>& K, const View<F>
             active = false;
         }
     }
+    st.publish(K.counters, lane);
 }

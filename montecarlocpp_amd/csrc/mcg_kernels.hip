@@ -761,60 +761,35 @@ struct View {
     double* diff;
 };
 
-// Stage one solve's tables, planes, subdomains and pores in LDS and clear
-// the LDS tally; the caller synchronises.  Layout: [scat alias | vel | mfp]
-// (when kLdsTables), planes, subdomains, pores, tally direct, tally diff
-// (only when the scene has 1-D tallies, the only users of range adds).
+// A solve's view of LDS at `lds`.  Layout: [scat alias | vel | mfp] (when
+// kLdsTables), planes, subdomains, pores, tally direct, tally diff (only when
+// the scene has 1-D tallies, the only users of range adds).
 template <typename F, bool kLdsTables, bool kLdsTally>
-__device__ View<F> stage(const KParams<F>& K, unsigned char* lds, int tid, int nthreads) {
+__device__ __forceinline__ View<F> view_of(const KParams<F>& K, unsigned char* lds) {
     const int ntab = kLdsTables ? K.nmodes : 0;
     View<F> v;
     size_t off = (size_t(ntab) * (8 + 2 * sizeof(F)) + 15) & ~size_t(15);
-    DevPlane<F>* s_planes = reinterpret_cast<DevPlane<F>*>(lds + off);
+    v.planes = reinterpret_cast<const DevPlane<F>*>(lds + off);
     off = (off + sizeof(DevPlane<F>) * K.nplanes + 15) & ~size_t(15);
-    DevSdom<F>* s_sdoms = reinterpret_cast<DevSdom<F>*>(lds + off);
+    v.sdoms = reinterpret_cast<const DevSdom<F>*>(lds + off);
     off = (off + sizeof(DevSdom<F>) * K.nsdom + 15) & ~size_t(15);
-    DevPore<F>* s_pores = reinterpret_cast<DevPore<F>*>(lds + off);
+    v.pores = reinterpret_cast<const DevPore<F>*>(lds + off);
     off = (off + sizeof(DevPore<F>) * K.npore + 15) & ~size_t(15);
-    double* s_direct = reinterpret_cast<double*>(lds + off);
-    double* s_diff = s_direct + size_t(K.rows) * K.cols;
-    if (kLdsTables) {
-        uint64_t* w_scat = reinterpret_cast<uint64_t*>(lds);
-        F* w_vel = reinterpret_cast<F*>(lds + 8 * size_t(ntab));
-        F* w_mfp = w_vel + ntab;
-        for (int i = tid; i < ntab; i += nthreads) {
-            w_scat[i] = K.scat_alias[i];
-            w_vel[i] = K.mode_vel[i];
-            w_mfp[i] = K.mode_mfp[i];
-        }
-        v.scat = w_scat;
-        v.vel = w_vel;
-        v.mfp = w_mfp;
+    if constexpr (kLdsTables) {
+        v.scat = reinterpret_cast<const uint64_t*>(lds);
+        v.vel = reinterpret_cast<const F*>(lds + 8 * size_t(ntab));
+        v.mfp = v.vel + ntab;
     } else {
         v.scat = K.scat_alias;
         v.vel = K.mode_vel;
         v.mfp = K.mode_mfp;
     }
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(K.planes);
-    uint32_t* dst = reinterpret_cast<uint32_t*>(s_planes);
-    const int np = int(sizeof(DevPlane<F>) / 4) * K.nplanes;
-    for (int i = tid; i < np; i += nthreads) dst[i] = src[i];
-    src = reinterpret_cast<const uint32_t*>(K.sdoms);
-    dst = reinterpret_cast<uint32_t*>(s_sdoms);
-    const int ns = int(sizeof(DevSdom<F>) / 4) * K.nsdom;
-    for (int i = tid; i < ns; i += nthreads) dst[i] = src[i];
-    src = reinterpret_cast<const uint32_t*>(K.pores);
-    dst = reinterpret_cast<uint32_t*>(s_pores);
-    const int nq = int(sizeof(DevPore<F>) / 4) * K.npore;
-    for (int i = tid; i < nq; i += nthreads) dst[i] = src[i];
-    if (kLdsTally) {
-        const int n = K.rows * K.cols + (K.lds_diff ? K.rows * (K.cols + 1) : 0);
-        for (int i = tid; i < n; i += nthreads) s_direct[i] = 0.0;
+    if constexpr (kLdsTally) {
         // both in LDS, so the compiler addresses them as LDS (ds_add_f64);
         // without 1-D tallies the difference array is neither allocated nor
         // used (range adds come only from 1-D tallies)
-        v.direct = s_direct;
-        v.diff = s_diff;
+        v.direct = reinterpret_cast<double*>(lds + off);
+        v.diff = v.direct + size_t(K.rows) * K.cols;
     } else {
         // workgroups are dealt to the XCDs in turn, so copy w % ncopies keeps
         // a workgroup's atomics in its own XCD's L2
@@ -822,9 +797,40 @@ __device__ View<F> stage(const KParams<F>& K, unsigned char* lds, int tid, int n
         v.direct = c == 0 ? K.direct : K.priv + size_t(c - 1) * size_t(K.copy_stride);
         v.diff = c == 0 ? K.diff : v.direct + (K.diff - K.direct);
     }
-    v.planes = s_planes;
-    v.sdoms = s_sdoms;
-    v.pores = s_pores;
+    return v;
+}
+
+// Stage one solve's tables, planes, subdomains and pores in LDS and clear
+// the LDS tally; the caller synchronises.
+template <typename F, bool kLdsTables, bool kLdsTally>
+__device__ View<F> stage(const KParams<F>& K, unsigned char* lds, int tid, int nthreads) {
+    const View<F> v = view_of<F, kLdsTables, kLdsTally>(K, lds);
+    if (kLdsTables) {
+        const int ntab = K.nmodes;
+        uint64_t* w_scat = const_cast<uint64_t*>(v.scat);
+        F *w_vel = const_cast<F*>(v.vel), *w_mfp = const_cast<F*>(v.mfp);
+        for (int i = tid; i < ntab; i += nthreads) {
+            w_scat[i] = K.scat_alias[i];
+            w_vel[i] = K.mode_vel[i];
+            w_mfp[i] = K.mode_mfp[i];
+        }
+    }
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(K.planes);
+    uint32_t* dst = reinterpret_cast<uint32_t*>(const_cast<DevPlane<F>*>(v.planes));
+    const int np = int(sizeof(DevPlane<F>) / 4) * K.nplanes;
+    for (int i = tid; i < np; i += nthreads) dst[i] = src[i];
+    src = reinterpret_cast<const uint32_t*>(K.sdoms);
+    dst = reinterpret_cast<uint32_t*>(const_cast<DevSdom<F>*>(v.sdoms));
+    const int ns = int(sizeof(DevSdom<F>) / 4) * K.nsdom;
+    for (int i = tid; i < ns; i += nthreads) dst[i] = src[i];
+    src = reinterpret_cast<const uint32_t*>(K.pores);
+    dst = reinterpret_cast<uint32_t*>(const_cast<DevPore<F>*>(v.pores));
+    const int nq = int(sizeof(DevPore<F>) / 4) * K.npore;
+    for (int i = tid; i < nq; i += nthreads) dst[i] = src[i];
+    if (kLdsTally) {
+        const int n = K.rows * K.cols + (K.lds_diff ? K.rows * (K.cols + 1) : 0);
+        for (int i = tid; i < n; i += nthreads) v.direct[i] = 0.0;
+    }
     return v;
 }
 
@@ -1453,6 +1459,7 @@ __global__ void __launch_bounds__(1024) trajectory_kernel(KParams<F> K) {
     Lane<F> L;
     WalkOf<F, kDefer> W;
     LaneStats st;
+    bool drain = false;   // left the loop with bundles for the drain
     if constexpr (sizeof(F) == 4) {
         // FP32: each lane also holds its next bundle, emitted ahead of time
         // (N, valid while `full`), so a lane whose bundle ends continues at
@@ -1495,11 +1502,9 @@ __global__ void __launch_bounds__(1024) trajectory_kernel(KParams<F> K) {
                 }
             }
             if (__ballot(active || walking || full || !drained) == 0ull) break;
-            if (__builtin_expect_with_probability(__ballot(drained) != 0ull, 0, kDrainRare) && __ballot(full) == 0ull &&
-                popc(__ballot(active)) <= kDrainLanes && K.trace_id < 0) {
-                if constexpr (kDefer != 0)
-                    while (__ballot(walking) != 0ull) walk_some<kWalkUnroll>(W, walking, sink);
-                general_drain<F, kDefer>(K, V, sink, lane, lt_mask, L, active, st);
+            if (__ballot(drained) != 0ull && __ballot(full) == 0ull && popc(__ballot(active)) <= kDrainLanes &&
+                K.trace_id < 0) {
+                drain = true;
                 break;
             }
             if (active && !walking) {
@@ -1530,9 +1535,7 @@ __global__ void __launch_bounds__(1024) trajectory_kernel(KParams<F> K) {
             }
             if (__ballot(active || walking) == 0ull) break;
             if (__ballot(finished) != 0ull && popc(__ballot(active)) <= kDrainLanes && K.trace_id < 0) {
-                if constexpr (kDefer != 0)
-                    while (__ballot(walking) != 0ull) walk_some<kWalkUnroll>(W, walking, sink);
-                general_drain<F, kDefer>(K, V, sink, lane, lt_mask, L, active, st);
+                drain = true;
                 break;
             }
             if (active && !walking) {
@@ -1545,7 +1548,13 @@ __global__ void __launch_bounds__(1024) trajectory_kernel(KParams<F> K) {
             if constexpr (kDefer != 0) walk_phase(W, walking, active, sink);
         }
     }
-    st.publish(K.counters, lane);
+    if (drain) {
+        if constexpr (kDefer != 0)
+            while (__ballot(walking) != 0ull) walk_some<kWalkUnroll>(W, walking, sink);
+        general_drain<F, kLdsTables, kLdsTally, kDefer>(kernarg_address(), lds_offset(lds), lane, L, active, st);
+    } else {
+        st.publish(K.counters, lane);
+    }
     if (kLdsTally) {
         __syncthreads();
         flush_tally(V.direct, V.diff, K.direct, K.diff, K.rows, K.cols, K.lds_diff != 0, tid, blockDim.x);
