@@ -2237,9 +2237,14 @@ DevScene<F>& dev_scene(mcg_scene* sc) {
                           : reinterpret_cast<DevScene<F>&>(sc->d32);
 }
 
-// Scene and problem fields of a solve's kernel parameters (buffers aside).
-bool absorbs(const HostScene& h);
+// Whether some face absorbs bundles (otherwise they end at the scatter cap).
+bool absorbs(const HostScene& h) {
+    for (const auto& p : h.planes)
+        if (p.kind == MCG_ISOT) return true;
+    return false;
+}
 
+// Scene and problem fields of a solve's kernel parameters (buffers aside).
 template <typename F>
 void fill_params(mcg_scene* sc, const HostProblem& p, KParams<F>& K) {
     const HostScene& h = sc->host;
@@ -2396,11 +2401,7 @@ const void* pick_box_kernel(bool tables, int rows, int axes, bool narrow) {
                                   : pick_box_kernel<F, 3>(tables, rows, narrow));
 }
 
-// Parts a map may be split into.  Past this the repeated steps cost more than
-// they save: a part costs a full run of the bundles (2e-10 s a scatter-step
-// with a fine map's walk), the global map 1e-10 s per added cell and row, so
-// 64 parts pay from about 130 adds a step, which a map of that size
-// (64 x 160 KiB) takes.
+// Parts a map may be split into (their claim counters lie behind the tallies).
 constexpr int kMaxParts = 64;
 
 // LDS of a box solve's faces and tally, with its tables or without.
@@ -2410,15 +2411,69 @@ size_t box_lds_bytes(const BoxCell<F>& B, bool tables) {
            (tables ? box_lds_tables<F>(B.nmodes) : 0);
 }
 
-// LDS of a box launch: the faces and the tally (in parts, when `split`, if the
-// whole does not fit), and the tables when they fit beside them.  False when
-// the tally does not fit.
+// Cells a flight crosses into, on average, on the box's tally grid: a mode's
+// flight is cut short by the faces (the box's mean chord, 4 V / S), and an axis
+// takes half of its length.
 template <typename F>
-bool box_lds_plan(BoxCell<F>& B, bool split, bool tables_allowed, size_t limit, bool& tables, size_t& bytes) {
+double mean_crossings(const HostScene& h, const BoxCell<F>& B) {
+    const DevSdom<double>& S = h.sdoms[0];
+    double cuts = 0.0, length = 0.0, weight = 0.0;
+    for (int a = 0; a < 3; ++a) cuts += 0.5 / (S.bmax[a] - S.bmin[a]);
+    for (size_t m = 0; m < h.mode_cell.size(); ++m) {
+        const double w = h.scat[h.mode_cell[m]], mfp = h.mode_mfp[m];
+        if (mfp > 0.0) length += w / (1.0 / mfp + cuts);
+        weight += w;
+    }
+    double per_metre = 0.0;
+    for (int q = 0; q < 3; ++q) per_metre += std::fabs(double(B.div[q]) * double(B.inv[q]));
+    return weight > 0.0 ? 0.5 * length / weight * per_metre : 0.0;
+}
+
+// Whether a map past the LDS is tallied in parts rather than in global memory.
+// Each part runs every flight and its walk again; global memory is bound by
+// the rate of FP64 atomics, one per cell and row.  Measured with 1e6 bundles in
+// boxes of 0.1 to 100 um, ns a scatter-step:
+//   global memory    0.03 + 0.063 per add (1 Temp row, 2.6 adds: 0.23; 4 rows,
+//                    18: 1.11, 87: 5.3, 250: 12.3), both precisions;
+//   each part, FP32  0.02 + 0.0015 per crossing (0.3: 0.019, 7: 0.033, 46:
+//                    0.089, 193: 0.26);
+//   each part, FP64  0.05 + 0.0022 (two axes; 3.5: 0.073, 41: 0.19, 193: 0.46)
+//                    or 0.0042 (three; 7: 0.098, 46: 0.23) per crossing, and
+//                    more with few bundles, whose longest walks the parts'
+//                    fuller CUs run slower (18 parts, 193 crossings, 1e4
+//                    bundles: 2.6; a quarter of that where nothing absorbs
+//                    and bundles are of one length).
+// Few bundles, with all parts' on half of the lanes at once, take parts: each
+// bundle's chain is then what counts, and is shorter in LDS (1e4 bundles, 2 to 8
+// parts: 0.17 to 0.83 of the time, 12 to 18 parts in FP32 0.4 to 0.97).
+// Parts against global memory, ms: porous film 128 x 128 Multi (4 parts) 2e5 FP32
+// 5.5 / 156, FP64 15 / 154; 64 x 64 x 64 Multi (52) 2e5 FP64 in boxes of 0.3 um
+// 12 / 7.0, 30 um 24 / 3.4, FP32 4.6 / 6.9 and 8.3 / 3.3; 1100 x 1100 Temp (60)
+// FP32 26 / 20; 600 x 600 Temp (18) 1e6 FP64 0.3 um 39 / 52, 30 um 20 / 10.
+template <typename F>
+bool parts_pay(const HostScene& h, const BoxCell<F>& B, int rows, int64_t bundles, int cus) {
+    if (double(bundles) * B.parts <= (sizeof(F) == 4 ? 512.0 : 256.0) * cus) return true;
+    const double crossings = mean_crossings(h, B);
+    double part = 0.02 + 0.0015 * crossings;
+    if (sizeof(F) == 8) {
+        const double few = (absorbs(h) ? 80.0 : 20.0) / double(std::max<int64_t>(bundles, 1));
+        part = 0.05 + ((h.grid_2d ? 0.0022 : 0.0042) + few) * crossings;
+    }
+    return B.parts * part <= 0.03 + 0.063 * rows * (1.0 + crossings);
+}
+
+// LDS of a box launch: the faces and the tally (in parts, when `split`, if the
+// whole does not fit and they pay), and the tables when they fit beside them.
+// False when the tally does not fit.
+template <typename F>
+bool box_lds_plan(const mcg_scene* sc, int64_t bundles, BoxCell<F>& B, bool split, bool tables_allowed, bool& tables,
+                  size_t& bytes) {
+    const size_t limit = sc->lds_limit;
     const size_t faces = 6 * sizeof(BoxFace<F>);
     const int64_t room = limit > faces ? int64_t((limit - faces) / sizeof(double)) : 0;
     if (B.tally == 2 && int64_t(B.rows) * B.cols > room) {
         if (!split || room == 0) return false;
+        const int rows = B.rows;
         if (B.cols <= room) {
             const int fit = int(room / B.cols);
             B.parts = (B.rows + fit - 1) / fit;
@@ -2429,7 +2484,7 @@ bool box_lds_plan(BoxCell<F>& B, bool split, bool tables_allowed, size_t limit, 
             B.rows = 1;
             B.cols = (B.cols + B.colparts - 1) / B.colparts;
         }
-        if (B.parts > kMaxParts) return false;
+        if (B.parts > kMaxParts || !parts_pay(sc->host, B, rows, bundles, sc->num_cu)) return false;
     }
     bytes = box_lds_bytes(B, false);
     if (bytes > limit) return false;
@@ -2463,13 +2518,6 @@ __global__ void fold_copies_kernel(double* a, size_t n, const double* priv, size
 
 // Private copies of a tally that stays in global memory (one per XCD)
 constexpr int kTallyCopies = 8;
-
-// Whether some face absorbs bundles (otherwise they end at the scatter cap).
-bool absorbs(const HostScene& h) {
-    for (const auto& p : h.planes)
-        if (p.kind == MCG_ISOT) return true;
-    return false;
-}
 
 // Share of the ids left that a grab takes in a single solve on `lanes` lanes.
 float claim_share(const HostScene& h, double lanes) {
@@ -2526,7 +2574,7 @@ int launch_solve(mcg_scene* sc, const HostProblem& p, KParams<F>& K, hipStream_t
     bool box_tables = false;
     size_t box_lds = 0;
     if (K.trace_id < 0 && !(h.has_grid && sc->tune.defer_walks < 0) && box_cell<F>(h, p, cell) &&
-        box_lds_plan<F>(cell, K.part_next != nullptr, sc->tune.lds_tables >= 0, sc->lds_limit, box_tables, box_lds)) {
+        box_lds_plan<F>(sc, p.count, cell, K.part_next != nullptr, sc->tune.lds_tables >= 0, box_tables, box_lds)) {
         cell.counts = K.c_nscat != nullptr;
         const int axes = cell.tally == 2 ? (h.grid_2d ? 2 : 3) : 0;
         const bool narrow = box_narrow<F>(axes, double(p.count) * cell.parts, sc->num_cu, kNarrowPerLane);
@@ -3181,6 +3229,8 @@ struct BatchWork {
         size_t with = 0;                 // LDS with every solve's tables staged
         std::vector<BoxCell<F>> cells;
         std::vector<int> cell_of;
+        int64_t bundles = 0;
+        for (int i = 0; i < n; ++i) bundles += P[i].count;
         for (int i = 0; i < n; ++i) {
             if (sc[i]->device != sc[0]->device) return set_error(MCG_EINVAL, "batch scenes on different devices");
             const HostScene& h = sc[i]->host;
@@ -3188,7 +3238,7 @@ struct BatchWork {
             bool tab = false;
             size_t bytes = 0;
             const bool ok = !(h.has_grid && tune && tune->defer_walks < 0) && box_cell<F>(h, P[i], c) &&
-                            box_lds_plan<F>(c, true, tables, limit, tab, bytes) && (c.tally == 2 || tab);
+                            box_lds_plan<F>(sc[i], bundles, c, true, tables, tab, bytes) && (c.tally == 2 || tab);
             if (!ok) {
                 general.push_back(i);
                 continue;
@@ -3233,9 +3283,9 @@ struct BatchWork {
             box_block = tune && tune->block ? tune->block : (per_cu == 1 ? 1024 : 512);
             if (box_block < 64 || box_block > 1024 || box_block % 64 != 0)
                 return set_error(MCG_EINVAL, "block must be a multiple of 64 from 64 to 1024");
-            double bundles = 0.0;
-            for (int i : box_of) bundles += double(P[i].count);
-            box_slim = box_narrow<F>(box_axes, bundles, sc[0]->num_cu, kNarrowBatch);
+            double boxed = 0.0;
+            for (int i : box_of) boxed += double(P[i].count);
+            box_slim = box_narrow<F>(box_axes, boxed, sc[0]->num_cu, kNarrowBatch);
             if (box_slim) box_block = std::min(box_block, kNarrowThreads);
             per_cu = std::min(per_cu, std::max(1, (box_slim ? kNarrowThreads : 2048) / box_block));
             if (tune && tune->blocks_per_cu > 0) per_cu = std::min(per_cu, int(tune->blocks_per_cu));
