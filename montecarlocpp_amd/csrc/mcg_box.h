@@ -1193,15 +1193,23 @@ __global__ void __launch_bounds__(kThreads) box_kernel(KParams<F> Karg, BoxCell<
 // (the last bundles' remaining steps, during which lanes idle), so a workgroup
 // should make few visits and those where most work is left:
 //  - it starts at the solve its share of the estimated work lies in
-//    (BoxSolve::work_before), so solves begin with workgroups in proportion;
+//    (BoxSolve::work_before), so solves begin with workgroups in proportion,
+//    and goes on to those that begin in its share, so small solves are visited
+//    once each;
 //  - then it takes the solve with the most estimated work left per workgroup
 //    already on it, and leaves a solve to the workgroups on it when what is
-//    left is no more than one bundle per lane of theirs.
+//    left is no more than one bundle per lane of theirs.  A solve is taken by
+//    an atomic count of its visitors: workgroups that look at the same moment
+//    do not all go to the same one.
 // Every solve is finished: one with unclaimed bundles and no visitor is always
-// taken, and a visitor leaves only when nothing is unclaimed (a stale read of
-// a counter can only add a visit that finds nothing).
+// taken (the first to count itself as a visitor stays), and a visitor leaves
+// only when nothing is unclaimed (a stale read of a counter can only add a
+// visit that finds nothing).
 // Every solve visited in turn by the general step, before, and this: 256 slabs
 // 17.7 -> 12.1 ms a call, 24 mixed solves replayed 19.9 -> 10.3 ms, same box.
+// Many small solves, every one visited in turn / picked without shares and
+// takes / this (ms): 4000 slabs of 200 FP32 38.6 / 20.5 / 0.57, FP64 3.9 / 34.7 /
+// 1.5; 512 of 1e3 FP64 0.94 / 1.28 / 0.38.
 template <typename F>
 struct BoxSolve {
     KParams<F> K;                  // first: box_run reads it through ParamPtr
@@ -1252,29 +1260,60 @@ __device__ int box_pick(const BoxSolve<F>* solves, int n, unsigned char* lds, in
     return best == 0ull ? -1 : int(uint32_t(best));
 }
 
-// kAxes: axes of the grids among the solves (0 when all tallies are 1-D).
-template <typename F, int kAxes, int kThreads = 1024>
-__global__ void __launch_bounds__(kThreads) box_batch_kernel(const BoxSolve<F>* solves, int n) {
-    extern __shared__ __align__(16) unsigned char lds[];
-    const int tid = threadIdx.x, nthreads = blockDim.x;
-    // the solve this workgroup's share of the work starts in: the last one
-    // whose work begins at or before it
+// The last solve whose work begins at or before the middle of workgroup w's
+// share of the whole.
+template <typename F>
+__device__ __forceinline__ int box_share(const BoxSolve<F>* solves, int n, unsigned w) {
     const double total = solves[n - 1].work_before + solves[n - 1].work * double(solves[n - 1].K.count);
-    const double at = total * ((double(blockIdx.x) + 0.5) / double(gridDim.x));
+    const double at = total * ((double(w) + 0.5) / double(gridDim.x));
     int lo = 0, hi = n - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
         if (solves[mid].work_before <= at) lo = mid;
         else hi = mid - 1;
     }
-    for (int si = lo; si >= 0; si = box_pick(solves, n, lds, tid, nthreads)) {
+    return lo;
+}
+
+// Counts this workgroup as a visitor of the solve if it needs one more (uniform
+// over the workgroup; LDS is free).
+template <typename F>
+__device__ bool box_take(const BoxSolve<F>& s, unsigned char* lds, int tid, int nthreads) {
+    int* const taken = reinterpret_cast<int*>(lds);
+    if (tid == 0) {
+        uint32_t* const visitors = in_global(s.visitors);
+        const int64_t left =
+            s.K.count - int64_t(__hip_atomic_load(in_global(s.B.next), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        bool ok = left > 0;
+        if (ok) {
+            const uint32_t v = atomicAdd(visitors, 1u);
+            ok = v == 0 || left > int64_t(v) * nthreads;
+            if (!ok) atomicSub(visitors, 1u);
+        }
+        *taken = ok ? 1 : 0;
+    }
+    __syncthreads();
+    const bool ok = *taken != 0;
+    __syncthreads();
+    return ok;
+}
+
+// kAxes: axes of the grids among the solves (0 when all tallies are 1-D).
+template <typename F, int kAxes, int kThreads = 1024>
+__global__ void __launch_bounds__(kThreads) box_batch_kernel(const BoxSolve<F>* solves, int n) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int tid = threadIdx.x, nthreads = blockDim.x;
+    // this workgroup's share of the solves: from the last one whose work begins
+    // at or before the middle of its share of the work, to the next workgroup's
+    const int first = blockIdx.x == 0 ? 0 : box_share(solves, n, blockIdx.x);
+    const int last = blockIdx.x + 1 == gridDim.x ? n : box_share(solves, n, blockIdx.x + 1);
+    if (tid == 0) atomicAdd(in_global(solves[first].visitors), 1u);
+    for (int si = first, own = first; si >= 0;) {
         const auto* sv = (const __attribute__((address_space(4))) BoxSolve<F>*)(solves + __builtin_amdgcn_readfirstlane(si));
         const ParamPtr<F> kp = (ParamPtr<F>)sv;
         BoxCell<F> B = *(const BoxCell<F>*)&sv->B;
         B.k0 = kp->k0;
         B.k1 = kp->k1;
-        uint32_t* const visitors = in_global(sv->visitors);
-        if (tid == 0) atomicAdd(visitors, 1u);
         if (kAxes == 0 || B.tally != 2) {
             if (B.rowmask == 15) box_visit<F, true, 0, kMaxRows>(B, kp, lds, tid, nthreads);
             else box_visit<F, true, 0, 0>(B, kp, lds, tid, nthreads);
@@ -1287,6 +1326,17 @@ __global__ void __launch_bounds__(kThreads) box_batch_kernel(const BoxSolve<F>* 
                 else box_visit<F, false, kAxes, 0>(B, kp, lds, tid, nthreads);
             }
         }
-        if (tid == 0) atomicSub(visitors, 1u);
+        if (tid == 0) atomicSub(in_global(sv->visitors), 1u);
+        // the next solve: of this workgroup's share, then the one most in need
+        si = -1;
+        while (si < 0 && own + 1 < last) {
+            ++own;
+            if (box_take(solves[own], lds, tid, nthreads)) si = own;
+        }
+        while (si < 0) {
+            const int pick = box_pick(solves, n, lds, tid, nthreads);
+            if (pick < 0) break;
+            if (box_take(solves[pick], lds, tid, nthreads)) si = pick;
+        }
     }
 }
