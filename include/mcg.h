@@ -325,9 +325,8 @@ struct mcg_tune {
                                   engine carries one bundle per lane          */
     int32_t chunk;             /* history: bundle ids per wavefront grab, 0 =
                                   auto (in a single solve the most, at least
-                                  64: a grab takes a share of the ids left; in
-                                  a batch or server a grab below what the
-                                  wavefront's lanes need takes that many)      */
+                                  64: a grab takes a share of the ids left; a
+                                  batch or server takes 1 to 63 as 64)         */
     int32_t blocks_per_cu;     /* occupancy target (0 = auto)                   */
     int32_t lds_tables;        /* sampling tables in LDS: 1 yes, -1 no, 0 auto  */
     int32_t engine;            /* mcg_engine (single solves, mcg_solve)         */

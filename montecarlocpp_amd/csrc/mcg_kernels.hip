@@ -1400,8 +1400,9 @@ __device__ __forceinline__ void walk_phase(WalkN<F, NA>& W, bool& walking, bool 
 // grabs are few while much is left and the last ids spread over the
 // wavefronts.  In a batch, whose wavefronts come to a solve at any time, it
 // takes `chunk`, and no more than its lanes need (at least one id a lane)
-// within `tail` ids of the end.  Returns the id offset for lanes with `need`
-// (all lanes call, the pool and `seen` stay wave-uniform).
+// within `tail` ids of the end.  `chunk` is at least kWave: never fewer ids than
+// are handed out here.  Returns the id offset for lanes with `need` (all lanes
+// call, the pool and `seen` stay wave-uniform).
 template <typename Counter>
 __device__ __forceinline__ int64_t claim(bool need, int lane, uint64_t lt_mask, int64_t& base, int64_t& lim,
                                          Counter* counter, int chunk, int64_t count, float guide, int64_t tail,
@@ -1418,8 +1419,7 @@ __device__ __forceinline__ int64_t claim(bool need, int lane, uint64_t lt_mask, 
     } else {
         const int leader = __ffsll((long long)mask) - 1;
         unsigned long long fresh = 0;
-        // never fewer ids than are handed out here (a batch may ask for smaller grabs)
-        int want = max(chunk, cnt - int(avail));
+        int want = chunk;
         if (guide > 0.0f)
             want = max(int(fminf(float(count - seen) * guide, float(chunk))), max(cnt - int(avail), min(chunk, kWave)));
         if (lane == leader) {
@@ -3217,7 +3217,8 @@ struct BatchWork {
     int make(int n, mcg_scene* const* sc, const HostProblem* P, const mcg_tune* tune) {
         grab.clear();
         for (int i = 0; i < n; ++i)
-            grab.push_back(tune && tune->chunk > 0 ? tune->chunk : (absorbs(sc[i]->host) ? kChunk : kChunkBatchLong));
+            grab.push_back(tune && tune->chunk > 0 ? std::max(kWave, int(tune->chunk))   // claim needs one id a lane
+                                                   : (absorbs(sc[i]->host) ? kChunk : kChunkBatchLong));
         general.clear();
         box.clear();
         box_of.clear();
