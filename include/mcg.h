@@ -305,8 +305,8 @@ int mcg_trace_from(mcg_scene* scene, const mcg_problem_spec* prob, int64_t prop_
                    const double pos[3], const double* dir, double* rec, int64_t cap, int64_t* nrec);
 
 /* --------------------------------------------------------------- batching
- * Many independent solves in one persistent launch (two when scenes of one
- * axis-aligned box and others are mixed).  Each solve has its
+ * Many independent solves in one persistent launch (two side by side when
+ * scenes of one axis-aligned box and others are mixed).  Each solve has its
  * own scene, problem and output; results equal those of mcg_solve. */
 enum mcg_engine {
     MCG_ENGINE_HISTORY = 0,    /* persistent kernel, a bundle per lane for its

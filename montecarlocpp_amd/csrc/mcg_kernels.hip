@@ -3198,8 +3198,33 @@ int launch_batch(const BatchPlan& B, const KParams<F>* kp, int nsolves, hipStrea
     return MCG_OK;
 }
 
+// A second stream for the launches of a batch of both kinds.
+struct SideStream {
+    hipStream_t stream = nullptr;
+    hipEvent_t fork = nullptr, join = nullptr;
+    ~SideStream() {
+        if (stream) {
+            (void)hipStreamSynchronize(stream);
+            (void)hipStreamDestroy(stream);
+        }
+        if (fork) (void)hipEventDestroy(fork);
+        if (join) (void)hipEventDestroy(join);
+    }
+    int open() {
+        if (!stream) HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+        if (!fork) HIP_TRY(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
+        if (!join) HIP_TRY(hipEventCreateWithFlags(&join, hipEventDisableTiming));
+        return MCG_OK;
+    }
+};
+
 // A batch's launches: its one-box solves in one box_batch_kernel launch, the
-// others in one batch_kernel launch.
+// others in one batch_kernel launch, side by side.  Each ends on a few long
+// bundles; the other kind's workgroups take the CUs that it no longer fills.
+// One after the other / side by side, ms: 24 tees, slabs, bars and porous films of
+// 1e5 FP32 19.9 / 13.7, FP64 29.6 / 22.7; bars of 300 and 100 columns FP32 4.25 /
+// 3.56, FP64 8.2 / 7.5 (all in the general kernel: 16.4, 33.7, 3.59, 7.1).  The
+// general launch goes first: second, FP32 18.7 and 4.1.
 template <typename F>
 struct BatchWork {
     std::vector<int> general;            // solves of the general kernel
@@ -3343,17 +3368,32 @@ struct BatchWork {
         }
     }
 
-    // Enqueues both launches (box_dev, k_dev: device copies of box, kparams).
-    int launch(const BoxSolve<F>* box_dev, const KParams<F>* k_dev, hipStream_t stream) const {
+    bool mixed() const { return !box.empty() && !general.empty(); }
+
+    // Enqueues both launches on `stream` (box_dev, k_dev: device copies of box,
+    // kparams); the box one goes by `side`, opened, when both are there, and
+    // second, so that it is the one to fill up.
+    int launch(const BoxSolve<F>* box_dev, const KParams<F>* k_dev, hipStream_t stream, SideStream& side) const {
+        if (mixed()) {
+            HIP_TRY(hipEventRecord(side.fork, stream));
+            HIP_TRY(hipStreamWaitEvent(side.stream, side.fork, 0));
+        }
+        if (!general.empty()) {
+            int rc = launch_batch<F>(plan, k_dev, int(general.size()), stream);
+            if (rc) return rc;
+        }
         if (!box.empty()) {
             const void* fn = box_kernel_fn();
             int nbox = int(box.size());
             HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(box_lds)));
             void* args[] = {&box_dev, &nbox};
-            HIP_TRY(hipLaunchKernel(fn, dim3(box_grid), dim3(box_block), args, box_lds, stream));
+            HIP_TRY(hipLaunchKernel(fn, dim3(box_grid), dim3(box_block), args, box_lds, mixed() ? side.stream : stream));
             HIP_TRY(hipGetLastError());
         }
-        if (!general.empty()) return launch_batch<F>(plan, k_dev, int(general.size()), stream);
+        if (mixed()) {
+            HIP_TRY(hipEventRecord(side.join, side.stream));
+            HIP_TRY(hipStreamWaitEvent(stream, side.join, 0));
+        }
         return MCG_OK;
     }
     // Sets the kernels' LDS attributes (before a capture).
@@ -3417,11 +3457,13 @@ int run_batch(int n, mcg_scene* const* scenes, const HostProblem* P, double* con
     HIP_TRY(hipMemset(direct.p, 0, direct.n * sizeof(double)));
     HIP_TRY(hipMemset(diff.p, 0, diff.n * sizeof(double)));
     HIP_TRY(hipMemset(ctr.p, 0, ctr.n * sizeof(unsigned long long)));
+    SideStream side;
+    if (B.mixed() && (rc = side.open())) return rc;
     hipEvent_t e0, e1;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
     HIP_TRY(hipEventRecord(e0, 0));
-    if ((rc = B.launch(bp.p, kp.p, 0))) return rc;
+    if ((rc = B.launch(bp.p, kp.p, 0, side))) return rc;
     HIP_TRY(hipEventRecord(e1, 0));
     HIP_TRY(hipEventSynchronize(e1));
     float ms = 0.f;
@@ -3617,6 +3659,7 @@ struct GraphBatch : GraphBatchBase {
     DevBuf<BoxSolve<F>> bp;
     std::vector<KParams<F>> K;
     hipStream_t stream = nullptr;
+    SideStream side;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -3663,12 +3706,13 @@ struct GraphBatch : GraphBatchBase {
         HIP_TRY(hipEventCreate(&e1));
         // the kernel's LDS limit is an attribute of the function, set before capture
         if ((rc = B.prepare())) return rc;
+        if (B.mixed() && (rc = side.open())) return rc;
         HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
         const size_t total = direct.n + diff.n + ctr.n;
         const int zblocks = int(std::min<size_t>(1024, (total + 255) / 256));
         hipLaunchKernelGGL(zero_kernel, dim3(std::max(1, zblocks)), dim3(256), 0, stream, direct.p, direct.n,
                            diff.p, diff.n, ctr.p, ctr.n);
-        rc = B.launch(bp.p, kp.p, stream);
+        rc = B.launch(bp.p, kp.p, stream, side);
         hipGraph_t g = nullptr;
         const hipError_t ec = hipStreamEndCapture(stream, &g);
         if (rc) {
@@ -3783,6 +3827,7 @@ struct StepSlot {
     DevBuf<BoxSolve<double>> bp64;
     DevBuf<unsigned long long> nx32, nx64;   // per-request bundle claim counters of the step
     hipStream_t stream = nullptr;            // this slot's stream (default priority)
+    SideStream side;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     hipEvent_t ez = nullptr;                 // after the step's clearing of newly admitted requests
     bool ez_set = false;
@@ -3997,7 +4042,8 @@ int enqueue_group(mcg_server* sv, StepSlot& slot, const std::vector<Request*>& r
     if (!B.box.empty())
         HIP_TRY(hipMemcpy(bpbuf.p, B.box.data(), B.box.size() * sizeof(BoxSolve<F>), hipMemcpyHostToDevice));
     HIP_TRY(hipMemsetAsync(nxbuf.p, 0, words * sizeof(unsigned long long), slot.stream));
-    return B.launch(bpbuf.p, kpbuf.p, slot.stream);
+    if (B.mixed() && (rc = slot.side.open())) return rc;
+    return B.launch(bpbuf.p, kpbuf.p, slot.stream, slot.side);
 }
 
 // Hand out fair shares of the step budget and enqueue the step in `slot`;
