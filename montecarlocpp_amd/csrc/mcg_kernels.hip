@@ -2604,7 +2604,17 @@ int launch_solve(mcg_scene* sc, const HostProblem& p, KParams<F>& K, hipStream_t
         // 1.05 -> 0.79 ms; FP64 1e5 6.7 -> 1.7 ms with the finer grabs.
         const int64_t share = int64_t(sc->num_cu) * blocks_per_cu;
         const int64_t lanes = (p.count + share - 1) / share;
-        block = int(std::min<int64_t>(block, std::max<int64_t>(128, (lanes + 63) / 64 * 64)));
+        int small = int(std::min<int64_t>(block, std::max<int64_t>(128, (lanes + 63) / 64 * 64)));
+        // Adding in global memory, workgroups of 3 or 6 wavefronts are slower
+        // (porous film, 1000 x 1000 Temp, 1e5 FP32: 128 / 192 / 256 / 320 / 384 /
+        // 512 threads 143.0 / 149.5 / 141.2 / 144.4 / 158.0 / 141.0 ms): powers
+        // of two.
+        if (!tally) {
+            int even = 128;
+            while (even < small) even *= 2;
+            small = std::min(block, even);
+        }
+        block = small;
     }
     const int64_t needed = (p.count + block - 1) / block;
     const int grid = int(std::max<int64_t>(1, std::min<int64_t>(int64_t(sc->num_cu) * blocks_per_cu, needed)));
