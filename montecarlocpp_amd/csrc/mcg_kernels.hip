@@ -2812,14 +2812,18 @@ int run_solve_static(mcg_scene* sc, const HostProblem& p, double* out, mcg_stats
     double* const direct = reinterpret_cast<double*>(base);
     double* const diff = direct + nd;
     unsigned long long* const ctr = reinterpret_cast<unsigned long long*>(diff + nf);
-    double* const sol = reinterpret_cast<double*>(ctr + C_COUNT);
+    // the claim counters of a map's parts, where they fit (without them a map
+    // past the LDS is tallied in global memory)
+    const size_t parts = words + kMaxParts <= MCG_STATIC_SCRATCH_BYTES / 8 ? kMaxParts : 0;
+    double* const sol = reinterpret_cast<double*>(ctr + C_COUNT + parts);
     int64_t* const cdf = reinterpret_cast<int64_t*>(sol + nd);
     HIP_TRY(hipMemcpy(cdf, p.emit_cdf.data(), ncdf * sizeof(int64_t), hipMemcpyHostToDevice));
     hipLaunchKernelGGL(zero_kernel, dim3(int(std::min<size_t>(1024, (nd + nf + 255) / 256 + 1))), dim3(256), 0, 0,
-                       direct, nd + nf, static_cast<double*>(nullptr), size_t(0), ctr, size_t(C_COUNT));
+                       direct, nd + nf, static_cast<double*>(nullptr), size_t(0), ctr, size_t(C_COUNT + parts));
     HIP_TRY(hipGetLastError());
     KParams<F> K{};
     fill_params<F>(sc, p, K);
+    if (parts) K.part_next = ctr + C_COUNT;
     K.emit_cdf = cdf;
     K.direct = direct;
     K.diff = diff;
