@@ -1306,7 +1306,7 @@ __global__ void __launch_bounds__(kThreads) box_batch_kernel(const BoxSolve<F>* 
     // this workgroup's share of the solves: from the last one whose work begins
     // at or before the middle of its share of the work, to the next workgroup's
     const int first = blockIdx.x == 0 ? 0 : box_share(solves, n, blockIdx.x);
-    const int last = blockIdx.x + 1 == gridDim.x ? n : box_share(solves, n, blockIdx.x + 1);
+    int last = -1;   // looked up when it is needed: a search of global memory
     if (tid == 0) atomicAdd(in_global(solves[first].visitors), 1u);
     for (int si = first, own = first; si >= 0;) {
         const auto* sv = (const __attribute__((address_space(4))) BoxSolve<F>*)(solves + __builtin_amdgcn_readfirstlane(si));
@@ -1329,6 +1329,7 @@ __global__ void __launch_bounds__(kThreads) box_batch_kernel(const BoxSolve<F>* 
         if (tid == 0) atomicSub(in_global(sv->visitors), 1u);
         // the next solve: of this workgroup's share, then the one most in need
         si = -1;
+        if (last < 0) last = blockIdx.x + 1 == gridDim.x ? n : box_share(solves, n, blockIdx.x + 1);
         while (si < 0 && own + 1 < last) {
             ++own;
             if (box_take(solves[own], lds, tid, nthreads)) si = own;
