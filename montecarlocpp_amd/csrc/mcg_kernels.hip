@@ -2466,9 +2466,10 @@ bool parts_pay(const HostScene& h, const BoxCell<F>& B, int rows, int64_t bundle
 // whole does not fit and they pay), and the tables when they fit beside them.
 // False when the tally does not fit.
 template <typename F>
-bool box_lds_plan(const mcg_scene* sc, int64_t bundles, BoxCell<F>& B, bool split, bool tables_allowed, bool& tables,
-                  size_t& bytes) {
+bool box_lds_plan(const mcg_scene* sc, int64_t bundles, BoxCell<F>& B, bool split, int tables_knob, int block,
+                  bool& tables, size_t& bytes) {
     const size_t limit = sc->lds_limit;
+    const bool tables_allowed = tables_knob >= 0;
     const size_t faces = 6 * sizeof(BoxFace<F>);
     const int64_t room = limit > faces ? int64_t((limit - faces) / sizeof(double)) : 0;
     if (B.tally == 2 && int64_t(B.rows) * B.cols > room) {
@@ -2488,8 +2489,15 @@ bool box_lds_plan(const mcg_scene* sc, int64_t bundles, BoxCell<F>& B, bool spli
     }
     bytes = box_lds_bytes(B, false);
     if (bytes > limit) return false;
-    tables = tables_allowed && box_lds_bytes(B, true) <= limit;
-    if (tables) bytes = box_lds_bytes(B, true);
+    const size_t with = box_lds_bytes(B, true);
+    tables = tables_allowed && with <= limit;
+    // workgroups asked for so small that beside the tables too few fit a CU do
+    // without them (bar 1e7 FP64, blocks of 64 / 128 / 256: 50 / 27 / 13.9 ms
+    // with tables, 9.1 / 7.6 / 7.5 without; FP32 15.0 / 8.3 / 4.9 and 5.0 / 3.9 /
+    // 3.6)
+    if (tables && tables_knob == 0 && block > 0 && limit / with * block < 512 && limit / with < limit / bytes)
+        tables = false;
+    if (tables) bytes = with;
     return true;
 }
 
@@ -2574,7 +2582,8 @@ int launch_solve(mcg_scene* sc, const HostProblem& p, KParams<F>& K, hipStream_t
     bool box_tables = false;
     size_t box_lds = 0;
     if (K.trace_id < 0 && !(h.has_grid && sc->tune.defer_walks < 0) && box_cell<F>(h, p, cell) &&
-        box_lds_plan<F>(sc, p.count, cell, K.part_next != nullptr, sc->tune.lds_tables >= 0, box_tables, box_lds)) {
+        box_lds_plan<F>(sc, p.count, cell, K.part_next != nullptr, sc->tune.lds_tables, sc->tune.block, box_tables,
+                        box_lds)) {
         cell.counts = K.c_nscat != nullptr;
         const int axes = cell.tally == 2 ? (h.grid_2d ? 2 : 3) : 0;
         const bool narrow = box_narrow<F>(axes, double(p.count) * cell.parts, sc->num_cu, kNarrowPerLane);
@@ -3266,6 +3275,11 @@ struct BatchWork {
             return set_error(MCG_EINVAL, "defer_walks must be -1, 0 or 1");
         const size_t limit = sc[0]->lds_limit;
         const bool tables = !(tune && tune->lds_tables < 0);
+        // FP64 1-D solves in workgroups of at most 128 threads: one fits a CU
+        // beside the tables and the fixed row stride, two in the general kernel
+        // (16 bars of 3e5 in a batch, blocks of 64 / 128 / 256: 24.5 / 13.4 / 7.0
+        // ms, general 18.8 / 12.1 / 8.3)
+        const bool lone = sizeof(F) == 8 && tune && tune->block > 0 && tune->block <= 128;
         size_t with = 0;                 // LDS with every solve's tables staged
         std::vector<BoxCell<F>> cells;
         std::vector<int> cell_of;
@@ -3278,7 +3292,8 @@ struct BatchWork {
             bool tab = false;
             size_t bytes = 0;
             const bool ok = !(h.has_grid && tune && tune->defer_walks < 0) && box_cell<F>(h, P[i], c) &&
-                            box_lds_plan<F>(sc[i], bundles, c, true, tables, tab, bytes) && (c.tally == 2 || tab);
+                            box_lds_plan<F>(sc[i], bundles, c, true, tables ? 1 : -1, 0, tab, bytes) && (c.tally == 2 || tab) &&
+                            !(lone && c.tally != 2);
             if (!ok) {
                 general.push_back(i);
                 continue;
