@@ -3445,6 +3445,13 @@ struct BatchWork {
     }
 };
 
+// Whether a batch of both kinds has launches of different default blocks.
+template <typename F>
+bool default_blocks_differ(int n, mcg_scene* const* scenes, const HostProblem* P) {
+    BatchWork<F> w;
+    return w.make(n, scenes, P, nullptr) == MCG_OK && w.mixed() && w.box_block != w.plan.block;
+}
+
 template <typename F>
 int run_batch(int n, mcg_scene* const* scenes, const HostProblem* P, double* const* outs,
               mcg_stats* stats, const mcg_tune* tune) {
@@ -4509,10 +4516,11 @@ int mcg_autotune(mcg_scene* scene, const mcg_problem_spec* prob, int64_t sample_
     const mcg_tune saved = scene->tune;
     mcg_tune top = saved;
     double top_rate = -1.0;
-    // candidates: the history kernel's block, table placement and grab size;
-    // the event engine's bundles in flight, bundles per thread and rounds
-    // between regroupings
-    std::vector<mcg_tune> cand;
+    // candidates: the defaults (whose shape for a small solve no fixed block
+    // has); the history kernel's block, table placement and grab size; the
+    // event engine's bundles in flight, bundles per thread and rounds between
+    // regroupings
+    std::vector<mcg_tune> cand{mcg_tune{}};
     static const int blocks[] = {64, 128, 256, 512, 1024};
     static const int tables[] = {1, -1};
     static const int chunks[] = {64, 256, 1024};
@@ -4626,8 +4634,13 @@ int mcg_autotune_batch(int32_t n, mcg_scene* const* scenes, const mcg_problem_sp
     };
     static const int blocks[] = {128, 256, 512, 1024};
     static const int tables[] = {1, -1};
-    static const int chunks[] = {64, 256, 1024};
+    static const int chunks[] = {0, 64, 256, 1024};
     int rc;
+    // the defaults are among these shapes, unless the batch's two launches
+    // differ in their block
+    if (prec == MCG_FP64 ? mcg::default_blocks_differ<double>(n, sc.data(), P.data())
+                         : mcg::default_blocks_differ<float>(n, sc.data(), P.data()))
+        if ((rc = measure(mcg_tune{}))) return rc;
     for (int b : blocks)
         for (int t : tables)
             for (int c : chunks) {
@@ -4638,7 +4651,8 @@ int mcg_autotune_batch(int32_t n, mcg_scene* const* scenes, const mcg_problem_sp
                 if ((rc = measure(cand))) return rc;
             }
     // FP32 batches with 2-D / 3-D grids: the best shape with its tally walks
-    // deferred and walked inside the step (FP64 batches walk inside the step)
+    // deferred and walked inside the step (FP64 batches defer those of one box
+    // only, where walking inside the step is no gain)
     bool grid = false;
     for (int i = 0; i < n; ++i) grid = grid || scenes[i]->host.has_grid;
     if (grid && prec != MCG_FP64) {
