@@ -104,8 +104,9 @@ constexpr int kEmitQuorumFp64 = MCG_EMIT_QUORUM_FP64;
 #define MCG_SLOT_QUORUM 16
 #endif
 constexpr int kSlotQuorum = MCG_SLOT_QUORUM;
-// FP32 single solve: the end phase starts this many bundles per lane of the
-// grid before the last id
+// FP32: the end phase starts this many bundles per lane of the grid (in a batch,
+// of the workgroups a one-box solve's share of the work brings) before the last
+// id
 #ifndef MCG_TAIL_LANES
 #define MCG_TAIL_LANES 2
 #endif
@@ -152,7 +153,8 @@ struct KParams {
     int32_t lds_tally;
     int32_t lds_diff;      // the LDS tally holds the range-add difference array (1-D tallies)
     int32_t chunk;         // bundle ids a wavefront claims at a time, at most
-    int64_t tail;          // FP32: ids from the end where only idle lanes take a next bundle (0: never)
+    int64_t tail;          // FP32: ids from the end where only idle lanes take a next bundle, and one-box
+                           // solves of a batch smaller grabs (0: never)
     float guide;           // share of the ids left that a wavefront claims at a time
     int64_t trace_id;      // bundle whose steps are recorded, -1 for none
     double* trace;         // MCG_TRACE_WIDTH doubles per step
@@ -1399,8 +1401,8 @@ __device__ __forceinline__ void walk_phase(WalkN<F, NA>& W, bool& walking, bool 
 // (`seen`: the counter after it), from one id a lane to `chunk`, so that
 // grabs are few while much is left and the last ids spread over the
 // wavefronts.  In a batch, whose wavefronts come to a solve at any time, it
-// takes `chunk`, and no more than its lanes need (at least one id a lane)
-// within `tail` ids of the end.  `chunk` is at least kWave: never fewer ids than
+// takes `chunk`, and (one-box FP32) no more than its lanes need, at least one id
+// a lane, within `tail` ids of the end.  `chunk` is at least kWave: never fewer ids than
 // are handed out here.  Returns the id offset for lanes with `need` (all lanes
 // call, the pool and `seen` stay wave-uniform).
 template <typename Counter>
@@ -1486,7 +1488,7 @@ __global__ void __launch_bounds__(1024) trajectory_kernel(KParams<F> K) {
                 (__popcll(me) >= kSlotQuorum || __popcll(__ballot(empty && !active && !walking)) >= kEmitQuorum ||
                  __ballot(active || walking) == 0ull)) {
                 const int64_t mine = claim(empty, lane, lt_mask, pool_base, pool_lim, K.next, K.chunk, K.count,
-                                           K.guide, sizeof(F) == 4 ? K.tail : 0, seen);
+                                           K.guide, 0, seen);
                 if (empty) {
                     if (mine < K.count) {
                         emit<F>(K, K.flux_alias, V.mfp, K.first + mine, N);
@@ -1523,7 +1525,7 @@ __global__ void __launch_bounds__(1024) trajectory_kernel(KParams<F> K) {
             const bool need = !active && !finished && !walking;
             if (emit_now<kEmitQuorumFp64>(need, active || walking)) {
                 const int64_t mine = claim(need, lane, lt_mask, pool_base, pool_lim, K.next, K.chunk, K.count,
-                                           K.guide, sizeof(F) == 4 ? K.tail : 0, seen);
+                                           K.guide, 0, seen);
                 if (need) {
                     if (mine < K.count) {
                         emit<F>(K, K.flux_alias, V.mfp, K.first + mine, L);
@@ -1643,7 +1645,7 @@ __global__ void __launch_bounds__(1024) batch_kernel(const KParams<F>* __restric
             const bool need = !active && !finished && !walking;
             if (emit_now(need, active || walking)) {
                 const int64_t mine = claim(need, lane, lt_mask, pool_base, pool_lim, K.next, K.chunk, K.count,
-                                           K.guide, sizeof(F) == 4 ? K.tail : 0, seen);
+                                           0.0f, 0, seen);
                 if (need) {
                     if (mine < K.count) {
                         emit<F>(K, K.flux_alias, V.mfp, K.first + mine, L);
@@ -2282,10 +2284,10 @@ void fill_params(mcg_scene* sc, const HostProblem& p, KParams<F>& K) {
 // The wavefront-uniform description of a scene that is one axis-aligned box
 // (mcg_box.h); false when the scene or the problem needs the general kernel:
 //  - faces other than specular, diffuse, partial, isothermal or periodic onto
-//    the box itself by a pure translation along the face's axis;
+//    the box itself by a pure translation;
 //  - a tally by scatter order (more than kMaxRows rows), a 1-D tally of more
-//    than kBoxCols - 1 cells (the fixed LDS stride), grid axes that are not
-//    x, y, z in order;
+//    than kBoxCols - 1 cells (the fixed LDS stride), a tally axis along more
+//    than one coordinate;
 //  - maxscat past 32 bits (the step compares 32-bit counts).
 // Its values are those of the uploaded records, so a step's operands are the
 // general kernel's.
