@@ -42,8 +42,8 @@ enum : uint32_t { kCodeIntrinsic = 24, kCodePore = 28 };
 // for fewer rows).  Four FP64 LDS adds a crossing bound such a map: the LDS
 // takes 10 cycles for an add of 20 lanes and 20 for one of 64 (bank conflicts
 // even out), so fuller phases pay although they leave fewer lanes to step.
-// Porous film 1e7, 64 x 64, quorum 20 / 32 / 40 / 44 / 48: 70.8 / 66.6 / 65.1 /
-// 64.7 / 66.1 ms; 24 mixed solves replayed 11.07 / 11.1 / 11.2 / 11.3 / 11.5 ms.
+// Porous film 1e7, 64 x 64, quorum 28 / 32 / 36 / 40 / 44: 68.0 / 67.2 / 65.9 /
+// 65.6 / 64.7 ms; 24 mixed solves replayed 10.2 / 10.1 / 10.1 / 10.4 / 10.6 ms.
 // One row at a time (a 128 x 128 map in parts) is bound by the steps: quorum
 // 20 / 28 / 36 / 44: 9.6 / 9.8 / 10.2 / 11.3 ms.
 constexpr int kBoxWalkQuorum4 = 36;
