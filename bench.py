@@ -11,7 +11,8 @@ tallies and sampling tables.  One timed step is one complete field solve
 
 Printed: one JSON line with the scatter-step throughput, the roofline
 object of the trajectory kernel (algorithmic bytes = 96 B of bundle state
-round trip per scatter-step), the tally error of the FP32-flight run against
+round trip per scatter-step, a model: the kernel keeps the state in registers,
+so the fraction can pass 1), the tally error of the FP32-flight run against
 the FP64 run of the same streams, the FP64 CPU checker timed on the same
 workload on the host cores (whose result for the first seed the GPU's FP64
 and FP32 runs are also compared with), and secondary objects:

@@ -224,7 +224,8 @@ class Scene:
 
 
 def batch_solve(scenes_, probs, tune=None):
-    """mcg_batch_solve: all solves in one persistent launch (per precision).
+    """mcg_batch_solve: all solves in one persistent launch (per precision; two
+    side by side when scenes of one box and others are mixed).
     Returns (list of fields, list of stats dicts)."""
     n = len(scenes_)
     infos = [sc.plan(p) for sc, p in zip(scenes_, probs)]
