@@ -3340,9 +3340,21 @@ struct BatchWork {
             box_block = tune && tune->block ? tune->block : (per_cu == 1 ? 1024 : 512);
             if (box_block < 64 || box_block > 1024 || box_block % 64 != 0)
                 return set_error(MCG_EINVAL, "block must be a multiple of 64 from 64 to 1024");
-            double boxed = 0.0;
-            for (int i : box_of) boxed += double(P[i].count);
-            box_slim = box_narrow<F>(box_axes, boxed, sc[0]->num_cu, kNarrowBatch);
+            double boxed = 0.0, work = 0.0, fewer = 0.0;
+            for (size_t j = 0; j < box.size(); ++j) {
+                const double n = double(P[box_of[j]].count), w = box[j].work * n;
+                boxed += n;
+                work += w;
+                if (box[j].B.tally == 2 && box[j].B.rowmask != 15) fewer += w;
+            }
+            // With three axes the 1024-thread FP64 kernel spills in the walk of a
+            // map of fewer rows (other tallies, parts): a quarter of the work in
+            // such maps takes the 512-thread one.  1024 / 512 threads: 8 porous
+            // films 16 x 16 x 4 of 5e5 Flux 28.7 / 20.0 ms, 8 of 30 x 30 x 14 in
+            // 3 parts of 2e5 66.7 / 44.1, 8 Multi maps and one in parts 10.8 /
+            // 8.9; Multi alone 21.6 / 23.8.
+            box_slim = box_narrow<F>(box_axes, box_axes == 3 && 4.0 * fewer > work ? 0.0 : boxed, sc[0]->num_cu,
+                                     kNarrowBatch);
             if (box_slim) box_block = std::min(box_block, kNarrowThreads);
             per_cu = std::min(per_cu, std::max(1, (box_slim ? kNarrowThreads : 2048) / box_block));
             if (tune && tune->blocks_per_cu > 0) per_cu = std::min(per_cu, int(tune->blocks_per_cu));
