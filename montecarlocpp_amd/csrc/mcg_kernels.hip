@@ -2573,6 +2573,18 @@ int launch_box(mcg_scene* sc, const HostProblem& p, KParams<F>& K, BoxCell<F>& c
     return MCG_OK;
 }
 
+// Whether a one-box solve keeps its kernel: an FP64 map of three axes and more
+// bundles than the 512-thread kernel takes goes through the general one, whose
+// walk does not spill (the box kernel's 1024 threads have 128 registers each,
+// and it spills 60 to 100).  4e6 bundles, box / general: porous film 16 x 16 x 4
+// Multi 32.1 / 21.0 ms, 30 x 30 x 5 47.0 / 25.8, box of 12^3 3.6 / 1.6, of 5 x 4 x 3
+// 3.0 / 1.7.  Parts and, round a pore, the one row of a Temp map stay (16 x 16 x 4
+// 17.7 / 20.6).
+template <typename F>
+bool wide_box_pays(const BoxCell<F>& B, int axes, bool narrow) {
+    return sizeof(F) == 4 || axes != 3 || narrow || B.parts > 1 || (B.rows == 1 && B.pore >= 0);
+}
+
 // Launch shape and LDS plan of a single solve, then the launch on `stream`
 // (K holds the solve's buffers; its LDS and tail fields are set here).
 template <typename F>
@@ -2589,8 +2601,10 @@ int launch_solve(mcg_scene* sc, const HostProblem& p, KParams<F>& K, hipStream_t
         cell.counts = K.c_nscat != nullptr;
         const int axes = cell.tally == 2 ? (h.grid_2d ? 2 : 3) : 0;
         const bool narrow = box_narrow<F>(axes, double(p.count) * cell.parts, sc->num_cu, kNarrowPerLane);
-        return launch_box<F>(sc, p, K, cell, pick_box_kernel<F>(box_tables, cell.rows, axes, narrow), narrow, box_lds,
-                             stream);
+        if (wide_box_pays<F>(cell, axes, narrow)) {
+            return launch_box<F>(sc, p, K, cell, pick_box_kernel<F>(box_tables, cell.rows, axes, narrow), narrow,
+                                 box_lds, stream);
+        }
     }
     const size_t geo = lds_bytes<F>(h, rows, false, false);
     const LdsPlan lp = plan_lds(geo, lds_bytes<F>(h, rows, true, false) - geo,
