@@ -2602,6 +2602,15 @@ int launch_solve(mcg_scene* sc, const HostProblem& p, KParams<F>& K, hipStream_t
         const int axes = cell.tally == 2 ? (h.grid_2d ? 2 : 3) : 0;
         const bool narrow = box_narrow<F>(axes, double(p.count) * cell.parts, sc->num_cu, kNarrowPerLane);
         if (wide_box_pays<F>(cell, axes, narrow)) {
+            // FP64 maps of more bundles than the 512-thread kernel takes: small
+            // workgroups without the tables in LDS, which the 1024-thread
+            // kernel otherwise fills a CU with one by one (4e6 bundles, with /
+            // without: porous film 16 x 16 18.6 / 16.4 ms, 60 x 60 Flux 32.8 /
+            // 23.0, film 12 x 6 26.9 / 23.8, bar 20 x 4 7.3 / 6.0)
+            if (sizeof(F) == 8 && axes != 0 && !narrow && box_tables && sc->tune.lds_tables == 0) {
+                box_tables = false;
+                box_lds = box_lds_bytes(cell, false);
+            }
             return launch_box<F>(sc, p, K, cell, pick_box_kernel<F>(box_tables, cell.rows, axes, narrow), narrow,
                                  box_lds, stream);
         }
