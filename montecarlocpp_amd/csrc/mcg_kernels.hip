@@ -2623,6 +2623,10 @@ int launch_solve(mcg_scene* sc, const HostProblem& p, KParams<F>& K, hipStream_t
     const size_t lds = lp.bytes;
     if (lds > sc->lds_limit) return set_error(MCG_ERANGE, "geometry exceeds the LDS budget");
     K.lds_tally = tally ? 1 : 0;
+    // FP64 steps are long and the counter's 20 ns a grab is little beside them:
+    // the first grabs of 1024 ids are too much for one wavefront (two boxes 4e6
+    // 1.48 -> 1.28 ms with 256, box of 12^3 4e6 1.85 -> 1.65, 1e7 3.98 -> 3.42)
+    if (sizeof(F) == 8 && sc->tune.chunk <= 0) K.chunk = std::min(K.chunk, kChunk);
     const void* fn = pick_kernel<F>(KernelKind::Trajectory, tables, tally,
                                     walk_axes<F>(h.has_grid, h.grid_2d, h.grid_cells, KernelKind::Trajectory,
                                                  sc->tune.defer_walks));
