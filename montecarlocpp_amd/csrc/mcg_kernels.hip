@@ -55,6 +55,7 @@ constexpr int kWave = 64;
 // launch shapes of small solves below are part of the last four).  With 1 for
 // long bundles octet FP32 1e6 takes 4.9 ms, with 4 for short ones slab FP32
 // 1e6 0.59 instead of 0.48 ms.
+// FP64 solves of the general kernel take kChunk at most (launch_solve).
 constexpr int kGuideShort = 1, kChunkShort = 1024;
 constexpr int kGuideLong = 4, kChunkLong = 256;
 // A batch's grabs, by the same reasons: against 256 throughout, 24 mixed FP32
@@ -2579,10 +2580,12 @@ int launch_box(mcg_scene* sc, const HostProblem& p, KParams<F>& K, BoxCell<F>& c
 // and it spills 60 to 100).  4e6 bundles, box / general: porous film 16 x 16 x 4
 // Multi 32.1 / 21.0 ms, 30 x 30 x 5 47.0 / 25.8, box of 12^3 3.6 / 1.6, of 5 x 4 x 3
 // 3.0 / 1.7.  Parts and, round a pore, the one row of a Temp map stay (16 x 16 x 4
-// 17.7 / 20.6).
+// 17.7 / 20.6), and so does a map that fits the LDS only beside the box kernel's
+// records (23 x 20 x 11 Multi, 2e6 bundles: box 3.4 / 25.7, round a pore 25.1 / 297).
 template <typename F>
-bool wide_box_pays(const BoxCell<F>& B, int axes, bool narrow) {
-    return sizeof(F) == 4 || axes != 3 || narrow || B.parts > 1 || (B.rows == 1 && B.pore >= 0);
+bool wide_box_pays(const HostScene& h, int rows, size_t lds_limit, const BoxCell<F>& B, int axes, bool narrow) {
+    return sizeof(F) == 4 || axes != 3 || narrow || B.parts > 1 || (B.rows == 1 && B.pore >= 0) ||
+           lds_bytes<F>(h, rows, false, true) > lds_limit;
 }
 
 // Launch shape and LDS plan of a single solve, then the launch on `stream`
@@ -2601,7 +2604,7 @@ int launch_solve(mcg_scene* sc, const HostProblem& p, KParams<F>& K, hipStream_t
         cell.counts = K.c_nscat != nullptr;
         const int axes = cell.tally == 2 ? (h.grid_2d ? 2 : 3) : 0;
         const bool narrow = box_narrow<F>(axes, double(p.count) * cell.parts, sc->num_cu, kNarrowPerLane);
-        if (wide_box_pays<F>(cell, axes, narrow)) {
+        if (wide_box_pays<F>(h, rows, sc->lds_limit, cell, axes, narrow)) {
             // FP64 maps of more bundles than the 512-thread kernel takes: small
             // workgroups without the tables in LDS, which the 1024-thread
             // kernel otherwise fills a CU with one by one (4e6 bundles, with /
